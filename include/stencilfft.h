@@ -297,7 +297,8 @@ typedef enum {
     ZM_STAGE_LINE = 0,     /* fused FFT1a + exchange + twiddle + FFT1b pass */
     ZM_STAGE_A = 1,        /* FFT1a + pack + exchange */
     ZM_STAGE_B = 2,        /* unpack + twiddle + FFT1b */
-    ZM_STAGE_REPACK = 3,   /* repack-transpose */
+    ZM_STAGE_REPACK = 3,   /* repack-transpose; where a line pass's tiles hold it, counted with no
+                              time of its own (ZM_STAGE_LINE has it) */
     ZM_STAGE_LAPLACE = 4,
     ZM_STAGE_DERIV = 5,    /* dx4 / dy4 */
     ZM_STAGE_SPECTRAL = 6,

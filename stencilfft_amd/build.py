@@ -16,7 +16,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 BUILD_DIR = os.path.join(HERE, "_build")
 LIB_PATH = os.path.join(HERE, "libstencilfft.so")
-SOURCES = ["plan.hip", "fft.hip", "line_fast.hip", "stencil.hip", "spectral.hip"]
+SOURCES = ["plan.hip", "fft.hip", "line_fast.hip", "line_pass_f32.hip", "line_pass_f64.hip", "stencil.hip",
+           "spectral.hip"]
 ARCH = "gfx950"
 
 # No packed-FP32 instructions: hipcc would otherwise form v_pk_* FP32 ops from

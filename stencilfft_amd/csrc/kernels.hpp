@@ -69,6 +69,67 @@ hipError_t launch_line_fast(const Cx<T>* in, Cx<T>* out, const Geo& g, const Lin
 int line_table_entries(int vec, int m);
 hipError_t launch_line_tables(double2* t64, float2* t32, int vec, int m, hipStream_t stream);
 
+// A bit permutation v -> sum over fields of ((v >> from) & mask) << to.
+struct BitField {
+    int from, mask, to;
+};
+template <int K>
+struct BitMap {
+    BitField f[K];
+};
+
+// Line passes over natural-order lines (line_pass.hpp).  A line has an index
+// lambda in [0, N^(d-1)); a workgroup takes 2^lines of consecutive ones.  Each
+// end of the pass places element n of line lambda at bits(l, lambda) +
+// bits(n, n) of the field; a packed end maps the memory-order element e of a
+// line's rank rows there instead, and `pk` maps e to its sample n.
+struct LinePassArgs {
+    BitMap<4> in_l, out_l;
+    BitMap<3> in_n, out_n, pk;
+    int lgroups;    // log2 of the line groups per field
+    int groups;     // line groups of the whole batch
+    int xcd;        // consecutive groups on one XCD
+    int64_t field;  // elements per field
+};
+
+// A spectral multiplier between the two transforms of a pass: f0, f1 map
+// lambda to the frequencies of the other axes (axis 0 first; f1 in 3D only).
+struct SpectralArgs {
+    int kind, conj, dims;
+    double p0, p1, kscale;
+    BitMap<4> f0, f1;
+    const double* half_sin;  // sin(pi s / N), s the signed wavenumber of f < N
+};
+
+// kinds of line pass: the two ends and the direction
+enum LinePass {
+    LP_ROW_FWD = 0,    // packed -> row
+    LP_ROW_INV = 1,    // row -> packed
+    LP_TILE_FWD = 2,   // tile -> row
+    LP_TILE_INV = 3,   // row -> tile
+    LP_TILE_SPEC = 4,  // tile -> multiplier -> tile
+    LP_ROW_SPEC = 5    // packed -> multiplier -> packed
+};
+struct LinePassInfo {
+    int lines_log2;  // log2 of the lines per workgroup; -1: not built
+    int occupancy;   // workgroups per CU
+    bool loop;       // workgroups loop over groups (else one group each)
+    int tables;      // twiddle table entries
+};
+// Lines of 2^ln points; small: the variant for fields with few line groups;
+// radix16: the split with the largest radices, where it differs.
+struct LinePassSize {
+    int ln;
+    bool small, radix16;
+};
+template <typename T>
+LinePassInfo line_pass_info(LinePass kind, const LinePassSize& size);
+template <typename T>
+hipError_t launch_line_pass_tables(LinePass kind, const LinePassSize& size, Cx<T>* tables, hipStream_t stream);
+template <typename T>
+hipError_t launch_line_pass(LinePass kind, const LinePassSize& size, const Cx<T>* in, Cx<T>* out, const LinePassArgs& a,
+                            const Cx<T>* tables, double scale, const SpectralArgs& sp, int grid, hipStream_t stream);
+
 // stencils: E = element type (T or Cx<T>)
 enum StencilOp { OP_LAPLACE = 0, OP_DX4 = 1, OP_DY4 = 2, OP_DZ4 = 3 };
 template <typename T>

@@ -1,0 +1,71 @@
+// line_maps.hpp -- host side of the natural-order line passes: the address maps
+// of their ends for every (N, P, B) and axis.
+#pragma once
+
+#include "kernels.hpp"
+
+namespace zm {
+
+// ---------------------------------------------------------------------------
+// Address maps of the natural-order line passes (line_pass.hpp).  With lower-
+// case names for the log2 of N, P, B, L, VEC, .. a rank slab holds 2^(d l)
+// elements and rank ids run col, row, depth; a line's index lambda counts, from
+// its lowest bits, the position y its tile runs along, the untouched index e
+// (3D) and the rank coordinates off the axis.
+//
+// Between the y and the z pass of a tiled 3D transform a slab holds [row]
+// [depth][col] instead of [depth][row][col]: a z tile then reads runs L
+// elements apart like a y tile, where runs L^2 apart (512 KB at 512^3) cost
+// the inverse pass 11% (0.409 -> 0.368 ms, FP32).
+// ---------------------------------------------------------------------------
+inline BitField field_of(int from, int nbits, int to) { return BitField{from, (1 << nbits) - 1, to}; }
+
+struct NatMaps {
+    const Geo& g;
+    int d, lvp, lm, slab;
+    explicit NatMaps(const Geo& geo)
+        : g(geo), d(geo.dims), lvp(geo.lvec - geo.lp), lm(geo.lb + geo.lp), slab(geo.dims * geo.ll) {}
+
+    int member(int axis) const { return slab + axis * g.lp; }  // shift of the axis's own rank coordinate
+    // lambda -> line base: y at shift `ys`, e at `es`, the ranks off `axis`
+    BitMap<4> lines(int axis, int ys, int es) const {
+        const int lo = member(axis == 0 ? 1 : 0), hi = member(axis == 2 ? 1 : 2);
+        if (d == 2) return {{field_of(0, g.ll, ys), field_of(g.ll, g.lp, lo), {}, {}}};
+        return {{field_of(0, g.ll, ys), field_of(g.ll, g.ll, es), field_of(2 * g.ll, g.lp, lo),
+                 field_of(2 * g.ll + g.lp, g.lp, hi)}};
+    }
+    // rows: the lines of a pass on its reciprocal (or packed) side
+    BitMap<4> row_lines(int axis, bool tiled) const {
+        const bool swapped = axis == 2 || (axis == 1 && tiled && d == 3);
+        return swapped ? lines(axis, 2 * g.ll, g.ll) : lines(axis, g.ll, 2 * g.ll);
+    }
+    // reciprocal row: k = k1 + VEC k2 -> k1 % VP + k2 VP of member k1 / VP
+    BitMap<3> row(int axis) const {
+        return {{field_of(0, lvp, 0), field_of(lvp, g.lp, member(axis)), field_of(g.lvec, lm, lvp)}};
+    }
+    // memory-order element of the P rank rows of a packed line, and its sample n
+    BitMap<3> packed(int axis) const { return {{field_of(0, g.ll, 0), field_of(g.ll, g.lp, member(axis)), {}}}; }
+    BitMap<3> packed_to_n() const {
+        return {{field_of(0, g.lvec, lm), field_of(g.lvec, g.lb, 0), field_of(g.ll, g.lp, g.lb)}};
+    }
+    // tile (before the repack): sample n = jj M + gm B + j in local index
+    // jj B + j of member gm, L elements apart
+    BitMap<4> tile_lines(int axis) const { return lines(axis, 0, 2 * g.ll); }
+    BitMap<3> tile(int axis) const {
+        return {{field_of(0, g.lb, g.ll), field_of(g.lb, g.lp, member(axis)), field_of(lm, g.lvec, g.lb + g.ll)}};
+    }
+    // both ends of pass `kind` along `axis`
+    void ends(LinePass kind, int axis, bool tiled, LinePassArgs* a) const {
+        const BitMap<4> rl = row_lines(axis, tiled), tl = tile_lines(axis);
+        const BitMap<3> rn = row(axis), tn = tile(axis), pn = packed(axis);
+        const bool tin = kind == LP_TILE_FWD || kind == LP_TILE_SPEC, tout = kind == LP_TILE_INV || kind == LP_TILE_SPEC;
+        const bool pin = kind == LP_ROW_FWD || kind == LP_ROW_SPEC, pout = kind == LP_ROW_INV || kind == LP_ROW_SPEC;
+        a->in_l = tin ? tl : rl;
+        a->in_n = tin ? tn : pin ? pn : rn;
+        a->out_l = tout ? tl : rl;
+        a->out_n = tout ? tn : pout ? pn : rn;
+        a->pk = packed_to_n();
+    }
+};
+
+}  // namespace zm

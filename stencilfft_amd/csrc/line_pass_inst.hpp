@@ -1,0 +1,149 @@
+// line_pass_inst.hpp -- instances and dispatch of the natural-order line
+// passes for one storage precision; included by line_pass_f32.hip and
+// line_pass_f64.hip, which compile in parallel.
+#pragma once
+
+#include "line_pass.hpp"
+
+namespace zm {
+namespace lp {
+
+constexpr size_t kLdsLimit = 160 * 1024;
+
+// Row and tile passes of 2^LN-point lines: log2 of the elements per thread and
+// of the lines per workgroup (and of the lines in the small variant), mode;
+// -1 lines: not built.  RADIX16: the alternative split of a plan that prefers
+// the largest radices (line_pass_radix16).
+template <typename T, int LN, bool RADIX16>
+struct Split {
+    static constexpr int row_ept = 4, row = -1, row_small = -1, tile_ept = 4, tile = -1, tile_small = -1;
+    static constexpr Mode row_mode = ONCE, tile_mode = ONCE;
+};
+#define ZM_SPLIT(T, LN, R16, RE, RL, RS, RM, TE, TL, TS, TM)                   \
+    template <>                                                                \
+    struct Split<T, LN, R16> {                                                 \
+        static constexpr int row_ept = RE, row = RL, row_small = RS;           \
+        static constexpr Mode row_mode = RM;                                   \
+        static constexpr int tile_ept = TE, tile = TL, tile_small = TS;        \
+        static constexpr Mode tile_mode = TM;                                  \
+    };
+
+constexpr bool is_row(int kind) { return kind == LP_ROW_FWD || kind == LP_ROW_INV || kind == LP_ROW_SPEC; }
+
+template <typename T, int LN, bool R16, int KIND, bool SMALL>
+struct Inst {
+    using S = Split<T, LN, R16>;
+    static constexpr bool ROWS = is_row(KIND);
+    static constexpr int LNP = LN, LLP = ROWS ? (SMALL ? S::row_small : S::row) : (SMALL ? S::tile_small : S::tile);
+    // multiplier tiles with at most 512 threads (256 VGPRs; the radices, and so
+    // the tables, are the same)
+    static constexpr int LEPT0 = ROWS ? S::row_ept : S::tile_ept;
+    static constexpr int LEPT = KIND == LP_TILE_SPEC && LN + LLP - LEPT0 > 9 ? LN + LLP - 9 : LEPT0;
+    // row multipliers only where no tile is built (FP64 N = 8192 spills)
+    static constexpr bool built =
+        LLP >= 0 && (KIND != LP_ROW_SPEC || (S::tile < 0 && !(sizeof(T) == 8 && LN == 13)));
+    static constexpr Mode MODE = SMALL ? ONCE : ROWS ? S::row_mode : S::tile_mode;
+    static constexpr int IN = KIND == LP_ROW_FWD || KIND == LP_ROW_SPEC    ? PACKED
+                              : KIND == LP_ROW_INV || KIND == LP_TILE_INV ? ROW
+                                                                          : TILE;
+    static constexpr int OUT = KIND == LP_ROW_INV || KIND == LP_ROW_SPEC    ? PACKED
+                               : KIND == LP_ROW_FWD || KIND == LP_TILE_FWD ? ROW
+                                                                           : TILE;
+    static constexpr int DIR = KIND == LP_TILE_SPEC || KIND == LP_ROW_SPEC ? SPEC
+                               : KIND == LP_ROW_INV || KIND == LP_TILE_INV ? INV
+                                                                           : FWD;
+    using K = Line<T, LN, LLP < 0 ? 4 : LLP, LEPT>;
+    static constexpr size_t lds() {
+        static_assert(K::lds_bytes(MODE == LOOP_LDS) <= kLdsLimit, "LDS");
+        return K::lds_bytes(MODE == LOOP_LDS);
+    }
+    static const void* fn() { return (const void*)&line_pass_kernel<T, LN, LLP, LEPT, IN, OUT, DIR, MODE>; }
+    static hipError_t prepare() {
+        if (lds() <= 65536) return hipSuccess;
+        return hipFuncSetAttribute(fn(), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds());
+    }
+};
+
+template <typename T, typename Op>
+auto with_line_pass(int kind, const LinePassSize& size, Op&& op) {
+#define ZM_LP3(LN, R16, KIND, SM)                                                 \
+    if constexpr (Inst<T, LN, R16, KIND, SM>::built) {                            \
+        if (size.ln == LN && size.radix16 == R16 && kind == KIND && size.small == SM) \
+            return op.template run<Inst<T, LN, R16, KIND, SM>>();                 \
+    }
+#define ZM_LP2(LN, R16, KIND) ZM_LP3(LN, R16, KIND, false) ZM_LP3(LN, R16, KIND, true)
+#define ZM_LP1(LN, KIND) ZM_LP2(LN, false, KIND) ZM_LP2(LN, true, KIND)
+#define ZM_LP(LN) \
+    ZM_LP1(LN, LP_ROW_FWD) ZM_LP1(LN, LP_ROW_INV) ZM_LP1(LN, LP_TILE_FWD) ZM_LP1(LN, LP_TILE_INV)
+    ZM_LP(4) ZM_LP(5) ZM_LP(6) ZM_LP(7) ZM_LP(8) ZM_LP(9) ZM_LP(10) ZM_LP(11) ZM_LP(12) ZM_LP(13)
+#undef ZM_LP
+#undef ZM_LP1
+#undef ZM_LP2
+#undef ZM_LP3
+    return op.none();
+}
+
+struct InfoOp {
+    template <typename I>
+    LinePassInfo run() {
+        LinePassInfo r{I::LLP, 0, I::MODE != ONCE, I::K::TW};
+        if (I::prepare() != hipSuccess ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&r.occupancy, I::fn(), I::K::NT, I::lds()) != hipSuccess)
+            r.occupancy = 0;
+        return r;
+    }
+    LinePassInfo none() { return LinePassInfo{-1, 0, false, 0}; }
+};
+
+template <typename T>
+struct TablesOp {
+    Cx<T>* out;
+    hipStream_t stream;
+    template <typename I>
+    hipError_t run() {
+        hipLaunchKernelGGL((line_pass_tables_kernel<T, I::LNP, I::LEPT>), dim3((I::K::TW + 255) / 256), dim3(256), 0,
+                           stream, out);
+        return hipGetLastError();
+    }
+    hipError_t none() { return hipErrorInvalidValue; }
+};
+
+template <typename T>
+struct LaunchOp {
+    const Cx<T>* in;
+    Cx<T>* out;
+    const LinePassArgs& a;
+    const Cx<T>* tables;
+    T scale;
+    const SpectralArgs& sp;
+    int grid;
+    hipStream_t stream;
+    template <typename I>
+    hipError_t run() {
+        const hipError_t e = I::prepare();
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL((line_pass_kernel<T, I::LNP, I::LLP, I::LEPT, I::IN, I::OUT, I::DIR, I::MODE>),
+                           dim3((unsigned)grid), dim3(I::K::NT), I::lds(), stream, in, out, a, tables, scale, sp);
+        return hipGetLastError();
+    }
+    hipError_t none() { return hipErrorInvalidValue; }
+};
+
+}  // namespace lp
+
+template <typename T>
+LinePassInfo line_pass_info(LinePass kind, const LinePassSize& size) {
+    return lp::with_line_pass<T>((int)kind, size, lp::InfoOp{});
+}
+template <typename T>
+hipError_t launch_line_pass_tables(LinePass kind, const LinePassSize& size, Cx<T>* tables, hipStream_t stream) {
+    return lp::with_line_pass<T>((int)kind, size, lp::TablesOp<T>{tables, stream});
+}
+template <typename T>
+hipError_t launch_line_pass(LinePass kind, const LinePassSize& size, const Cx<T>* in, Cx<T>* out, const LinePassArgs& a,
+                            const Cx<T>* tables, double scale, const SpectralArgs& sp, int grid, hipStream_t stream) {
+    return lp::with_line_pass<T>((int)kind, size,
+                                 lp::LaunchOp<T>{in, out, a, tables, (T)scale, sp, grid, stream});
+}
+
+}  // namespace zm

@@ -12,6 +12,7 @@
 
 #include "../../include/stencilfft.h"
 #include "kernels.hpp"
+#include "line_maps.hpp"
 #include "maps.hpp"
 
 using zm::Geo;
@@ -37,12 +38,24 @@ struct zm_plan {
     float2* ltab32;
     int fast_grid_fwd, fast_grid_inv;
     int fast_grid_lapx;  // the fused Laplacian + x pass's grid (0: not built for this plan)
+    // natural-order line passes (line_pass.hpp) by axis; grid 0: not used
+    struct NatPass {
+        zm::LinePass kind;
+        zm::LinePassSize size;
+        int grid;
+        const void* tables;
+        zm::LinePassArgs args;
+    };
+    NatPass nat_fwd[3], nat_inv[3];
+    bool tiled;            // the passes after the first axis hold the repacks
+    void* nat_tables[2];  // twiddles of the row and of the tile passes
     // per-stage timing (zm_timing_*)
     bool timing;
     struct Timed {
         int stage;
         hipEvent_t start, stop;
         bool own_start;  // start is this entry's own event, not the previous launch's stop
+        bool own_stop;   // false: a stage that ran inside the previous launch (start == stop, no time of its own)
     };
     std::vector<Timed> timed;
     hipEvent_t last_stop;  // completion event of the previous timed launch
@@ -60,7 +73,7 @@ namespace {
 template <typename F>
 hipError_t timed_launch(zm_plan* p, int stage, hipStream_t stream, F&& launch, bool record = true) {
     if (!p->timing || !record) return launch();
-    zm_plan::Timed t{stage, nullptr, nullptr, false};
+    zm_plan::Timed t{stage, nullptr, nullptr, false, true};
     hipError_t e = hipSuccess;
     if (p->last_stop && p->last_stream == stream) {
         t.start = p->last_stop;
@@ -83,10 +96,17 @@ hipError_t timed_launch(zm_plan* p, int stage, hipStream_t stream, F&& launch, b
     return e;
 }
 
+// A stage that ran inside the launch just timed: counted, with no time of its
+// own (the launch's stage holds it).
+void timed_inside(zm_plan* p, int stage, bool record) {
+    if (p->timing && record && p->last_stop)
+        p->timed.push_back(zm_plan::Timed{stage, p->last_stop, p->last_stop, false, false});
+}
+
 void drop_timing(zm_plan* p) {
     for (auto& t : p->timed) {
         if (t.own_start) (void)hipEventDestroy(t.start);
-        (void)hipEventDestroy(t.stop);
+        if (t.own_stop) (void)hipEventDestroy(t.stop);
     }
     p->timed.clear();
     p->last_stop = nullptr;
@@ -162,6 +182,89 @@ int ipow(int a, int e) {
 constexpr int kLineTarget = 4096;
 constexpr int kStageTarget = 4096;
 constexpr size_t kMaxLds = 160 * 1024;
+
+// FP64 lines of 256 points run as 16 x 16 on at most two ranks per axis and as
+// 8 x 8 x 4 on more.  16 x 16 rounds once less: the FP64 rounding noise of a
+// 32-step 256^3 rollout is 6.1e-7 against 1.0e-6 of its gradient, at equal
+// speed (four 256^3 fields, P = 2: forward 1.135 against 1.131 ms, inverse
+// 1.149 against 1.081).  But its last pass stores runs of 16 / P values: P = 4
+// 0.357 against 0.300 ms, P = 8 0.820 against 0.290.
+zm::LinePassSize nat_size(const Geo& g, bool fp64) {
+    return zm::LinePassSize{g.ln, false, fp64 && g.ln == 8 && g.p <= 2};
+}
+
+// The pass `kind` along `axis`, or grid 0 where it is not built.
+template <typename T>
+zm_plan::NatPass nat_pass(const zm_plan* p, int cus, zm::LinePass kind, int axis) {
+    const Geo& g = p->geo;
+    const zm::NatMaps m(g);
+    zm_plan::NatPass np{kind, nat_size(g, sizeof(T) == 8), 0, nullptr, {}};
+    const int lines = g.ln * (g.dims - 1);  // log2 of the lines per field
+    zm::LinePassInfo info = zm::line_pass_info<T>(kind, np.size);
+    if (info.lines_log2 < 0) return np;
+    // too few groups to fill the CUs: fewer lines per group
+    if (((int64_t)p->batch << (lines - info.lines_log2)) < cus) {
+        np.size.small = true;
+        const zm::LinePassInfo si = zm::line_pass_info<T>(kind, np.size);
+        if (si.lines_log2 >= 0) info = si;
+        else np.size.small = false;
+    }
+    const int64_t groups = (int64_t)p->batch << (lines - info.lines_log2);
+    if (info.occupancy <= 0 || groups > INT32_MAX) return np;
+    const int64_t resident = (int64_t)info.occupancy * cus;
+    np.grid = (int)(info.loop && resident < groups ? resident : groups);
+    const bool rows = kind == zm::LP_ROW_FWD || kind == zm::LP_ROW_INV;
+    np.tables = p->nat_tables[rows ? 0 : 1];
+    zm::LinePassArgs& a = np.args;
+    a.lgroups = lines - info.lines_log2;
+    a.groups = (int)groups;
+    // tile loads of consecutive groups share the cache lines of shorter runs
+    // and DRAM pages: 512^3 FP32 y + z 0.83 -> 0.80 ms, 2048^2 FP32 0.32 ->
+    // 0.25 ms; stores do not (2048^2 FP64 0.223 -> 0.234 ms), nor do short
+    // lines (128^3 FP32 0.091 -> 0.107 ms)
+    a.xcd = kind == zm::LP_TILE_FWD && g.ln >= 9;
+    a.field = g.field;
+    m.ends(kind, axis, p->tiled, &a);
+    return np;
+}
+
+// The twiddle tables and passes of a plan's natural-order line passes.
+template <typename T>
+hipError_t choose_nat_passes(zm_plan* p, int cus) {
+    const int ln = p->geo.ln, d = p->geo.dims;
+    const zm::LinePass kinds[2] = {zm::LP_ROW_FWD, zm::LP_TILE_FWD};
+    for (int i = 0; i < 2; i++) {
+        const zm::LinePassSize size = nat_size(p->geo, sizeof(T) == 8);
+        const zm::LinePassInfo info = zm::line_pass_info<T>(kinds[i], size);
+        if (info.lines_log2 < 0) continue;
+        hipError_t e = hipMalloc(&p->nat_tables[i], sizeof(zm::Cx<T>) * (size_t)info.tables);
+        if (e == hipSuccess) e = zm::launch_line_pass_tables<T>(kinds[i], size, (zm::Cx<T>*)p->nat_tables[i], nullptr);
+        if (e != hipSuccess) return e;
+    }
+    p->tiled = p->nat_tables[1] != nullptr;
+    for (int axis = 1; axis < d && p->tiled; axis++) {
+        p->nat_fwd[axis] = nat_pass<T>(p, cus, zm::LP_TILE_FWD, axis);
+        p->nat_inv[axis] = nat_pass<T>(p, cus, zm::LP_TILE_INV, axis);
+        if (!p->nat_fwd[axis].grid || !p->nat_inv[axis].grid) p->tiled = false;
+    }
+    // At N >= 4096 the specialised pass (line_fast.hip) is as fast or faster as
+    // a row pass where it is built (forward + inverse: 4096^2 FP32 0.293
+    // against 0.306 ms, eight fields 2.43 against 2.32; 8192^2 FP32 line 0.20
+    // against 0.22-0.23 ms); elsewhere the generic one took 8192^2, P = 1,
+    // B = 32 4.54 against 1.46 ms.
+    const bool rows = p->nat_tables[0] && !(ln >= 12 && p->fast);
+    for (int axis = 0; axis < d; axis++) {
+        if (axis > 0 && p->tiled) break;
+        p->nat_fwd[axis] = p->nat_inv[axis] = zm_plan::NatPass{};
+        if (!rows) continue;
+        // the forward x pass keeps the fused Laplacian's radix order where the
+        // plan has that pass: zm_laplace_forward is bit for bit
+        // zm_forward(zm_laplace)
+        if (axis > 0 || !p->fast_grid_lapx) p->nat_fwd[axis] = nat_pass<T>(p, cus, zm::LP_ROW_FWD, axis);
+        p->nat_inv[axis] = nat_pass<T>(p, cus, zm::LP_ROW_INV, axis);
+    }
+    return hipSuccess;
+}
 
 }  // namespace
 
@@ -318,8 +421,16 @@ zm_status zm_plan_create(zm_plan** plan, const zm_shape* shape, zm_precision pre
             }
         }
     }
+    // the natural-order line passes (FP64 and FP32 vector ALU)
+    if (e == hipSuccess && !two_stage && !mfma) {
+        int cus = 0;
+        e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
+        if (e == hipSuccess) e = fp64 ? choose_nat_passes<double>(p, cus) : choose_nat_passes<float>(p, cus);
+    }
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess || (mfma && !p->fast)) {
+        for (void* t : p->nat_tables)
+            if (t) (void)hipFree(t);
         (void)hipFree(p->tw64);
         (void)hipFree(p->tw32);
         if (p->ltab64) (void)hipFree(p->ltab64);
@@ -339,6 +450,8 @@ zm_status zm_plan_destroy(zm_plan* p) {
     if (p->tw32 && hipFree(p->tw32) != hipSuccess) st = ZM_ERR_DEVICE;
     if (p->ltab64 && hipFree(p->ltab64) != hipSuccess) st = ZM_ERR_DEVICE;
     if (p->ltab32 && hipFree(p->ltab32) != hipSuccess) st = ZM_ERR_DEVICE;
+    for (void* t : p->nat_tables)
+        if (t && hipFree(t) != hipSuccess) st = ZM_ERR_DEVICE;
     if (p->own_scratch && hipFree(p->own_scratch) != hipSuccess) st = ZM_ERR_DEVICE;
     drop_timing(p);
     delete p;
@@ -413,9 +526,26 @@ struct Exec {
     const zm::Cx<T>* line_tables() const {
         return p->precision == ZM_FP64 ? (const zm::Cx<T>*)p->ltab64 : (const zm::Cx<T>*)p->ltab32;
     }
+    // natural-order line pass of one axis; a tile pass holds a repack stage,
+    // counted inside it
+    zm_status nat(const zm_plan::NatPass& np, const void* in, void* out, double scale) const {
+        const hipError_t e = timed_launch(p, ZM_STAGE_LINE, st, [&] {
+            return zm::launch_line_pass<T>(np.kind, np.size, (const zm::Cx<T>*)in, (zm::Cx<T>*)out,
+                                           np.args, (const zm::Cx<T>*)np.tables, scale, zm::SpectralArgs{}, np.grid,
+                                           st);
+        }, record);
+        if (e == hipSuccess && (np.kind == zm::LP_TILE_FWD || np.kind == zm::LP_TILE_INV))
+            timed_inside(p, ZM_STAGE_REPACK, record);
+        return launch_status(e);
+    }
+    // whether the transforms run without repack launches
+    bool tiled() const { return compute && p->tiled; }
+
     // lapx: the x pass of zm_laplace_forward (fast_grid_lapx != 0 only),
     // transforming `scale` times the input's Laplacian
     zm_status line(const void* in, void* out, int axis, bool fwd, double scale, bool lapx = false) const {
+        const zm_plan::NatPass& np = fwd ? p->nat_fwd[axis] : p->nat_inv[axis];
+        if (compute && !lapx && np.grid) return nat(np, in, out, scale);
         zm::LineArgs a{axis_stride(p, axis), (int)(p->dims.local / p->dims.l), p->lpb};
         if (p->fast && compute) {
             const int grid = lapx ? p->fast_grid_lapx : fwd ? p->fast_grid_fwd : p->fast_grid_inv;
@@ -454,11 +584,19 @@ struct Exec {
     }
 
     // forward_fft / forward_fft_3d (zmodel/transforms/fft.cu:199-339,
-    // fft3d.cu:234-412) as x-pass, repack, y-pass [, repack-yz, z-pass].
-    zm_status forward(const void* in, void* out, void* s) const {
+    // fft3d.cu:234-412) as x-pass, repack, y-pass [, repack-yz, z-pass]; with
+    // the tiled passes the repacks are part of the passes after them.
+    zm_status forward(const void* in, void* out, void* s, bool lapx = false, double lap_scale = 1.0) const {
         const bool d3 = p->shape.dims == 3;
+        if (!p->two_stage && tiled()) {
+            void* a = d3 ? out : s;
+            ZM_TRY(line(in, a, 0, true, lap_scale, lapx));
+            if (!d3) return line(s, out, 1, true, 1.0);
+            ZM_TRY(line(out, s, 1, true, 1.0));
+            return line(s, out, 2, true, 1.0);
+        }
         if (!p->two_stage) {
-            ZM_TRY(line(in, s, 0, true, 1.0));
+            ZM_TRY(line(in, s, 0, true, lap_scale, lapx));
             ZM_TRY(repack(s, out, d3 ? REPACK_XY : REPACK_2D, true));
             ZM_TRY(line(out, out, 1, true, 1.0));
             if (d3) {
@@ -495,17 +633,7 @@ struct Exec {
     // zm_forward(zm_laplace(in)).
     zm_status laplace_forward(const void* in, void* out, void* s, double lap_scale) const {
         if (p->two_stage) return ZM_ERR_UNSUPPORTED;
-        if (p->fast_grid_lapx > 0) {
-            const bool d3 = p->shape.dims == 3;
-            ZM_TRY(line(in, s, 0, true, lap_scale, true));
-            ZM_TRY(repack(s, out, d3 ? REPACK_XY : REPACK_2D, true));
-            ZM_TRY(line(out, out, 1, true, 1.0));
-            if (d3) {
-                ZM_TRY(repack(out, s, REPACK_YZ, true));
-                ZM_TRY(line(s, out, 2, true, 1.0));
-            }
-            return ZM_OK;
-        }
+        if (p->fast_grid_lapx > 0) return forward(in, out, s, true, lap_scale);
         ZM_TRY(launch_status(timed_launch(p, ZM_STAGE_LAPLACE, st, [&] {
             return zm::launch_stencil<T>(in, out, p->geo, p->batch, zm::OP_LAPLACE, true, lap_scale, false, st);
         }, record)));
@@ -516,6 +644,15 @@ struct Exec {
     // fft3d.cu:508-633): the reverse chain, scale applied once on the x-pass.
     zm_status inverse(const void* in, void* out, void* s, double scale) const {
         const bool d3 = p->shape.dims == 3;
+        if (!p->two_stage && tiled()) {
+            if (!d3) {
+                ZM_TRY(line(in, s, 1, false, 1.0));
+                return line(s, out, 0, false, scale);
+            }
+            ZM_TRY(line(in, s, 2, false, 1.0));
+            ZM_TRY(line(s, out, 1, false, 1.0));
+            return line(out, out, 0, false, scale);
+        }
         if (!p->two_stage) {
             if (d3) {
                 ZM_TRY(line(in, s, 2, false, 1.0));
@@ -826,7 +963,7 @@ zm_status zm_timing_read(zm_plan* p, zm_stage stage, int* count, double* total_m
         if (t.stage != (int)stage) continue;
         if (hipEventSynchronize(t.stop) != hipSuccess) return ZM_ERR_DEVICE;
         float ms = 0.f;
-        if (hipEventElapsedTime(&ms, t.start, t.stop) != hipSuccess) return ZM_ERR_DEVICE;
+        if (t.own_stop && hipEventElapsedTime(&ms, t.start, t.stop) != hipSuccess) return ZM_ERR_DEVICE;
         tot += ms;
         c++;
     }

@@ -3,6 +3,7 @@
 #include "common.hpp"
 #include "kernels.hpp"
 #include "maps.hpp"
+#include "spectral_math.hpp"
 
 namespace zm {
 
@@ -42,8 +43,6 @@ __device__ __forceinline__ Coord decode_coord(const Geo& g, int64_t i) {
     c.did = (g.dims == 3) ? (id >> (2 * g.lp)) : 0;
     return c;
 }
-
-__device__ __forceinline__ int signed_wavenumber(int k, int n) { return k <= n / 2 ? k : k - n; }
 
 // Frequencies of element i of the reciprocal layout: 2D kx <- (cid, lr),
 // ky <- (rid, lc) (zmodel/utils.h:265-268); 3D kc <- (cid, lr),

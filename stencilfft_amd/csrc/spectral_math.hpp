@@ -1,0 +1,78 @@
+// spectral_math.hpp -- the reciprocal-space multipliers, evaluated in FP64 for
+// every storage precision, shared by the standalone multiplier kernel
+// (spectral.hip) and the line passes that apply one between a forward and an
+// inverse transform (line_pass.hpp).
+#pragma once
+
+#include "common.hpp"
+#include "kernels.hpp"
+
+namespace zm {
+
+__device__ __forceinline__ int signed_wavenumber(int k, int n) { return k <= n / 2 ? k : k - n; }
+
+// The part of a multiplier that one line of the last transform axis shares:
+// the sum of squared wavenumbers and of squared half-angle sines of the other
+// axes, and the imaginary part of the dx4 symbol (2D, axis 0).
+struct LineSymbol {
+    double k2, h2, im;
+};
+
+// Kinds: 0 Poisson -1/|k|^2 (k = 0 -> 0), 1 heat exp(-p0 |k|^2 p1), 2 constant
+// p0, 3 stencil symbol (Laplacian scale p0, dx4 delta p1), 4 Poisson times the
+// stencil symbol.
+//
+// The stencil symbol is that of the periodic 5-/7-point Laplacian (scaled by
+// p0) plus, in 2D, the 4th-order x-derivative [1, -8, 0, 8, -1] / (12 delta)
+// when delta != 0: for the mode exp(2 pi i k x / N), theta = 2 pi k / N,
+//   Laplacian: p0 * sum_d (2 cos theta_d - 2) = -4 p0 sum_d sin^2(theta_d / 2)
+//   dx4:       i (8 sin theta_x - sin 2 theta_x) / (6 delta)
+// (the sin^2 form has no cancellation at small k).  Axis 0 is the
+// packed-column (gc) wavenumber, the axis zm_dx4 differentiates.
+__device__ __forceinline__ LineSymbol line_symbol(const SpectralArgs& sp, int f0, int f1, int n) {
+    LineSymbol ls{0.0, 0.0, 0.0};
+    const int s0 = signed_wavenumber(f0, n), s1 = signed_wavenumber(f1, n);
+    ls.k2 = (double)s0 * s0 + (sp.dims == 3 ? (double)s1 * s1 : 0.0);
+    if (sp.kind >= 3) {
+        const double inv_n = 1.0 / (double)n;
+        double h = sinpi((double)s0 * inv_n);
+        ls.h2 = h * h;
+        if (sp.dims == 3) {
+            h = sinpi((double)s1 * inv_n);
+            ls.h2 += h * h;
+        }
+        if (sp.p1 != 0.0) {
+            const double t = 2.0 * (double)s0 * inv_n;  // theta_x / pi
+            ls.im = (8.0 * sinpi(t) - sinpi(2.0 * t)) / (6.0 * sp.p1);
+            if (sp.conj) ls.im = -ls.im;
+        }
+    }
+    return ls;
+}
+
+// The multiplier at frequency f of the last axis; half_sin[f] = sin(pi s / N)
+// of its signed wavenumber s.
+__device__ __forceinline__ void line_multiplier(const SpectralArgs& sp, const LineSymbol& ls, int f, int n, double* mr,
+                                                double* mi) {
+    const int s = signed_wavenumber(f, n);
+    const double k2 = sp.kscale * sp.kscale * (ls.k2 + (double)s * s);
+    *mi = 0.0;
+    if (sp.kind == 0) {
+        *mr = (k2 == 0.0) ? 0.0 : -1.0 / k2;  // 1 / (-|k|^2), mean mode removed
+    } else if (sp.kind == 1) {
+        *mr = exp(-sp.p0 * k2 * sp.p1);  // heat: exp(-nu |k|^2 dt)
+    } else if (sp.kind == 2) {
+        *mr = sp.p0;
+    } else {
+        const double h = sp.half_sin[f];
+        *mr = -4.0 * sp.p0 * (ls.h2 + h * h);
+        *mi = ls.im;
+        if (sp.kind == 4) {
+            const double poisson = (k2 == 0.0) ? 0.0 : -1.0 / k2;
+            *mr *= poisson;
+            *mi *= poisson;
+        }
+    }
+}
+
+}  // namespace zm
