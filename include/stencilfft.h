@@ -239,6 +239,18 @@ zm_status zm_spectral_multiply(zm_plan* plan, const void* in, void* out, zm_spec
 zm_status zm_spectral_multiply_adjoint(zm_plan* plan, const void* in, void* out, zm_spectral kind, double p0,
                                        double p1, double length, void* stream);
 
+/* out = zm_inverse(scale) of the multiplier of zm_forward(in): a spectral
+ * solve on real-space fields (Poisson, heat, ..), and its adjoint, the same
+ * with the conjugate multiplier (the forward and inverse adjoints cancel).
+ * The last axis's two passes and the multiplier run as one kernel where the
+ * plan has it (N <= 2048, 2D N = 4096, 2D FP32 N = 8192; FP64 and FP32 vector
+ * ALU), else as the three calls; the values agree with them to rounding.
+ * ZM_PATH_TWO_STAGE plans get ZM_ERR_UNSUPPORTED.  Buffers as zm_forward. */
+zm_status zm_spectral_solve(zm_plan* plan, const void* in, void* out, zm_spectral kind, double p0, double p1,
+                            double length, double scale, void* scratch, void* stream);
+zm_status zm_spectral_solve_adjoint(zm_plan* plan, const void* in, void* out, zm_spectral kind, double p0, double p1,
+                                    double length, double scale, void* scratch, void* stream);
+
 /* ---------------------------------------------------------------------- */
 /* index maps (host, pure, thread-safe): zmodel/utils.h:99-320             */
 /* ---------------------------------------------------------------------- */

@@ -89,6 +89,8 @@ SIGNATURES = {
     "zm_dz4_adjoint": (_I, [_VP, _VP, _VP, _D, _I, _VP]),
     "zm_spectral_multiply": (_I, [_VP, _VP, _VP, _I, _D, _D, _D, _VP]),
     "zm_spectral_multiply_adjoint": (_I, [_VP, _VP, _VP, _I, _D, _D, _D, _VP]),
+    "zm_spectral_solve": (_I, [_VP, _VP, _VP, _I, _D, _D, _D, _D, _VP, _VP]),
+    "zm_spectral_solve_adjoint": (_I, [_VP, _VP, _VP, _I, _D, _D, _D, _D, _VP, _VP]),
     "zm_packed_to_block_cyclic": (_I, [_SP, _I]),
     "zm_block_cyclic_to_packed": (_I, [_SP, _I]),
     "zm_real_to_global": (None, [_SP, _I, _I, _I, _I, _IP, _IP]),

@@ -9,6 +9,8 @@ adjoint, computed by the library's adjoint entry points:
                           transposed stencil, -dx4)
   spectral multiplier  -> zm_spectral_multiply_adjoint (conjugate multiplier;
                           the real kinds are self-adjoint)
+  spectral solve       -> zm_spectral_solve_adjoint (the conjugate multiplier
+                          between the same two transforms)
 For complex tensors torch passes dL/d(conj y) and expects A^H of it back, which
 is exactly the adjoint.  No tensors are saved for backward.
 """
@@ -96,6 +98,17 @@ class _Spectral(torch.autograd.Function):
                 None, None, None, None, None)
 
 
+class _SpectralSolve(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, plan, *args):
+        ctx.plan, ctx.args = plan, args
+        return plan.spectral_solve(x.contiguous(), *args)
+
+    @staticmethod
+    def backward(ctx, g):
+        return (ctx.plan.spectral_solve(g.contiguous(), *ctx.args, adjoint=True),) + (None,) * (1 + len(ctx.args))
+
+
 def fft(x, plan):
     """forward_fft: real-space packed layout -> reciprocal layout."""
     return _Forward.apply(x, plan)
@@ -126,3 +139,10 @@ def dz4(x, plan, delta=1.0):
 
 def spectral(x, plan, kind, p0=0.0, p1=0.0, length=1.0):
     return _Spectral.apply(x, plan, kind, float(p0), float(p1), float(length))
+
+
+def spectral_solve(x, plan, kind, p0=0.0, p1=0.0, length=1.0, scale=None):
+    """ifft(spectral(fft(x))) with `scale` (default 1/N^d) as one operator."""
+    if scale is None:
+        scale = 1.0 / float(plan.shape.n) ** plan.shape.dims
+    return _SpectralSolve.apply(x, plan, kind, float(p0), float(p1), float(length), float(scale))

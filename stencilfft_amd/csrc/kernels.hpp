@@ -97,7 +97,7 @@ struct LinePassArgs {
 struct SpectralArgs {
     int kind, conj, dims;
     double p0, p1, kscale;
-    BitMap<4> f0, f1;
+    BitMap<3> f0, f1;
     const double* half_sin;  // sin(pi s / N), s the signed wavenumber of f < N
 };
 
@@ -138,6 +138,9 @@ hipError_t launch_stencil(const void* in, void* out, const Geo& g, int batch, St
 
 // twiddle tables exp(-2 pi i t / n), t in [0, n), computed in FP64
 hipError_t launch_twiddles(double2* tw64, float2* tw32, int n, hipStream_t stream);
+
+// half_sin[f] = sin(pi s / n), s the signed wavenumber of f < n
+hipError_t launch_half_sin(double* half_sin, int n, hipStream_t stream);
 
 // reciprocal-space multiplier
 template <typename T>

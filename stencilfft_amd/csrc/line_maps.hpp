@@ -54,6 +54,15 @@ struct NatMaps {
     BitMap<3> tile(int axis) const {
         return {{field_of(0, g.lb, g.ll), field_of(g.lb, g.lp, member(axis)), field_of(lm, g.lvec, g.lb + g.ll)}};
     }
+    // frequency of an axis off the last one, by lambda: its rank coordinate is
+    // at bit `rank`, its local (reciprocal) index at bit `local`
+    BitMap<3> frequency(int local, int rank) const {
+        return {{field_of(local, lvp, 0), field_of(local + lvp, g.ll - lvp, g.lvec), field_of(rank, g.lp, lvp)}};
+    }
+    // frequencies of axis 0 and (3D) axis 1 of the last axis's lines: the rows
+    // of the y pass are kx; the rows of the z pass are kc (e) and kr (y)
+    BitMap<3> frequency0() const { return d == 2 ? frequency(0, g.ll) : frequency(g.ll, 2 * g.ll); }
+    BitMap<3> frequency1() const { return d == 2 ? BitMap<3>{} : frequency(0, 2 * g.ll + g.lp); }
     // both ends of pass `kind` along `axis`
     void ends(LinePass kind, int axis, bool tiled, LinePassArgs* a) const {
         const BitMap<4> rl = row_lines(axis, tiled), tl = tile_lines(axis);

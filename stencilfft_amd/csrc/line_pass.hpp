@@ -191,6 +191,9 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
     };
     auto packed_lds = [&](int e) -> int { return (e >> LN) * K::LS + K::pad(bits(a.pk, e & (N - 1))); };
 
+    // a multiplier pass writes where it reads
+    const BitMap<4>& out_l = DIR == SPEC ? a.in_l : a.out_l;
+    const BitMap<3>& out_n = DIR == SPEC ? a.in_n : a.out_n;
     // An address is a per-thread part plus a uniform one per register, the sum
     // of the offsets of the register number's bits: radix index r (ROW, TILE)
     // or memory-order sweep k (PACKED).
@@ -199,10 +202,10 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
 #pragma unroll
     for (int i = 0; i < NB; i++) {
         in_bit[i] = IN == PACKED ? packed_off(a.in_l, a.in_n, NT << i) : bits(a.in_n, (N / RIN) << i);
-        out_bit[i] = OUT == PACKED ? packed_off(a.out_l, a.out_n, NT << i) : bits(a.out_n, (N / ROUT) << i);
+        out_bit[i] = OUT == PACKED ? packed_off(out_l, out_n, NT << i) : bits(out_n, (N / ROUT) << i);
         lds_bit[i] = packed_lds(NT << i);
     }
-    const int in_thread = packed_off(a.in_l, a.in_n, tid), out_thread = packed_off(a.out_l, a.out_n, tid),
+    const int in_thread = packed_off(a.in_l, a.in_n, tid), out_thread = packed_off(out_l, out_n, tid),
               lds_thread = packed_lds(tid);  // PACKED
     auto uniform_off = [&](const int* bit, int r) -> int {
         int o = 0;
@@ -232,7 +235,7 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
         }
     };
     auto store = [&](int g, const C* v) __attribute__((always_inline)) {
-        C* gb = out + group_base(a.out_l, g);
+        C* gb = out + group_base(out_l, g);
 #pragma unroll
         for (int k = 0; k < EPT; k++) {
             C x = v[k];
@@ -243,7 +246,7 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
                 int l, j;
                 K::template item<POUT, TOUT>(tid, k / ROUT, l, j);
                 C* p = gb + uniform_off(out_bit, k % ROUT);
-                st_nt(p + (bits(a.out_l, l) + bits(a.out_n, j)), x);
+                st_nt(p + (bits(out_l, l) + bits(out_n, j)), x);
             }
         }
     };
@@ -317,21 +320,30 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
             constexpr int R = 1 << K::lr(NP - 1);
             const int lam0 = (g & ((1 << a.lgroups) - 1)) << LLP;
             K::template write<NP - 1, true, false>(lds, v, tid);
+            auto multiply = [&](auto fc) __attribute__((always_inline)) {
+                constexpr int FAMILY = decltype(fc)::value;
 #pragma unroll 1
-            for (int k = 0; k < EPT / R; k++) {
-                int l, j;
-                K::template item<NP - 1, false>(tid, k, l, j);
-                const LineSymbol ls = line_symbol(sp, bits(sp.f0, lam0 + l), bits(sp.f1, lam0 + l), N);
+                for (int k = 0; k < EPT / R; k++) {
+                    int l, j;
+                    K::template item<NP - 1, false>(tid, k, l, j);
+                    int lam = lam0 + l;
+                    asm volatile("" : "+v"(lam));  // uniform for one-line groups: scalar registers are short
+                    // packed ends: 2D, N >= 4096
+                    const LineSymbol ls = line_symbol<FAMILY, IN == PACKED>(sp, bits(sp.f0, lam), bits(sp.f1, lam), N);
 #pragma unroll 1
-                for (int r = 0; r < R; r++) {
-                    const int f = j + r * (N / R);
-                    C* p = lds + l * K::LS + K::pad(f);
-                    double mr, mi;
-                    line_multiplier(sp, ls, f, N, &mr, &mi);
-                    const double vx = (double)p->x, vy = (double)p->y;
-                    *p = C{(T)(vx * mr - vy * mi), (T)(vx * mi + vy * mr)};
+                    for (int r = 0; r < R; r++) {
+                        const int f = j + r * (N / R);
+                        C* p = lds + l * K::LS + K::pad(f);
+                        double mr, mi;
+                        line_multiplier<FAMILY>(sp, ls, f, N, &mr, &mi);
+                        const double vx = (double)p->x, vy = (double)p->y;
+                        *p = C{(T)(vx * mr - vy * mi), (T)(vx * mi + vy * mr)};
+                    }
                 }
-            }
+            };
+            if (sp.kind == 1) multiply(IC<SF_HEAT>{});
+            else if (sp.kind >= 3) multiply(IC<SF_STENCIL>{});
+            else multiply(IC<SF_PLAIN>{});
             K::template read<NP - 1, true, false>(lds, v, tid);
         }
         if constexpr (DIR != FWD) {

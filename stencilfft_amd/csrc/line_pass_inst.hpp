@@ -42,16 +42,16 @@ struct Inst {
     // row multipliers only where no tile is built (FP64 N = 8192 spills)
     static constexpr bool built =
         LLP >= 0 && (KIND != LP_ROW_SPEC || (S::tile < 0 && !(sizeof(T) == 8 && LN == 13)));
-    static constexpr Mode MODE = SMALL ? ONCE : ROWS ? S::row_mode : S::tile_mode;
+    static constexpr int DIR = KIND == LP_TILE_SPEC || KIND == LP_ROW_SPEC ? SPEC
+                               : KIND == LP_ROW_INV || KIND == LP_TILE_INV ? INV
+                                                                           : FWD;
+    static constexpr Mode MODE = SMALL || DIR == SPEC ? ONCE : ROWS ? S::row_mode : S::tile_mode;
     static constexpr int IN = KIND == LP_ROW_FWD || KIND == LP_ROW_SPEC    ? PACKED
                               : KIND == LP_ROW_INV || KIND == LP_TILE_INV ? ROW
                                                                           : TILE;
     static constexpr int OUT = KIND == LP_ROW_INV || KIND == LP_ROW_SPEC    ? PACKED
                                : KIND == LP_ROW_FWD || KIND == LP_TILE_FWD ? ROW
                                                                            : TILE;
-    static constexpr int DIR = KIND == LP_TILE_SPEC || KIND == LP_ROW_SPEC ? SPEC
-                               : KIND == LP_ROW_INV || KIND == LP_TILE_INV ? INV
-                                                                           : FWD;
     using K = Line<T, LN, LLP < 0 ? 4 : LLP, LEPT>;
     static constexpr size_t lds() {
         static_assert(K::lds_bytes(MODE == LOOP_LDS) <= kLdsLimit, "LDS");
@@ -73,8 +73,9 @@ auto with_line_pass(int kind, const LinePassSize& size, Op&& op) {
     }
 #define ZM_LP2(LN, R16, KIND) ZM_LP3(LN, R16, KIND, false) ZM_LP3(LN, R16, KIND, true)
 #define ZM_LP1(LN, KIND) ZM_LP2(LN, false, KIND) ZM_LP2(LN, true, KIND)
-#define ZM_LP(LN) \
-    ZM_LP1(LN, LP_ROW_FWD) ZM_LP1(LN, LP_ROW_INV) ZM_LP1(LN, LP_TILE_FWD) ZM_LP1(LN, LP_TILE_INV)
+#define ZM_LP(LN)                                                                                 \
+    ZM_LP1(LN, LP_ROW_FWD) ZM_LP1(LN, LP_ROW_INV) ZM_LP1(LN, LP_TILE_FWD) ZM_LP1(LN, LP_TILE_INV) \
+    ZM_LP1(LN, LP_TILE_SPEC) ZM_LP1(LN, LP_ROW_SPEC)
     ZM_LP(4) ZM_LP(5) ZM_LP(6) ZM_LP(7) ZM_LP(8) ZM_LP(9) ZM_LP(10) ZM_LP(11) ZM_LP(12) ZM_LP(13)
 #undef ZM_LP
 #undef ZM_LP1

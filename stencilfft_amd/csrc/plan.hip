@@ -47,8 +47,10 @@ struct zm_plan {
         zm::LinePassArgs args;
     };
     NatPass nat_fwd[3], nat_inv[3];
+    NatPass nat_spec;      // the last axis forward, a spectral multiplier, and back
     bool tiled;            // the passes after the first axis hold the repacks
     void* nat_tables[2];  // twiddles of the row and of the tile passes
+    double* half_sin;      // sin(pi s / N) by frequency
     // per-stage timing (zm_timing_*)
     bool timing;
     struct Timed {
@@ -213,7 +215,7 @@ zm_plan::NatPass nat_pass(const zm_plan* p, int cus, zm::LinePass kind, int axis
     if (info.occupancy <= 0 || groups > INT32_MAX) return np;
     const int64_t resident = (int64_t)info.occupancy * cus;
     np.grid = (int)(info.loop && resident < groups ? resident : groups);
-    const bool rows = kind == zm::LP_ROW_FWD || kind == zm::LP_ROW_INV;
+    const bool rows = kind == zm::LP_ROW_FWD || kind == zm::LP_ROW_INV || kind == zm::LP_ROW_SPEC;
     np.tables = p->nat_tables[rows ? 0 : 1];
     zm::LinePassArgs& a = np.args;
     a.lgroups = lines - info.lines_log2;
@@ -263,7 +265,10 @@ hipError_t choose_nat_passes(zm_plan* p, int cus) {
         if (axis > 0 || !p->fast_grid_lapx) p->nat_fwd[axis] = nat_pass<T>(p, cus, zm::LP_ROW_FWD, axis);
         p->nat_inv[axis] = nat_pass<T>(p, cus, zm::LP_ROW_INV, axis);
     }
-    return hipSuccess;
+    p->nat_spec = nat_pass<T>(p, cus, p->tiled ? zm::LP_TILE_SPEC : zm::LP_ROW_SPEC, d - 1);
+    if (!p->nat_spec.grid) return hipSuccess;
+    const hipError_t e = hipMalloc(&p->half_sin, sizeof(double) * (size_t)p->geo.n);
+    return e == hipSuccess ? zm::launch_half_sin(p->half_sin, p->geo.n, nullptr) : e;
 }
 
 }  // namespace
@@ -429,6 +434,7 @@ zm_status zm_plan_create(zm_plan** plan, const zm_shape* shape, zm_precision pre
     }
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess || (mfma && !p->fast)) {
+        if (p->half_sin) (void)hipFree(p->half_sin);
         for (void* t : p->nat_tables)
             if (t) (void)hipFree(t);
         (void)hipFree(p->tw64);
@@ -450,6 +456,7 @@ zm_status zm_plan_destroy(zm_plan* p) {
     if (p->tw32 && hipFree(p->tw32) != hipSuccess) st = ZM_ERR_DEVICE;
     if (p->ltab64 && hipFree(p->ltab64) != hipSuccess) st = ZM_ERR_DEVICE;
     if (p->ltab32 && hipFree(p->ltab32) != hipSuccess) st = ZM_ERR_DEVICE;
+    if (p->half_sin && hipFree(p->half_sin) != hipSuccess) st = ZM_ERR_DEVICE;
     for (void* t : p->nat_tables)
         if (t && hipFree(t) != hipSuccess) st = ZM_ERR_DEVICE;
     if (p->own_scratch && hipFree(p->own_scratch) != hipSuccess) st = ZM_ERR_DEVICE;
@@ -528,14 +535,17 @@ struct Exec {
     }
     // natural-order line pass of one axis; a tile pass holds a repack stage,
     // counted inside it
-    zm_status nat(const zm_plan::NatPass& np, const void* in, void* out, double scale) const {
+    zm_status nat(const zm_plan::NatPass& np, const void* in, void* out, double scale,
+                  const zm::SpectralArgs& sp = zm::SpectralArgs{}) const {
         const hipError_t e = timed_launch(p, ZM_STAGE_LINE, st, [&] {
             return zm::launch_line_pass<T>(np.kind, np.size, (const zm::Cx<T>*)in, (zm::Cx<T>*)out,
-                                           np.args, (const zm::Cx<T>*)np.tables, scale, zm::SpectralArgs{}, np.grid,
-                                           st);
+                                           np.args, (const zm::Cx<T>*)np.tables, scale, sp, np.grid, st);
         }, record);
-        if (e == hipSuccess && (np.kind == zm::LP_TILE_FWD || np.kind == zm::LP_TILE_INV))
+        if (e == hipSuccess && np.kind >= zm::LP_TILE_FWD && np.kind <= zm::LP_TILE_SPEC)
             timed_inside(p, ZM_STAGE_REPACK, record);
+        if (e == hipSuccess && np.kind == zm::LP_TILE_SPEC) timed_inside(p, ZM_STAGE_REPACK, record);
+        if (e == hipSuccess && (np.kind == zm::LP_TILE_SPEC || np.kind == zm::LP_ROW_SPEC))
+            timed_inside(p, ZM_STAGE_SPECTRAL, record);
         return launch_status(e);
     }
     // whether the transforms run without repack launches
@@ -685,6 +695,47 @@ struct Exec {
         ZM_TRY(stage_a(s, out, 0, false, scale));
         return ZM_OK;
     }
+    zm_status multiply(const void* in, void* out, const zm::SpectralArgs& sp) const {
+        return launch_status(timed_launch(p, ZM_STAGE_SPECTRAL, st, [&] {
+            return zm::launch_spectral<T>((const zm::Cx<T>*)in, (zm::Cx<T>*)out, p->geo, p->batch, sp.kind, sp.p0,
+                                          sp.p1, sp.kscale, sp.conj != 0, st);
+        }, record));
+    }
+
+    // inverse(scale) after the multiplier after forward.  The last axis's
+    // forward pass, the multiplier and its inverse pass are one kernel, which
+    // holds the spectrum of a line group in LDS: two to four sweeps of the
+    // field less than the three calls.
+    zm_status solve(const void* in, void* out, void* s, double scale, zm::SpectralArgs sp) const {
+        const bool d3 = p->shape.dims == 3;
+        if (p->two_stage) return ZM_ERR_UNSUPPORTED;
+        if (!p->nat_spec.grid) {
+            ZM_TRY(forward(in, out, s));
+            ZM_TRY(multiply(out, out, sp));
+            return inverse(out, out, s, scale);
+        }
+        const zm::NatMaps m(p->geo);
+        sp.f0 = m.frequency0();
+        sp.f1 = m.frequency1();
+        sp.half_sin = p->half_sin;
+        if (!p->tiled) {  // 2D
+            ZM_TRY(line(in, s, 0, true, 1.0));
+            ZM_TRY(repack(s, out, REPACK_2D, true));
+            ZM_TRY(nat(p->nat_spec, out, out, 1.0, sp));
+            ZM_TRY(repack(out, s, REPACK_2D, false));
+            return line(s, out, 0, false, scale);
+        }
+        if (!d3) {
+            ZM_TRY(line(in, s, 0, true, 1.0));
+            ZM_TRY(nat(p->nat_spec, s, out, 1.0, sp));
+            return line(out, out, 0, false, scale);
+        }
+        ZM_TRY(line(in, out, 0, true, 1.0));
+        ZM_TRY(line(out, s, 1, true, 1.0));
+        ZM_TRY(nat(p->nat_spec, s, out, 1.0, sp));
+        ZM_TRY(line(out, s, 1, false, 1.0));
+        return line(s, out, 0, false, scale);
+    }
 };
 
 zm_status check_io(const zm_plan* p, const void* in, const void* out) {
@@ -821,23 +872,40 @@ zm_status zm_dz4_adjoint(zm_plan* p, const void* in, void* out, double delta, zm
     return deriv(p, in, out, delta, element, stream, zm::OP_DZ4, true);
 }
 
-static zm_status spectral(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
-                          double length, void* stream, bool conj) {
-    if (!p || !in || !out) return ZM_ERR_INVALID_ARG;
+// Checks a multiplier's parameters; fills all of its arguments but the line
+// maps of the fused pass.
+static zm_status spectral_args(const zm_plan* p, zm_spectral kind, double p0, double p1, double length, bool conj,
+                               zm::SpectralArgs* sp) {
     if ((int)kind < (int)ZM_SPECTRAL_POISSON || (int)kind > (int)ZM_SPECTRAL_POISSON_STENCIL) return ZM_ERR_INVALID_ARG;
     if (!(length > 0.0)) return ZM_ERR_INVALID_ARG;
     // the dx4 symbol is defined on the 2D layout only, like zm_dx4
     if ((kind == ZM_SPECTRAL_STENCIL || kind == ZM_SPECTRAL_POISSON_STENCIL) && p1 != 0.0 && p->shape.dims != 2)
         return ZM_ERR_INVALID_ARG;
-    const double kscale = 2.0 * M_PI / length;
+    *sp = zm::SpectralArgs{(int)kind, conj ? 1 : 0, p->shape.dims, p0, p1, 2.0 * M_PI / length, {}, {}, nullptr};
+    return ZM_OK;
+}
+
+static zm_status spectral(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
+                          double length, void* stream, bool conj) {
+    if (!p || !in || !out) return ZM_ERR_INVALID_ARG;
+    zm::SpectralArgs sp;
+    ZM_TRY(spectral_args(p, kind, p0, p1, length, conj, &sp));
     const hipStream_t st = (hipStream_t)stream;
-    return launch_status(timed_launch(p, ZM_STAGE_SPECTRAL, st, [&] {
-        if (p->precision == ZM_FP64)
-            return zm::launch_spectral<double>((const double2*)in, (double2*)out, p->geo, p->batch, (int)kind, p0, p1,
-                                               kscale, conj, st);
-        return zm::launch_spectral<float>((const float2*)in, (float2*)out, p->geo, p->batch, (int)kind, p0, p1, kscale,
-                                          conj, st);
-    }));
+    if (p->precision == ZM_FP64) return Exec<double>{p, st, true, (const double2*)p->tw64}.multiply(in, out, sp);
+    return Exec<float>{p, st, true, (const float2*)p->tw32}.multiply(in, out, sp);
+}
+
+static zm_status spectral_solve(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
+                                double length, double scale, void* scratch, void* stream, bool conj) {
+    ZM_TRY(check_io(p, in, out));
+    zm::SpectralArgs sp;
+    ZM_TRY(spectral_args(p, kind, p0, p1, length, conj, &sp));
+    void* s = nullptr;
+    ZM_TRY(scratch_for(p, scratch, &s));
+    if (s == in || s == out) return ZM_ERR_ALIAS;
+    const hipStream_t st = (hipStream_t)stream;
+    if (p->precision == ZM_FP64) return Exec<double>{p, st, true, (const double2*)p->tw64}.solve(in, out, s, scale, sp);
+    return Exec<float>{p, st, true, (const float2*)p->tw32}.solve(in, out, s, scale, sp);
 }
 
 zm_status zm_spectral_multiply(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
@@ -848,6 +916,16 @@ zm_status zm_spectral_multiply(zm_plan* p, const void* in, void* out, zm_spectra
 zm_status zm_spectral_multiply_adjoint(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
                                        double length, void* stream) {
     return spectral(p, in, out, kind, p0, p1, length, stream, true);
+}
+
+zm_status zm_spectral_solve(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
+                            double length, double scale, void* scratch, void* stream) {
+    return spectral_solve(p, in, out, kind, p0, p1, length, scale, scratch, stream, false);
+}
+
+zm_status zm_spectral_solve_adjoint(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
+                                    double length, double scale, void* scratch, void* stream) {
+    return spectral_solve(p, in, out, kind, p0, p1, length, scale, scratch, stream, true);
 }
 
 zm_status zm_real_index_table(zm_plan* p, int64_t* out, void* stream) {

@@ -27,6 +27,17 @@ hipError_t launch_twiddles(double2* tw64, float2* tw32, int n, hipStream_t strea
     return hipGetLastError();
 }
 
+__global__ void half_sin_kernel(double* half_sin, int n) {
+    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f < n) half_sin[f] = sinpi((double)signed_wavenumber(f, n) * (1.0 / (double)n));
+}
+
+hipError_t launch_half_sin(double* half_sin, int n, hipStream_t stream) {
+    const unsigned threads = 256;
+    hipLaunchKernelGGL(half_sin_kernel, dim3((n + threads - 1) / threads), dim3(threads), 0, stream, half_sin, n);
+    return hipGetLastError();
+}
+
 struct Coord {
     int did, rid, cid, ld, lr, lc;
 };

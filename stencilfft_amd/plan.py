@@ -319,6 +319,22 @@ class Plan:
                    _stream(stream)), "zm_spectral_multiply")
         return out
 
+    def spectral_solve(self, x, kind: str, p0: float = 0.0, p1: float = 0.0, length: float = 1.0, scale: float = 1.0,
+                       out=None, scratch=None, stream=None, adjoint: bool = False):
+        """inverse(m(k) forward(x), scale): the two transforms of the last axis and
+        the multiplier in one kernel where the plan has it (the three calls on
+        two-stage plans)."""
+        out = self._out(x, out)
+        if self.two_stage:
+            y = self.forward(x, scratch=scratch, stream=stream)
+            self.spectral_multiply(y, kind, p0, p1, length, out=y, stream=stream, adjoint=adjoint)
+            return self.inverse(y, scale, out=out, scratch=scratch, stream=stream)
+        sp = self._scratch(scratch, x, out)
+        fn = L._lib().zm_spectral_solve_adjoint if adjoint else L._lib().zm_spectral_solve
+        L.check(fn(self._h, _ptr(x), _ptr(out), self.SPECTRAL_KINDS[kind], float(p0), float(p1), float(length),
+                   float(scale), sp, _stream(stream)), "zm_spectral_solve")
+        return out
+
     # ---- per-stage timing (zm_timing_*) ----
     def timing(self, enable: bool = True):
         L.check(L._lib().zm_timing_enable(self._h, 1 if enable else 0), "zm_timing_enable")

@@ -26,17 +26,14 @@ from . import autograd as ag
 
 
 def poisson_solve(f, plan, length=1.0):
-    y = ag.fft(f, plan)
-    y = ag.spectral(y, plan, "poisson", length=length)
-    return ag.ifft(y, plan)
+    return ag.spectral_solve(f, plan, "poisson", length=length)
 
 
 def poisson_residual(f, g, plan, length=1.0, form="spatial"):
     """Laplacian_5pt(u) + dx4(u) - g with u = poisson_solve(f), h = delta = 1/N."""
     n = plan.shape.n
     if form == "spectral":
-        y = ag.spectral(ag.fft(f, plan), plan, "poisson_stencil", float(n * n), 1.0 / n, length)
-        return ag.ifft(y, plan) - g
+        return ag.spectral_solve(f, plan, "poisson_stencil", float(n * n), 1.0 / n, length) - g
     if form != "spatial":
         raise ValueError(f"unknown form {form!r}")
     u = poisson_solve(f, plan, length)
@@ -53,8 +50,7 @@ def poisson_loss(f, g, plan, length=1.0, form="spatial"):
 
 
 def heat_step(u, plan, nu, dt, lap_scale=1.0, length=1.0):
-    y = ag.spectral(ag.fft(u, plan), plan, "heat", nu, dt, length)
-    return ag.ifft(y, plan) + dt * ag.laplace(u, plan, scale=lap_scale)
+    return ag.spectral_solve(u, plan, "heat", nu, dt, length) + dt * ag.laplace(u, plan, scale=lap_scale)
 
 
 class _Rollout(torch.autograd.Function):
@@ -97,8 +93,6 @@ def adjoint_heat(g, plan, nsteps, nu, dt, lap_scale=1.0, length=1.0):
     adjoint kernels directly: step^H = F^H M IFFT^H + dt Lap (M real, Lap symmetric)."""
     n_d = float(plan.shape.n) ** plan.shape.dims
     for _ in range(nsteps):
-        a = plan.inverse_adjoint(g.contiguous(), 1.0 / n_d)
-        a = plan.spectral_multiply(a, "heat", nu, dt, length)
-        a = plan.forward_adjoint(a)
+        a = plan.spectral_solve(g.contiguous(), "heat", nu, dt, length, 1.0 / n_d, adjoint=True)
         g = a + dt * plan.laplace(g.contiguous(), lap_scale)
     return g

@@ -2,8 +2,9 @@
 // layout algebra (csrc/maps.hpp), over every valid (N, P, B) up to a size:
 // each end of each pass is a permutation of the field, the packed and tile ends
 // hold sample n of the line where the real-space maps put it, the row end holds
-// frequency k where the reciprocal maps do, and the passes chain: what one
-// writes as rows the next reads as tiles.  Prints the number of shapes.
+// frequency k where the reciprocal maps do, the passes chain (what one writes as
+// rows the next reads as tiles), and a multiplier's maps give the lines'
+// frequencies.  Prints the number of shapes.
 #include <cstdio>
 #include <vector>
 
@@ -49,6 +50,13 @@ static bool check(int d, int n, int p, int b) {
     const MapShape ms = make_map_shape(n, p, b);
     const NatMaps m(g);
     const int lines = d == 3 ? n * n : n, L = g.l;
+    // frequencies of the other axes for the last axis's lines
+    for (int lam = 0; lam < lines; lam++) {
+        const int y = lam & (L - 1), e = (lam >> g.ll) & (L - 1);
+        const int o = lam >> ((d - 1) * g.ll), cid = o & (p - 1), rid = o >> g.lp;
+        if (at(m.frequency0(), lam) != recip_to_freq(ms, cid, d == 2 ? y : e)) return fail("frequency 0", d, n, p, b, d - 1);
+        if (d == 3 && at(m.frequency1(), lam) != recip_to_freq(ms, rid, y)) return fail("frequency 1", d, n, p, b, 2);
+    }
     for (int tiled = 0; tiled < 2; tiled++)
         for (int axis = 0; axis < d; axis++)
             for (int kind = LP_ROW_FWD; kind <= LP_ROW_SPEC; kind++) {
