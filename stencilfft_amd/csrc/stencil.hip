@@ -351,6 +351,17 @@ __global__ void __launch_bounds__(256) deriv4_march_kernel(const E* __restrict__
 // Longer strips re-read fewer halo positions; shorter ones give more
 // workgroups: neither wins everywhere.
 // A K that does not divide the line count falls back to K=1.
+// Where those shapes give fewer than kMarchFill workgroups (two per CU), a
+// smaller field would leave CUs idle: one line per thread and strips halved
+// down to kMarchShort positions until there are about four (z: eight) per CU.
+// dy4 1024^2 FP32 86 -> 5.4 us (8 workgroups before), 4096^2 FP32 129 -> 55;
+// dx4 2048^2 FP32 26 -> 16; dz4 256^3 FP32 160 -> 57, real FP64 155 -> 57,
+// 64^3 31 -> 4.3.  With the limit at 1024 workgroups dz4 512^3 took 0.434
+// against 0.407 ms; with the z target for y, dy4 4096^2 67 against 55 us.
+constexpr int kMarchFill = 512, kMarchShort = 8;
+template <int AXIS>
+constexpr int kMarchTarget = AXIS == 2 ? 2048 : 1024;
+
 template <typename E, typename S, int AXIS, int K, int RING, int AHEAD, bool NTL>
 static hipError_t launch_march(const E* in, E* out, const Geo& g, int batch, int lines, int len, int tmax, S denom,
                                bool negate, hipStream_t stream, int order = 0) {
@@ -359,10 +370,17 @@ static hipError_t launch_march(const E* in, E* out, const Geo& g, int batch, int
             return launch_march<E, S, AXIS, 1, 16, 12, NTL>(in, out, g, batch, lines, len, tmax, denom, negate, stream,
                                                             order);
     }
-    const int T = len < tmax ? len : tmax;
+    int T = len < tmax ? len : tmax;
+    const int64_t sets = ((int64_t)lines + 256 * K - 1) / (256 * K);
+    if (sets * (len / T) * batch < kMarchFill) {
+        if constexpr (K > 1)
+            return launch_march<E, S, AXIS, 1, 16, 12, NTL>(in, out, g, batch, lines, len, tmax, denom, negate, stream,
+                                                            order);
+        while (T > kMarchShort && sets * (len / T) * batch < kMarchTarget<AXIS>) T >>= 1;
+    }
     int lstrips = 0;
     while ((T << lstrips) < len) lstrips++;
-    const unsigned blocks = (unsigned)(((int64_t)lines + 256 * K - 1) / (256 * K)) << lstrips;
+    const unsigned blocks = (unsigned)sets << lstrips;
     hipLaunchKernelGGL((deriv4_march_kernel<E, S, AXIS, K, RING, AHEAD, NTL>), dim3(blocks, (unsigned)batch),
                        dim3(256), 0, stream, in, out, g, T, lstrips, lines, denom, negate ? 1 : 0, order);
     return hipGetLastError();
@@ -764,9 +782,11 @@ static hipError_t laplace_zmarch_inst(const E* in, E* out, const Geo& g, int bat
     while ((1 << ltiles) < ntiles) ltiles++;
     // depth strips: the longest (up to 128 planes) that still gives 512
     // workgroups (two per CU); 512^3 FP32 ran 0.41 ms at 128 planes against
-    // 0.45-0.47 ms at 32-64
+    // 0.45-0.47 ms at 32-64.  Small fields go down to 4 planes: with 32 at
+    // least, 64^3 and 128^3 FP32 ran on 16 and 128 workgroups (17.0 -> 4.5,
+    // 26.3 -> 10.0 us)
     int tz = g.n < 128 ? g.n : 128;
-    while (tz > 32 && (int64_t)ntiles * g.p * (g.n / tz) * batch < 512) tz >>= 1;
+    while (tz > 4 && (int64_t)ntiles * g.p * (g.n / tz) * batch < 512) tz >>= 1;
     const unsigned blocks = (unsigned)((int64_t)ntiles * g.p * (g.n / tz));
     const size_t lds = sizeof(E) * (size_t)(R + 2) * (size_t)(g.l + 2 * g.vec);
     const bool two = 2 * R * g.vec > NTH;
