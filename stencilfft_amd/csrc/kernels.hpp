@@ -77,6 +77,14 @@ template <int K>
 struct BitMap {
     BitField f[K];
 };
+inline BitField bit_field(int from, int nbits, int to) { return BitField{from, (1 << nbits) - 1, to}; }
+template <int K>
+__device__ __forceinline__ int bits(const BitMap<K>& m, int v) {
+    int r = 0;
+#pragma unroll
+    for (int i = 0; i < K; i++) r += ((v >> m.f[i].from) & m.f[i].mask) << m.f[i].to;
+    return r;
+}
 
 // Line passes over natural-order lines (line_pass.hpp).  A line has an index
 // lambda in [0, N^(d-1)); a workgroup takes 2^lines of consecutive ones.  Each

@@ -1,5 +1,5 @@
-// line_maps.hpp -- host side of the natural-order line passes: the address maps
-// of their ends for every (N, P, B) and axis.
+// line_maps.hpp -- host side of the natural-order line passes and of the layout
+// converters: their address maps for every (N, P, B).
 #pragma once
 
 #include "kernels.hpp"
@@ -18,8 +18,6 @@ namespace zm {
 // elements apart like a y tile, where runs L^2 apart (512 KB at 512^3) cost
 // the inverse pass 11% (0.409 -> 0.368 ms, FP32).
 // ---------------------------------------------------------------------------
-inline BitField field_of(int from, int nbits, int to) { return BitField{from, (1 << nbits) - 1, to}; }
-
 struct NatMaps {
     const Geo& g;
     int d, lvp, lm, slab;
@@ -30,9 +28,9 @@ struct NatMaps {
     // lambda -> line base: y at shift `ys`, e at `es`, the ranks off `axis`
     BitMap<4> lines(int axis, int ys, int es) const {
         const int lo = member(axis == 0 ? 1 : 0), hi = member(axis == 2 ? 1 : 2);
-        if (d == 2) return {{field_of(0, g.ll, ys), field_of(g.ll, g.lp, lo), {}, {}}};
-        return {{field_of(0, g.ll, ys), field_of(g.ll, g.ll, es), field_of(2 * g.ll, g.lp, lo),
-                 field_of(2 * g.ll + g.lp, g.lp, hi)}};
+        if (d == 2) return {{bit_field(0, g.ll, ys), bit_field(g.ll, g.lp, lo), {}, {}}};
+        return {{bit_field(0, g.ll, ys), bit_field(g.ll, g.ll, es), bit_field(2 * g.ll, g.lp, lo),
+                 bit_field(2 * g.ll + g.lp, g.lp, hi)}};
     }
     // rows: the lines of a pass on its reciprocal (or packed) side
     BitMap<4> row_lines(int axis, bool tiled) const {
@@ -41,23 +39,23 @@ struct NatMaps {
     }
     // reciprocal row: k = k1 + VEC k2 -> k1 % VP + k2 VP of member k1 / VP
     BitMap<3> row(int axis) const {
-        return {{field_of(0, lvp, 0), field_of(lvp, g.lp, member(axis)), field_of(g.lvec, lm, lvp)}};
+        return {{bit_field(0, lvp, 0), bit_field(lvp, g.lp, member(axis)), bit_field(g.lvec, lm, lvp)}};
     }
     // memory-order element of the P rank rows of a packed line, and its sample n
-    BitMap<3> packed(int axis) const { return {{field_of(0, g.ll, 0), field_of(g.ll, g.lp, member(axis)), {}}}; }
+    BitMap<3> packed(int axis) const { return {{bit_field(0, g.ll, 0), bit_field(g.ll, g.lp, member(axis)), {}}}; }
     BitMap<3> packed_to_n() const {
-        return {{field_of(0, g.lvec, lm), field_of(g.lvec, g.lb, 0), field_of(g.ll, g.lp, g.lb)}};
+        return {{bit_field(0, g.lvec, lm), bit_field(g.lvec, g.lb, 0), bit_field(g.ll, g.lp, g.lb)}};
     }
     // tile (before the repack): sample n = jj M + gm B + j in local index
     // jj B + j of member gm, L elements apart
     BitMap<4> tile_lines(int axis) const { return lines(axis, 0, 2 * g.ll); }
     BitMap<3> tile(int axis) const {
-        return {{field_of(0, g.lb, g.ll), field_of(g.lb, g.lp, member(axis)), field_of(lm, g.lvec, g.lb + g.ll)}};
+        return {{bit_field(0, g.lb, g.ll), bit_field(g.lb, g.lp, member(axis)), bit_field(lm, g.lvec, g.lb + g.ll)}};
     }
     // frequency of an axis off the last one, by lambda: its rank coordinate is
     // at bit `rank`, its local (reciprocal) index at bit `local`
     BitMap<3> frequency(int local, int rank) const {
-        return {{field_of(local, lvp, 0), field_of(local + lvp, g.ll - lvp, g.lvec), field_of(rank, g.lp, lvp)}};
+        return {{bit_field(local, lvp, 0), bit_field(local + lvp, g.ll - lvp, g.lvec), bit_field(rank, g.lp, lvp)}};
     }
     // frequencies of axis 0 and (3D) axis 1 of the last axis's lines: the rows
     // of the y pass are kx; the rows of the z pass are kc (e) and kr (y)
@@ -76,5 +74,61 @@ struct NatMaps {
         a->pk = packed_to_n();
     }
 };
+
+// natural <-> packed conversion in tiles of 2^ltile elements (spectral.hip)
+struct ConvertArgs {
+    BitMap<6> nat;    // q -> natural index
+    BitMap<13> pk;    // q -> packed index
+    BitMap<3> order;  // tile element in the packed side's order (jj, r, rows) -> q
+    int ltile, lfield;
+};
+
+inline ConvertArgs convert_args(const Geo& g, int le) {
+    ConvertArgs a{};
+    const int d = g.dims, lm = g.lb + g.lp, slab = d * g.ll;
+    a.lfield = d * g.ln;
+    a.ltile = le < a.lfield ? le : a.lfield;
+    // bits of the tile: r and jj whole with rows above where they fit, else
+    // about half of the tile each
+    int lr = lm, lj = g.lvec;
+    while (lr + lj > a.ltile) {
+        if (lr > lj) lr--;
+        else lj--;
+    }
+    const int lrow = a.ltile - lr - lj, nrow = (d - 1) * g.ln;
+    a.order = {{bit_field(0, lj, lr), bit_field(lj, lr, 0), bit_field(lj + lr, lrow, lj + lr)}};
+    // q from its lowest bit: the tile's r, jj, rows, then the rest of each
+    int q = 0, fn = 0, fp = 0;
+    auto nat = [&](int nbits, int to) { a.nat.f[fn++] = bit_field(q, nbits, to); };
+    // bits [lo, hi) of a quantity whose bits [from, to) sit at `at` + from ..
+    auto packed = [&](int lo, int hi, int from, int to, int at) {
+        const int l = lo > from ? lo : from, h = hi < to ? hi : to;
+        if (l < h) a.pk.f[fp++] = bit_field(q + l - lo, h - l, at + l - from);
+    };
+    auto put_r = [&](int lo, int hi) {  // gm B + j -> j VEC, member rank gm
+        nat(hi - lo, lo);
+        packed(lo, hi, 0, g.lb, g.lvec);
+        packed(lo, hi, g.lb, lm, slab);
+        q += hi - lo;
+    };
+    auto put_j = [&](int lo, int hi) {
+        nat(hi - lo, lm + lo);
+        packed(lo, hi, 0, g.lvec, 0);
+        q += hi - lo;
+    };
+    auto put_rows = [&](int lo, int hi) {  // (row in block, rank, block) of rows, then planes
+        nat(hi - lo, g.ln + lo);
+        for (int axis = 1; axis < d; axis++) {
+            const int at = (axis - 1) * g.ln, local = axis * g.ll;
+            packed(lo, hi, at, at + g.lb, local);
+            packed(lo, hi, at + g.lb, at + lm, slab + axis * g.lp);
+            packed(lo, hi, at + lm, at + g.ln, local + g.lb);
+        }
+        q += hi - lo;
+    };
+    put_r(0, lr), put_j(0, lj), put_rows(0, lrow);
+    put_r(lr, lm), put_j(lj, g.lvec), put_rows(lrow, nrow);
+    return a;
+}
 
 }  // namespace zm

@@ -29,15 +29,6 @@
 namespace zm {
 namespace lp {
 
-// v -> sum over fields of ((v >> from) & mask) << to
-template <int K>
-__device__ __forceinline__ int bits(const BitMap<K>& m, int v) {
-    int r = 0;
-#pragma unroll
-    for (int i = 0; i < K; i++) r += ((v >> m.f[i].from) & m.f[i].mask) << m.f[i].to;
-    return r;
-}
-
 // Ends of a pass.  PACKED goes through LDS (its runs in n are strided in
 // memory); ROW and TILE are loaded and stored straight from the registers of
 // the first and last radix pass, lanes along n (ROW) or along the lines (TILE).

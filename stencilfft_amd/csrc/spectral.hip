@@ -2,6 +2,7 @@
 // device forms of the index maps and the natural <-> packed converters.
 #include "common.hpp"
 #include "kernels.hpp"
+#include "line_maps.hpp"
 #include "maps.hpp"
 #include "spectral_math.hpp"
 
@@ -180,26 +181,91 @@ hipError_t launch_index_table(int64_t* out, const Geo& g, bool reciprocal, hipSt
     return hipGetLastError();
 }
 
-// natural (row-major N^d) <-> real-space packed layout, one thread per packed
-// element: the composition of the block-cyclic distribution and vector_pack
-// that init_host performs on the host (zmodel/utils.cu:9-36, utils.h:99-108).
-template <typename T>
-__global__ void __launch_bounds__(256) natural_packed_kernel(const Cx<T>* in, Cx<T>* out, Geo g, int to_packed) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= g.field) return;
-    const MapShape ms = make_map_shape(g.n, g.p, g.b);
-    const int64_t nat = real_linear(g, ms, i);
-    const int64_t f = (int64_t)blockIdx.y * g.field;
-    if (to_packed) out[f + i] = in[f + nat];
-    else out[f + nat] = in[f + i];
+// natural (row-major N^d) <-> real-space packed layout: the composition of the
+// block-cyclic distribution and vector_pack that init_host performs on the host
+// (zmodel/utils.cu:9-36, utils.h:99-108).
+//
+// Of a row, column jj M + r (r = gm B + j) goes to packed column j VEC + jj of
+// rank column gm: a VEC x M transpose.  A workgroup moves a tile of RC
+// consecutive r by JC consecutive jj of one row, or of several rows where a row
+// is smaller, through LDS, so that both sides move runs (of RC elements in
+// natural order, of JC elements or more in the packed rows); one thread per
+// element had read or written every VEC-th element per lane.  Both sides are
+// permutations of the bits of one element index q, whose low `ltile` bits are
+// the element of the tile: r, jj, rows.
+// Memory-bound: tiles of 1024 elements (four per thread, as fast as 2048 or
+// 4096 and faster on small fields), plain loads (non-temporal ones missed
+// fields that the last-level cache still held: 2048^2 FP32 11.3 against 14.5
+// us) and non-temporal stores (4096^2 FP64 78 against 102 us).  to / from
+// packed against one thread per element: 4096^2 FP64 127 / 145 -> 78 / 78 us,
+// 8192^2 FP32 387 / 579 -> 189 / 185 (5.7 TB/s), 512^3 FP32 594 / 575 -> 391 /
+// 368, 1024^2 FP32 7.0 -> 5.0.
+// FULL: the field holds at least one tile (no guards).
+template <typename T, int LE, bool FULL>
+__global__ void __launch_bounds__(256) convert_kernel(const Cx<T>* __restrict__ in, Cx<T>* __restrict__ out,
+                                                      ConvertArgs a, int to_packed) {
+    using C = Cx<T>;
+    constexpr int EPT = (1 << LE) / 256, NB = LE - 8;
+    __shared__ C tile[(1 << LE) + (1 << (LE - 4)) + (1 << (LE - 8)) + 1];
+    const int tid = threadIdx.x;
+    auto pad = [](int i) { return i + (i >> 4) + (i >> 8); };  // distinct banks at every power-of-two stride
+    const int64_t f = (int64_t)blockIdx.y << a.lfield;
+    const int base = (int)blockIdx.x << a.ltile;
+    // every address is a part of this tile, of this thread and of register k,
+    // the last the sum of its bits' offsets
+    const int slot = bits(a.order, tid);
+    const C* const nat_in = in + f + bits(a.nat, base) + bits(a.nat, tid);
+    C* const nat_out = out + f + bits(a.nat, base) + bits(a.nat, tid);
+    const C* const pk_in = in + f + bits(a.pk, base) + bits(a.pk, slot);
+    C* const pk_out = out + f + bits(a.pk, base) + bits(a.pk, slot);
+    int nat_bit[NB], pk_bit[NB], slot_bit[NB];
+#pragma unroll
+    for (int i = 0; i < NB; i++) {
+        nat_bit[i] = bits(a.nat, 256 << i);
+        slot_bit[i] = bits(a.order, 256 << i);
+        pk_bit[i] = bits(a.pk, slot_bit[i]);
+    }
+    auto sum = [&](const int* bit, int k) {
+        int o = 0;
+#pragma unroll
+        for (int i = 0; i < NB; i++) o += (k >> i) & 1 ? bit[i] : 0;
+        return o;
+    };
+    const int n = FULL ? EPT : tid >= (1 << a.ltile) ? 0 : a.ltile > 8 ? 1 << (a.ltile - 8) : 1;
+    C v[EPT];
+    if (to_packed) {
+#pragma unroll
+        for (int k = 0; k < EPT; k++) v[k] = k < n ? nat_in[sum(nat_bit, k)] : C{0, 0};
+#pragma unroll
+        for (int k = 0; k < EPT; k++)
+            if (k < n) tile[pad(tid + 256 * k)] = v[k];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < EPT; k++)
+            if (k < n) st_nt(pk_out + sum(pk_bit, k), tile[pad(sum(slot_bit, k) + slot)]);
+    } else {
+#pragma unroll
+        for (int k = 0; k < EPT; k++) v[k] = k < n ? pk_in[sum(pk_bit, k)] : C{0, 0};
+#pragma unroll
+        for (int k = 0; k < EPT; k++)
+            if (k < n) tile[pad(sum(slot_bit, k) + slot)] = v[k];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < EPT; k++)
+            if (k < n) st_nt(nat_out + sum(nat_bit, k), tile[pad(tid + 256 * k)]);
+    }
 }
 
 template <typename T>
 hipError_t launch_natural_packed(const Cx<T>* in, Cx<T>* out, const Geo& g, int batch, bool to_packed,
                                  hipStream_t stream) {
-    const unsigned threads = 256;
-    const dim3 grid((unsigned)((g.field + threads - 1) / threads), (unsigned)batch);
-    hipLaunchKernelGGL((natural_packed_kernel<T>), grid, dim3(threads), 0, stream, in, out, g, to_packed ? 1 : 0);
+    constexpr int LE = 10;
+    const ConvertArgs a = convert_args(g, LE);
+    const dim3 grid((unsigned)(g.field >> a.ltile), (unsigned)batch);
+    if (a.ltile == LE)
+        hipLaunchKernelGGL((convert_kernel<T, LE, true>), grid, dim3(256), 0, stream, in, out, a, to_packed ? 1 : 0);
+    else
+        hipLaunchKernelGGL((convert_kernel<T, LE, false>), grid, dim3(256), 0, stream, in, out, a, to_packed ? 1 : 0);
     return hipGetLastError();
 }
 

@@ -4,7 +4,8 @@
 // hold sample n of the line where the real-space maps put it, the row end holds
 // frequency k where the reciprocal maps do, the passes chain (what one writes as
 // rows the next reads as tiles), and a multiplier's maps give the lines'
-// frequencies.  Prints the number of shapes.
+// frequencies.  The converters' maps are checked the same way.  Prints the
+// number of shapes.
 #include <cstdio>
 #include <vector>
 
@@ -121,6 +122,26 @@ static bool check(int d, int n, int p, int b) {
                     }
                 }
             }
+    // converters: tiles of several sizes, larger than the field among them
+    for (int le : {8, 11, 12}) {
+        const ConvertArgs a = convert_args(g, le);
+        std::vector<char> seen(g.field);
+        for (int q = 0; q < g.field; q++) {
+            const int nat = at(a.nat, q), pk = at(a.pk, q);
+            if (nat < 0 || nat >= g.field || seen[nat]++) return fail("natural side", d, n, p, b, 0);
+            const int gc = nat % n, gr = nat / n % n, gd = nat / n / n;
+            Where w{};
+            global_col_to_local(ms, gc, &w.cid, &w.lc);
+            global_row_to_local(ms, gr, &w.rid, &w.lr);
+            if (d == 3) global_row_to_local(ms, gd, &w.did, &w.ld);
+            if (addr(g, w) != pk) return fail("packed side", d, n, p, b, 0);
+        }
+        std::vector<char> slot(1 << a.ltile);
+        for (int e = 0; e < 1 << a.ltile; e++) {
+            const int s = at(a.order, e);
+            if (s < 0 || s >= 1 << a.ltile || slot[s]++) return fail("tile order", d, n, p, b, 0);
+        }
+    }
     return true;
 }
 
