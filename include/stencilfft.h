@@ -193,6 +193,10 @@ typedef enum { ZM_COMPLEX = 0, ZM_REAL = 1 } zm_element;
  * (laplace3d.cu:90-361).  The Laplacian is self-adjoint. */
 zm_status zm_laplace(zm_plan* plan, const void* in, void* out, double scale, zm_element element, void* stream);
 
+/* inout += alpha * zm_laplace(in, scale) for complex fields, rounded like the
+ * separate calls: the explicit part of a time step (no reference counterpart). */
+zm_status zm_laplace_add(zm_plan* plan, const void* in, void* inout, double scale, double alpha, void* stream);
+
 /* Periodic 4th-order central differences [1, -8, 0, 8, -1] / (12 delta) along
  * x (packed columns) or y (block-cyclic rows); B >= 2.  Replaces dx / dy
  * with their halo packers (zmodel/stencils/dx.cu:10-161, dy.cu:10-185, which
@@ -245,11 +249,21 @@ zm_status zm_spectral_multiply_adjoint(zm_plan* plan, const void* in, void* out,
  * The last axis's two passes and the multiplier run as one kernel where the
  * plan has it (N <= 2048, 2D N = 4096, 2D FP32 N = 8192; FP64 and FP32 vector
  * ALU), else as the three calls; the values agree with them to rounding.
+ * `factor`, when not NULL, is a device address holding an FP64 value that
+ * multiplies the multiplier (a loss's incoming gradient, say).
  * ZM_PATH_TWO_STAGE plans get ZM_ERR_UNSUPPORTED.  Buffers as zm_forward. */
 zm_status zm_spectral_solve(zm_plan* plan, const void* in, void* out, zm_spectral kind, double p0, double p1,
-                            double length, double scale, void* scratch, void* stream);
+                            double length, double scale, const double* factor, void* scratch, void* stream);
 zm_status zm_spectral_solve_adjoint(zm_plan* plan, const void* in, void* out, zm_spectral kind, double p0, double p1,
-                                    double length, double scale, void* scratch, void* stream);
+                                    double length, double scale, const double* factor, void* scratch,
+                                    void* stream);
+
+/* inout -= g, and *norm2 (one value of the plan's real type) = sum |inout|^2
+ * after it, accumulated in FP64 in a fixed order: the residual and the loss of
+ * a misfit (no reference counterpart).  partials: ZM_NORM_PARTIALS doubles of
+ * device memory. */
+#define ZM_NORM_PARTIALS 2048
+zm_status zm_residual_norm(zm_plan* plan, void* inout, const void* g, double* partials, void* norm2, void* stream);
 
 /* ---------------------------------------------------------------------- */
 /* index maps (host, pure, thread-safe): zmodel/utils.h:99-320             */

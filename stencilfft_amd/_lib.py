@@ -15,6 +15,7 @@ ZM_OK = 0
 (ZM_ERR_INVALID_ARG, ZM_ERR_SHAPE, ZM_ERR_UNSUPPORTED, ZM_ERR_DEVICE, ZM_ERR_ALIAS, ZM_ERR_LAUNCH,
  ZM_ERR_NOMEM, ZM_ERR_IO, ZM_ERR_SCRATCH_LIMIT) = range(1, 10)
 ZM_NOALLOC_SCRATCH_BYTES = 64 << 20
+ZM_NORM_PARTIALS = 2048
 STATUS_NAMES = {
     0: "ZM_OK",
     1: "ZM_ERR_INVALID_ARG",
@@ -89,8 +90,10 @@ SIGNATURES = {
     "zm_dz4_adjoint": (_I, [_VP, _VP, _VP, _D, _I, _VP]),
     "zm_spectral_multiply": (_I, [_VP, _VP, _VP, _I, _D, _D, _D, _VP]),
     "zm_spectral_multiply_adjoint": (_I, [_VP, _VP, _VP, _I, _D, _D, _D, _VP]),
-    "zm_spectral_solve": (_I, [_VP, _VP, _VP, _I, _D, _D, _D, _D, _VP, _VP]),
-    "zm_spectral_solve_adjoint": (_I, [_VP, _VP, _VP, _I, _D, _D, _D, _D, _VP, _VP]),
+    "zm_spectral_solve": (_I, [_VP, _VP, _VP, _I, _D, _D, _D, _D, _VP, _VP, _VP]),
+    "zm_spectral_solve_adjoint": (_I, [_VP, _VP, _VP, _I, _D, _D, _D, _D, _VP, _VP, _VP]),
+    "zm_laplace_add": (_I, [_VP, _VP, _VP, _D, _D, _VP]),
+    "zm_residual_norm": (_I, [_VP, _VP, _VP, _VP, _VP, _VP]),
     "zm_packed_to_block_cyclic": (_I, [_SP, _I]),
     "zm_block_cyclic_to_packed": (_I, [_SP, _I]),
     "zm_real_to_global": (None, [_SP, _I, _I, _I, _I, _IP, _IP]),

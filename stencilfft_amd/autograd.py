@@ -11,8 +11,11 @@ adjoint, computed by the library's adjoint entry points:
                           the real kinds are self-adjoint)
   spectral solve       -> zm_spectral_solve_adjoint (the conjugate multiplier
                           between the same two transforms)
+  heat step            -> itself (real multiplier, symmetric Laplacian)
+  Poisson misfit       -> the adjoint solve of twice the saved residual; the only
+                          operator that saves a tensor for backward
 For complex tensors torch passes dL/d(conj y) and expects A^H of it back, which
-is exactly the adjoint.  No tensors are saved for backward.
+is exactly the adjoint.
 """
 from __future__ import annotations
 
@@ -109,6 +112,33 @@ class _SpectralSolve(torch.autograd.Function):
         return (ctx.plan.spectral_solve(g.contiguous(), *ctx.args, adjoint=True),) + (None,) * (1 + len(ctx.args))
 
 
+class _HeatStep(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, plan, *args):
+        ctx.plan, ctx.args = plan, args
+        return plan.heat_step(x.contiguous(), *args)
+
+    @staticmethod
+    def backward(ctx, g):
+        return (ctx.plan.heat_step(g.contiguous(), *ctx.args),) + (None,) * (1 + len(ctx.args))
+
+
+class _SolveMisfit(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, g, plan, *args):
+        ctx.plan, ctx.args = plan, args
+        r = plan.spectral_solve(x.contiguous(), *args)
+        loss = plan.residual_norm(r, g)
+        ctx.save_for_backward(r)
+        return loss
+
+    @staticmethod
+    def backward(ctx, gloss):
+        (r,) = ctx.saved_tensors
+        grad = ctx.plan.spectral_solve(r, *ctx.args, adjoint=True, factor=2.0 * gloss.to(torch.float64))
+        return (grad,) + (None,) * (2 + len(ctx.args))
+
+
 def fft(x, plan):
     """forward_fft: real-space packed layout -> reciprocal layout."""
     return _Forward.apply(x, plan)
@@ -146,3 +176,14 @@ def spectral_solve(x, plan, kind, p0=0.0, p1=0.0, length=1.0, scale=None):
     if scale is None:
         scale = 1.0 / float(plan.shape.n) ** plan.shape.dims
     return _SpectralSolve.apply(x, plan, kind, float(p0), float(p1), float(length), float(scale))
+
+
+def heat_step(x, plan, nu, dt, lap_scale=1.0, length=1.0):
+    """ifft(exp(-nu |k|^2 dt) fft(x)) + dt laplace(x, lap_scale) as one operator."""
+    return _HeatStep.apply(x, plan, float(nu), float(dt), float(lap_scale), float(length))
+
+
+def solve_misfit(x, g, plan, kind, p0=0.0, p1=0.0, length=1.0):
+    """||spectral_solve(x) - g||^2, differentiable in x; g is a constant."""
+    scale = 1.0 / float(plan.shape.n) ** plan.shape.dims
+    return _SolveMisfit.apply(x, g, plan, kind, float(p0), float(p1), float(length), scale)

@@ -107,6 +107,7 @@ struct SpectralArgs {
     double p0, p1, kscale;
     BitMap<3> f0, f1;
     const double* half_sin;  // sin(pi s / N), s the signed wavenumber of f < N
+    const double* factor;    // device value times the multiplier (null: 1)
 };
 
 // kinds of line pass: the two ends and the direction
@@ -144,16 +145,26 @@ template <typename T>
 hipError_t launch_stencil(const void* in, void* out, const Geo& g, int batch, StencilOp op, bool complex_elems,
                           double coef, bool negate, hipStream_t stream);
 
+// out += alpha * coef * Laplacian(in)
+template <typename T>
+hipError_t launch_laplace_add(const Cx<T>* in, Cx<T>* out, const Geo& g, int batch, double coef, double alpha,
+                              hipStream_t stream);
+
 // twiddle tables exp(-2 pi i t / n), t in [0, n), computed in FP64
 hipError_t launch_twiddles(double2* tw64, float2* tw32, int n, hipStream_t stream);
 
 // half_sin[f] = sin(pi s / n), s the signed wavenumber of f < n
 hipError_t launch_half_sin(double* half_sin, int n, hipStream_t stream);
 
+// r -= g over n elements; *norm2 = sum |r|^2 (FP64 partial sums in `partials`)
+constexpr int kNormBlocks = 2048;
+template <typename T>
+hipError_t launch_residual_norm(Cx<T>* r, const Cx<T>* g, int64_t n, double* partials, T* norm2, hipStream_t stream);
+
 // reciprocal-space multiplier
 template <typename T>
 hipError_t launch_spectral(const Cx<T>* in, Cx<T>* out, const Geo& g, int batch, int kind, double p0, double p1,
-                           double kscale, bool conj, hipStream_t stream);
+                           double kscale, bool conj, const double* factor, hipStream_t stream);
 
 // index tables and natural <-> packed conversion
 hipError_t launch_index_table(int64_t* out, const Geo& g, bool reciprocal, hipStream_t stream);

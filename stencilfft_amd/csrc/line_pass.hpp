@@ -311,6 +311,7 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
             constexpr int R = 1 << K::lr(NP - 1);
             const int lam0 = (g & ((1 << a.lgroups) - 1)) << LLP;
             K::template write<NP - 1, true, false>(lds, v, tid);
+            const double factor = sp.factor ? *sp.factor : 1.0;
             auto multiply = [&](auto fc) __attribute__((always_inline)) {
                 constexpr int FAMILY = decltype(fc)::value;
 #pragma unroll 1
@@ -327,6 +328,7 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
                         C* p = lds + l * K::LS + K::pad(f);
                         double mr, mi;
                         line_multiplier<FAMILY>(sp, ls, f, N, &mr, &mi);
+                        mr *= factor, mi *= factor;
                         const double vx = (double)p->x, vy = (double)p->y;
                         *p = C{(T)(vx * mr - vy * mi), (T)(vx * mi + vy * mr)};
                     }

@@ -184,6 +184,7 @@ int ipow(int a, int e) {
 constexpr int kLineTarget = 4096;
 constexpr int kStageTarget = 4096;
 constexpr size_t kMaxLds = 160 * 1024;
+static_assert(ZM_NORM_PARTIALS == zm::kNormBlocks, "partial sums of zm_residual_norm");
 
 // FP64 lines of 256 points run as 16 x 16 on at most two ranks per axis and as
 // 8 x 8 x 4 on more.  16 x 16 rounds once less: the FP64 rounding noise of a
@@ -698,7 +699,7 @@ struct Exec {
     zm_status multiply(const void* in, void* out, const zm::SpectralArgs& sp) const {
         return launch_status(timed_launch(p, ZM_STAGE_SPECTRAL, st, [&] {
             return zm::launch_spectral<T>((const zm::Cx<T>*)in, (zm::Cx<T>*)out, p->geo, p->batch, sp.kind, sp.p0,
-                                          sp.p1, sp.kscale, sp.conj != 0, st);
+                                          sp.p1, sp.kscale, sp.conj != 0, sp.factor, st);
         }, record));
     }
 
@@ -844,6 +845,28 @@ zm_status zm_laplace(zm_plan* p, const void* in, void* out, double scale, zm_ele
     return run_stencil(p, in, out, zm::OP_LAPLACE, scale, false, element, stream);
 }
 
+zm_status zm_laplace_add(zm_plan* p, const void* in, void* inout, double scale, double alpha, void* stream) {
+    ZM_TRY(check_io(p, in, inout));
+    const hipStream_t st = (hipStream_t)stream;
+    return launch_status(timed_launch(p, ZM_STAGE_LAPLACE, st, [&] {
+        if (p->precision == ZM_FP64)
+            return zm::launch_laplace_add<double>((const double2*)in, (double2*)inout, p->geo, p->batch, scale, alpha, st);
+        return zm::launch_laplace_add<float>((const float2*)in, (float2*)inout, p->geo, p->batch, scale, alpha, st);
+    }));
+}
+
+zm_status zm_residual_norm(zm_plan* p, void* inout, const void* g, double* partials, void* norm2, void* stream) {
+    ZM_TRY(check_io(p, g, inout));
+    if (!partials || !norm2) return ZM_ERR_INVALID_ARG;
+    const hipStream_t st = (hipStream_t)stream;
+    const int64_t n = (int64_t)p->batch * p->dims.field;
+    return launch_status(timed_launch(p, ZM_STAGE_SPECTRAL, st, [&] {
+        if (p->precision == ZM_FP64)
+            return zm::launch_residual_norm<double>((double2*)inout, (const double2*)g, n, partials, (double*)norm2, st);
+        return zm::launch_residual_norm<float>((float2*)inout, (const float2*)g, n, partials, (float*)norm2, st);
+    }));
+}
+
 static zm_status deriv(zm_plan* p, const void* in, void* out, double delta, zm_element element, void* stream,
                        zm::StencilOp op, bool negate) {
     if (!p) return ZM_ERR_INVALID_ARG;
@@ -881,7 +904,7 @@ static zm_status spectral_args(const zm_plan* p, zm_spectral kind, double p0, do
     // the dx4 symbol is defined on the 2D layout only, like zm_dx4
     if ((kind == ZM_SPECTRAL_STENCIL || kind == ZM_SPECTRAL_POISSON_STENCIL) && p1 != 0.0 && p->shape.dims != 2)
         return ZM_ERR_INVALID_ARG;
-    *sp = zm::SpectralArgs{(int)kind, conj ? 1 : 0, p->shape.dims, p0, p1, 2.0 * M_PI / length, {}, {}, nullptr};
+    *sp = zm::SpectralArgs{(int)kind, conj ? 1 : 0, p->shape.dims, p0, p1, 2.0 * M_PI / length, {}, {}, nullptr, nullptr};
     return ZM_OK;
 }
 
@@ -896,10 +919,12 @@ static zm_status spectral(zm_plan* p, const void* in, void* out, zm_spectral kin
 }
 
 static zm_status spectral_solve(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
-                                double length, double scale, void* scratch, void* stream, bool conj) {
+                                double length, double scale, const double* factor, void* scratch, void* stream,
+                                bool conj) {
     ZM_TRY(check_io(p, in, out));
     zm::SpectralArgs sp;
     ZM_TRY(spectral_args(p, kind, p0, p1, length, conj, &sp));
+    sp.factor = factor;
     void* s = nullptr;
     ZM_TRY(scratch_for(p, scratch, &s));
     if (s == in || s == out) return ZM_ERR_ALIAS;
@@ -919,13 +944,14 @@ zm_status zm_spectral_multiply_adjoint(zm_plan* p, const void* in, void* out, zm
 }
 
 zm_status zm_spectral_solve(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
-                            double length, double scale, void* scratch, void* stream) {
-    return spectral_solve(p, in, out, kind, p0, p1, length, scale, scratch, stream, false);
+                            double length, double scale, const double* factor, void* scratch, void* stream) {
+    return spectral_solve(p, in, out, kind, p0, p1, length, scale, factor, scratch, stream, false);
 }
 
 zm_status zm_spectral_solve_adjoint(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
-                                    double length, double scale, void* scratch, void* stream) {
-    return spectral_solve(p, in, out, kind, p0, p1, length, scale, scratch, stream, true);
+                                    double length, double scale, const double* factor, void* scratch,
+                                    void* stream) {
+    return spectral_solve(p, in, out, kind, p0, p1, length, scale, factor, scratch, stream, true);
 }
 
 zm_status zm_real_index_table(zm_plan* p, int64_t* out, void* stream) {

@@ -121,7 +121,7 @@ __device__ __forceinline__ void stencil_symbol(const Geo& g, int s0, int s1, int
 // adjoint); the multiplier is formed in FP64 for every storage precision.
 template <typename T>
 __global__ void __launch_bounds__(256) spectral_kernel(const Cx<T>* in, Cx<T>* out, Geo g, int kind, double p0,
-                                                       double p1, double kscale, int conj) {
+                                                       double p1, double kscale, int conj, const double* factor) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= g.field) return;
     const MapShape ms = make_map_shape(g.n, g.p, g.b);
@@ -141,6 +141,7 @@ __global__ void __launch_bounds__(256) spectral_kernel(const Cx<T>* in, Cx<T>* o
         }
     }
     if (conj) mi = -mi;
+    if (factor) mr *= *factor, mi *= *factor;
     const int64_t at = (int64_t)blockIdx.y * g.field + i;
     const Cx<T> v = in[at];
     const double vx = (double)v.x, vy = (double)v.y;
@@ -149,18 +150,79 @@ __global__ void __launch_bounds__(256) spectral_kernel(const Cx<T>* in, Cx<T>* o
 
 template <typename T>
 hipError_t launch_spectral(const Cx<T>* in, Cx<T>* out, const Geo& g, int batch, int kind, double p0, double p1,
-                           double kscale, bool conj, hipStream_t stream) {
+                           double kscale, bool conj, const double* factor, hipStream_t stream) {
     const unsigned threads = 256;
     const dim3 grid((unsigned)((g.field + threads - 1) / threads), (unsigned)batch);
     hipLaunchKernelGGL((spectral_kernel<T>), grid, dim3(threads), 0, stream, in, out, g, kind, p0, p1, kscale,
-                       conj ? 1 : 0);
+                       conj ? 1 : 0, factor);
     return hipGetLastError();
 }
 
 template hipError_t launch_spectral<float>(const float2*, float2*, const Geo&, int, int, double, double, double,
-                                           bool, hipStream_t);
+                                           bool, const double*, hipStream_t);
 template hipError_t launch_spectral<double>(const double2*, double2*, const Geo&, int, int, double, double, double,
-                                            bool, hipStream_t);
+                                            bool, const double*, hipStream_t);
+
+// r -= g and the FP64 partial sums of |r|^2, one per block in a fixed order
+// (the sum does not depend on scheduling); norm_kernel adds them.  Memory-bound:
+// two reads and a write of the field, where the difference, its square and the
+// sum as separate passes read four times and write twice (8 x 4096^2 FP32: 1.16
+// ms as three torch kernels).
+template <typename T>
+__global__ void __launch_bounds__(256) residual_kernel(Cx<T>* r, const Cx<T>* g, int64_t n, double* partials) {
+    __shared__ double sums[256];
+    const int64_t step = (int64_t)gridDim.x * 1024;
+    double acc = 0.0;
+    for (int64_t i0 = (int64_t)blockIdx.x * 1024 + threadIdx.x; i0 < n; i0 += step) {
+        Cx<T> a[4], b[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int64_t i = i0 + 256 * k < n ? i0 + 256 * k : i0;
+            a[k] = ld_nt(r + i);
+            b[k] = ld_nt(g + i);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (i0 + 256 * k >= n) break;
+            const Cx<T> d = csub(a[k], b[k]);
+            st_nt(r + i0 + 256 * k, d);
+            acc += (double)d.x * (double)d.x + (double)d.y * (double)d.y;
+        }
+    }
+    sums[threadIdx.x] = acc;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) sums[threadIdx.x] += sums[threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) partials[blockIdx.x] = sums[0];
+}
+
+template <typename T>
+__global__ void __launch_bounds__(256) norm_kernel(const double* partials, int n, T* norm2) {
+    __shared__ double sums[256];
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < n; i += 256) acc += partials[i];
+    sums[threadIdx.x] = acc;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) sums[threadIdx.x] += sums[threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *norm2 = (T)sums[0];
+}
+
+template <typename T>
+hipError_t launch_residual_norm(Cx<T>* r, const Cx<T>* g, int64_t n, double* partials, T* norm2, hipStream_t stream) {
+    const int64_t want = (n + 1023) / 1024;
+    const int blocks = (int)(want < kNormBlocks ? want : kNormBlocks);
+    hipLaunchKernelGGL((residual_kernel<T>), dim3(blocks), dim3(256), 0, stream, r, g, n, partials);
+    hipLaunchKernelGGL((norm_kernel<T>), dim3(1), dim3(256), 0, stream, partials, blocks, norm2);
+    return hipGetLastError();
+}
+
+template hipError_t launch_residual_norm<float>(float2*, const float2*, int64_t, double*, float*, hipStream_t);
+template hipError_t launch_residual_norm<double>(double2*, const double2*, int64_t, double*, double*, hipStream_t);
 
 __global__ void __launch_bounds__(256) index_table_kernel(int64_t* out, Geo g, int reciprocal) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;

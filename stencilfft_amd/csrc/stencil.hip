@@ -150,9 +150,11 @@ __device__ __forceinline__ E lap_combine(E a, E b, E l, E r, E f, E k, E c, bool
     return s;
 }
 
-template <typename E, typename S>
+// ADD (all three Laplacian kernels): out += alpha * (the scaled Laplacian),
+// rounded like the sum of separate calls.
+template <typename E, typename S, bool ADD>
 __global__ void __launch_bounds__(256) laplace_kernel(const E* __restrict__ in, E* __restrict__ out, Geo g, S scale,
-                                                      int apply_scale) {
+                                                      int apply_scale, S alpha) {
 #pragma clang fp contract(off)
     using O = EOps<E>;
     constexpr bool REF = sizeof(S) == 8;
@@ -183,7 +185,9 @@ __global__ void __launch_bounds__(256) laplace_kernel(const E* __restrict__ in, 
     }
     E s = lap_combine<REF, O, E, S>(a, b, l, r, f, k, c, g.dims == 3);
     if (apply_scale) s = O::mul(s, scale);
-    out[(int64_t)blockIdx.y * g.field + i] = s;
+    E* const o = out + (int64_t)blockIdx.y * g.field + i;
+    if constexpr (ADD) s = O::add(*o, O::mul(s, alpha));
+    *o = s;
 }
 
 // [1, -8, 0, 8, -1] / (12 delta) in the reference's order (dx.cu:29-79):
@@ -429,9 +433,9 @@ static hipError_t launch_deriv4(const E* in, E* out, const Geo& g, int batch, in
 // lds[pos + 2 VEC].  3D: the rows of planes gd - 1 and gd + 1 are loaded
 // directly; the strips of those planes are grid.x * grid.y (a multiple of 8)
 // blocks away, so they run on the same XCD and the loads hit its L2.
-template <typename E, typename S, int K, bool D3, int HK>
+template <typename E, typename S, int K, bool D3, int HK, bool ADD>
 __global__ void __launch_bounds__(256) laplace_strip_kernel(const E* __restrict__ in, E* __restrict__ out, Geo g,
-                                                            int rows_per_strip, S scale, int apply_scale) {
+                                                            int rows_per_strip, S scale, int apply_scale, S alpha) {
 #pragma clang fp contract(off)
     using O = EOps<E>;
     extern __shared__ unsigned char smem_raw[];
@@ -510,6 +514,12 @@ __global__ void __launch_bounds__(256) laplace_strip_kernel(const E* __restrict_
         constexpr int U = decltype(uc)::value, C0 = (U + 1) & 3, D = (U + 2) & 3, X = (U + 3) & 3;
         constexpr int H = decltype(hc)::value, HN = H ^ 1;
         const int gr = g0 + t;
+        const int64_t oc = row_off(gd, gr, cid);
+        E old[ADD ? K : 1];
+        if constexpr (ADD) {
+#pragma unroll
+            for (int k = 0; k < K; k++) old[k] = ld(dst + oc + tid + 256 * k);
+        }
         if (t + 1 < rows_per_strip) {
             load_row(gd, gr + 2, rr[X]);
             if constexpr (D3) {
@@ -530,7 +540,6 @@ __global__ void __launch_bounds__(256) laplace_strip_kernel(const E* __restrict_
             }
         }
         __syncthreads();
-        const int64_t oc = row_off(gd, gr, cid);
 #pragma unroll
         for (int k = 0; k < K; k++) {
             const int pos = tid + 256 * k;
@@ -543,6 +552,7 @@ __global__ void __launch_bounds__(256) laplace_strip_kernel(const E* __restrict_
                 acc = lap_combine<sizeof(S) == 8, O, E, S>(rr[U][k], rr[D][k], row[pos], row[pos + 2 * VEC], c, c, c,
                                                            false);
             if (apply_scale) acc = O::mul(acc, scale);
+            if constexpr (ADD) acc = O::add(old[k], O::mul(acc, alpha));
             if constexpr (D3) dst[oc + pos] = acc;
             else st_nt(dst + oc + pos, acc);
         }
@@ -578,9 +588,9 @@ __global__ void __launch_bounds__(256) laplace_strip_kernel(const E* __restrict_
 // the FP64 one from 0.93 to 0.79 ms (1024^3 at L = 512: 8.05 to 6.75 ms).
 // NTH threads per workgroup; KE = R L / NTH tile elements per thread; KY, HX:
 // y-halo and x-halo elements per thread (guarded).
-template <typename E, typename S, int R, int KE, int KY, int HX, int NTH = 256>
+template <typename E, typename S, int R, int KE, int KY, int HX, int NTH, bool ADD>
 __global__ void __launch_bounds__(NTH) laplace_zmarch_kernel(const E* __restrict__ in, E* __restrict__ out, Geo g, int tz,
-                                                   int ltiles, S scale, int apply_scale) {
+                                                   int ltiles, S scale, int apply_scale, S alpha) {
 #pragma clang fp contract(off)
     using O = EOps<E>;
     extern __shared__ unsigned char smem_raw[];
@@ -660,6 +670,14 @@ __global__ void __launch_bounds__(NTH) laplace_zmarch_kernel(const E* __restrict
         constexpr int U = decltype(uc)::value, C0 = (U + 1) & 3, D = (U + 2) & 3, X = (U + 3) & 3;
         constexpr int H = decltype(hc)::value, HN = H ^ 1;
         const int gd = z0 + t;
+        E old[ADD ? KE : 1];
+        if constexpr (ADD) {
+#pragma unroll
+            for (int k = 0; k < KE; k++) {
+                const int e = tid + NTH * k;
+                old[k] = ld_nt(dst + row_off(gd, r0 + (e >> g.ll), cid) + (e & (L - 1)));
+            }
+        }
         if (t + 1 < tz) {
             load_plane(gd + 2, pl[X]);
             load_halo(gd + 1, yh[HN], xh[HN]);
@@ -691,6 +709,7 @@ __global__ void __launch_bounds__(NTH) laplace_zmarch_kernel(const E* __restrict
             const E a = tile[pos - W], b = tile[pos + W], l = tile[pos - VEC], rr = tile[pos + VEC];
             E acc = lap_combine<sizeof(S) == 8, O, E, S>(a, b, l, rr, pl[U][k], pl[D][k], pl[C0][k], true);
             if (apply_scale) acc = O::mul(acc, scale);
+            if constexpr (ADD) acc = O::add(old[k], O::mul(acc, alpha));
             dst[row_off(gd, r0 + r - 1, cid) + c] = acc;
         }
         __syncthreads();
@@ -716,8 +735,9 @@ static int strip_rows(const Geo& g, int batch) {
     return rows;
 }
 
-template <typename E, typename S>
-static hipError_t laplace_strip(const E* in, E* out, const Geo& g, int batch, double coef, hipStream_t stream) {
+template <typename E, typename S, bool ADD>
+static hipError_t laplace_strip(const E* in, E* out, const Geo& g, int batch, double coef, double alpha,
+                                hipStream_t stream) {
     const bool d3 = g.dims == 3;
     const int rows = strip_rows(g, batch);
     const dim3 grid((unsigned)(g.n / rows), (unsigned)g.p, (unsigned)(d3 ? batch * g.n : batch));
@@ -728,11 +748,11 @@ static hipError_t laplace_strip(const E* in, E* out, const Geo& g, int batch, do
     const bool one_halo = g.vec <= 256;
 #define ZM_STRIP2(KK, HH)                                                                                        \
     if (d3)                                                                                                     \
-        hipLaunchKernelGGL((laplace_strip_kernel<E, S, KK, true, HH>), grid, dim3(256), lds, stream, in, out, g,  \
-                           rows, sc, apply);                                                                    \
+        hipLaunchKernelGGL((laplace_strip_kernel<E, S, KK, true, HH, ADD>), grid, dim3(256), lds, stream, in, out, g,  \
+                           rows, sc, apply, (S)alpha);                                                                    \
     else                                                                                                        \
-        hipLaunchKernelGGL((laplace_strip_kernel<E, S, KK, false, HH>), grid, dim3(256), lds, stream, in, out, g, \
-                           rows, sc, apply);
+        hipLaunchKernelGGL((laplace_strip_kernel<E, S, KK, false, HH, ADD>), grid, dim3(256), lds, stream, in, out, g, \
+                           rows, sc, apply, (S)alpha);
 #define ZM_STRIP(KK)                \
     if (one_halo) {                 \
         ZM_STRIP2(KK, 1)            \
@@ -774,8 +794,9 @@ static bool zmarch_ok(const Geo& g, size_t es) {
     return R * g.vec <= 256 && g.n % R == 0 && (size_t)(R + 2) * (size_t)(g.l + 2 * g.vec) * es <= 65536;
 }
 
-template <typename E, typename S, int R, int KE, int KY, int NTH = 256>
-static hipError_t laplace_zmarch_inst(const E* in, E* out, const Geo& g, int batch, double coef, hipStream_t stream) {
+template <typename E, typename S, bool ADD, int R, int KE, int KY, int NTH = 256>
+static hipError_t laplace_zmarch_inst(const E* in, E* out, const Geo& g, int batch, double coef, double alpha,
+                                      hipStream_t stream) {
     if (KE * NTH != R * g.l || KY * NTH < 2 * g.l || 2 * R * g.vec > 2 * NTH) return hipErrorInvalidValue;
     const int ntiles = g.n / R;
     int ltiles = 0;
@@ -791,48 +812,50 @@ static hipError_t laplace_zmarch_inst(const E* in, E* out, const Geo& g, int bat
     const size_t lds = sizeof(E) * (size_t)(R + 2) * (size_t)(g.l + 2 * g.vec);
     const bool two = 2 * R * g.vec > NTH;
     if (two)
-        hipLaunchKernelGGL((laplace_zmarch_kernel<E, S, R, KE, KY, 2, NTH>), dim3(blocks, (unsigned)batch), dim3(NTH),
-                           lds, stream, in, out, g, tz, ltiles, (S)coef, coef != 1.0 ? 1 : 0);
+        hipLaunchKernelGGL((laplace_zmarch_kernel<E, S, R, KE, KY, 2, NTH, ADD>), dim3(blocks, (unsigned)batch), dim3(NTH),
+                           lds, stream, in, out, g, tz, ltiles, (S)coef, coef != 1.0 ? 1 : 0, (S)alpha);
     else
-        hipLaunchKernelGGL((laplace_zmarch_kernel<E, S, R, KE, KY, 1, NTH>), dim3(blocks, (unsigned)batch), dim3(NTH),
-                           lds, stream, in, out, g, tz, ltiles, (S)coef, coef != 1.0 ? 1 : 0);
+        hipLaunchKernelGGL((laplace_zmarch_kernel<E, S, R, KE, KY, 1, NTH, ADD>), dim3(blocks, (unsigned)batch), dim3(NTH),
+                           lds, stream, in, out, g, tz, ltiles, (S)coef, coef != 1.0 ? 1 : 0, (S)alpha);
     return hipGetLastError();
 }
 
-template <typename E, typename S>
-static hipError_t laplace_zmarch(const E* in, E* out, const Geo& g, int batch, double coef, hipStream_t stream) {
+template <typename E, typename S, bool ADD>
+static hipError_t laplace_zmarch(const E* in, E* out, const Geo& g, int batch, double coef, double alpha,
+                                 hipStream_t stream) {
     switch (g.l) {
-        case 32: return laplace_zmarch_inst<E, S, 8, 1, 1>(in, out, g, batch, coef, stream);
-        case 64: return laplace_zmarch_inst<E, S, 8, 2, 1>(in, out, g, batch, coef, stream);
-        case 128: return laplace_zmarch_inst<E, S, 8, 4, 1>(in, out, g, batch, coef, stream);
+        case 32: return laplace_zmarch_inst<E, S, ADD, 8, 1, 1>(in, out, g, batch, coef, alpha, stream);
+        case 64: return laplace_zmarch_inst<E, S, ADD, 8, 2, 1>(in, out, g, batch, coef, alpha, stream);
+        case 128: return laplace_zmarch_inst<E, S, ADD, 8, 4, 1>(in, out, g, batch, coef, alpha, stream);
         // 512 threads: 0.405 -> 0.399 ms (FP32) at 512^3
-        case 256: return laplace_zmarch_inst<E, S, 8, 4, 1, 512>(in, out, g, batch, coef, stream);
-        case 512: return laplace_zmarch_inst<E, S, 4, 8, 4>(in, out, g, batch, coef, stream);
-        case 1024: return laplace_zmarch_inst<E, S, 2, 8, 8>(in, out, g, batch, coef, stream);
+        case 256: return laplace_zmarch_inst<E, S, ADD, 8, 4, 1, 512>(in, out, g, batch, coef, alpha, stream);
+        case 512: return laplace_zmarch_inst<E, S, ADD, 4, 8, 4>(in, out, g, batch, coef, alpha, stream);
+        case 1024: return laplace_zmarch_inst<E, S, ADD, 2, 8, 8>(in, out, g, batch, coef, alpha, stream);
         default: return hipErrorInvalidValue;
     }
+}
+
+// 3D: the depth march where its tile fits, else the strip kernel
+template <typename E, typename S, bool ADD>
+static hipError_t laplace_dispatch(const E* in, E* out, const Geo& g, int batch, double coef, double alpha,
+                                   hipStream_t stream) {
+    if (zmarch_ok(g, sizeof(E))) return laplace_zmarch<E, S, ADD>(in, out, g, batch, coef, alpha, stream);
+    if (strip_ok(g, batch)) return laplace_strip<E, S, ADD>(in, out, g, batch, coef, alpha, stream);
+    const unsigned threads = 256;
+    const dim3 grid((unsigned)((g.field + threads - 1) / threads), (unsigned)batch);
+    hipLaunchKernelGGL((laplace_kernel<E, S, ADD>), grid, dim3(threads), 0, stream, in, out, g, (S)coef,
+                       coef != 1.0 ? 1 : 0, (S)alpha);
+    return hipGetLastError();
 }
 
 template <typename E, typename S>
 static hipError_t stencil_dispatch(const void* in, void* out, const Geo& g, int batch, StencilOp op, double coef,
                                    bool negate, hipStream_t stream) {
-    const unsigned threads = 256;
-    const dim3 grid((unsigned)((g.field + threads - 1) / threads), (unsigned)batch);
     const E* src = static_cast<const E*>(in);
     E* dst = static_cast<E*>(out);
-    // 3D: the depth march where its tile fits, else the strip kernel
-    if (op == OP_LAPLACE && zmarch_ok(g, sizeof(E))) {
-        return laplace_zmarch<E, S>(src, dst, g, batch, coef, stream);
-    } else if (op == OP_LAPLACE && strip_ok(g, batch)) {
-        return laplace_strip<E, S>(src, dst, g, batch, coef, stream);
-    } else if (op == OP_LAPLACE) {
-        hipLaunchKernelGGL((laplace_kernel<E, S>), grid, dim3(threads), 0, stream, src, dst, g, (S)coef,
-                           coef != 1.0 ? 1 : 0);
-    } else {
-        const int axis = op == OP_DX4 ? 0 : op == OP_DY4 ? 1 : 2;
-        return launch_deriv4<E, S>(src, dst, g, batch, axis, (S)coef, negate, stream);
-    }
-    return hipGetLastError();
+    if (op == OP_LAPLACE) return laplace_dispatch<E, S, false>(src, dst, g, batch, coef, 1.0, stream);
+    const int axis = op == OP_DX4 ? 0 : op == OP_DY4 ? 1 : 2;
+    return launch_deriv4<E, S>(src, dst, g, batch, axis, (S)coef, negate, stream);
 }
 
 template <typename T>
@@ -842,6 +865,14 @@ hipError_t launch_stencil(const void* in, void* out, const Geo& g, int batch, St
     return stencil_dispatch<T, T>(in, out, g, batch, op, coef, negate, stream);
 }
 
+template <typename T>
+hipError_t launch_laplace_add(const Cx<T>* in, Cx<T>* out, const Geo& g, int batch, double coef, double alpha,
+                              hipStream_t stream) {
+    return laplace_dispatch<Cx<T>, T, true>(in, out, g, batch, coef, alpha, stream);
+}
+
+template hipError_t launch_laplace_add<float>(const float2*, float2*, const Geo&, int, double, double, hipStream_t);
+template hipError_t launch_laplace_add<double>(const double2*, double2*, const Geo&, int, double, double, hipStream_t);
 template hipError_t launch_stencil<float>(const void*, void*, const Geo&, int, StencilOp, bool, double, bool,
                                           hipStream_t);
 template hipError_t launch_stencil<double>(const void*, void*, const Geo&, int, StencilOp, bool, double, bool,

@@ -320,20 +320,59 @@ class Plan:
         return out
 
     def spectral_solve(self, x, kind: str, p0: float = 0.0, p1: float = 0.0, length: float = 1.0, scale: float = 1.0,
-                       out=None, scratch=None, stream=None, adjoint: bool = False):
+                       out=None, scratch=None, stream=None, adjoint: bool = False, factor=None):
         """inverse(m(k) forward(x), scale): the two transforms of the last axis and
         the multiplier in one kernel where the plan has it (the three calls on
-        two-stage plans)."""
+        two-stage plans).  `factor`: a CUDA tensor of one float64 that
+        multiplies the multiplier."""
         out = self._out(x, out)
+        if factor is not None:
+            import torch
+            if factor.dtype != torch.float64 or factor.numel() != 1 or factor.device != x.device:
+                raise ValueError(f"factor must be one float64 on {x.device}, got {tuple(factor.shape)} {factor.dtype} "
+                                 f"on {factor.device}")
         if self.two_stage:
-            y = self.forward(x, scratch=scratch, stream=stream)
-            self.spectral_multiply(y, kind, p0, p1, length, out=y, stream=stream, adjoint=adjoint)
-            return self.inverse(y, scale, out=out, scratch=scratch, stream=stream)
+            import torch
+            ts = torch.cuda.ExternalStream(stream) if isinstance(stream, int) else stream
+            with torch.cuda.stream(ts):  # the spectrum belongs to the stream that uses it (None: the current one)
+                y = self.forward(x, scratch=scratch)
+                self.spectral_multiply(y, kind, p0, p1, length, out=y, adjoint=adjoint)
+                if factor is not None:
+                    y.mul_(factor.reshape(()).to(self.real_dtype))
+                return self.inverse(y, scale, out=out, scratch=scratch)
         sp = self._scratch(scratch, x, out)
         fn = L._lib().zm_spectral_solve_adjoint if adjoint else L._lib().zm_spectral_solve
         L.check(fn(self._h, _ptr(x), _ptr(out), self.SPECTRAL_KINDS[kind], float(p0), float(p1), float(length),
-                   float(scale), sp, _stream(stream)), "zm_spectral_solve")
+                   float(scale), _ptr(factor), sp, _stream(stream)), "zm_spectral_solve")
         return out
+
+    def laplace_add(self, x, acc, scale: float = 1.0, alpha: float = 1.0, stream=None):
+        """acc += alpha * laplace(x, scale) for complex fields; returns acc."""
+        self._check_tensor(x)
+        self._check_tensor(acc)
+        L.check(L._lib().zm_laplace_add(self._h, _ptr(x), _ptr(acc), float(scale), float(alpha), _stream(stream)),
+                "zm_laplace_add")
+        return acc
+
+    def heat_step(self, x, nu: float, dt: float, lap_scale: float = 1.0, length: float = 1.0, out=None, scratch=None,
+                  stream=None):
+        """inverse(exp(-nu |k|^2 dt) forward(x)) / N^d + dt * laplace(x, lap_scale)
+        (self-adjoint)."""
+        norm = 1.0 / float(self.shape.n) ** self.shape.dims
+        out = self.spectral_solve(x, "heat", nu, dt, length, norm, out=out, scratch=scratch, stream=stream)
+        return self.laplace_add(x, out, lap_scale, dt, stream=stream)
+
+    def residual_norm(self, acc, g):
+        """acc -= g on the current stream; returns sum |acc|^2, a 0-dim tensor of
+        the plan's real dtype."""
+        import torch
+        self._check_tensor(acc)
+        self._check_tensor(g)
+        partials = torch.empty(L.ZM_NORM_PARTIALS, dtype=torch.float64, device=acc.device)
+        norm2 = torch.empty((), dtype=self.real_dtype, device=acc.device)
+        L.check(L._lib().zm_residual_norm(self._h, _ptr(acc), _ptr(g), _ptr(partials), _ptr(norm2), _stream(None)),
+                "zm_residual_norm")
+        return norm2
 
     # ---- per-stage timing (zm_timing_*) ----
     def timing(self, enable: bool = True):

@@ -46,10 +46,17 @@ def sq_norm(r):
 
 
 def poisson_loss(f, g, plan, length=1.0, form="spatial"):
+    # a target that is a plain constant field: residual and norm in one pass
+    if (form == "spectral" and torch.is_tensor(f) and torch.is_tensor(g) and not g.requires_grad and g.is_contiguous()
+            and g.shape == f.shape and g.dtype == f.dtype == plan.complex_dtype and g.device == f.device):
+        n = plan.shape.n
+        return ag.solve_misfit(f, g, plan, "poisson_stencil", float(n * n), 1.0 / n, length)
     return sq_norm(poisson_residual(f, g, plan, length, form))
 
 
 def heat_step(u, plan, nu, dt, lap_scale=1.0, length=1.0):
+    if isinstance(dt, (int, float)):
+        return ag.heat_step(u, plan, nu, dt, lap_scale, length)
     return ag.spectral_solve(u, plan, "heat", nu, dt, length) + dt * ag.laplace(u, plan, scale=lap_scale)
 
 
@@ -91,8 +98,6 @@ def rollout(u0, step, nsteps, every=8):
 def adjoint_heat(g, plan, nsteps, nu, dt, lap_scale=1.0, length=1.0):
     """Pull a final-state gradient back through nsteps heat steps with the
     adjoint kernels directly: step^H = F^H M IFFT^H + dt Lap (M real, Lap symmetric)."""
-    n_d = float(plan.shape.n) ** plan.shape.dims
     for _ in range(nsteps):
-        a = plan.spectral_solve(g.contiguous(), "heat", nu, dt, length, 1.0 / n_d, adjoint=True)
-        g = a + dt * plan.laplace(g.contiguous(), lap_scale)
+        g = plan.heat_step(g.contiguous(), nu, dt, lap_scale, length)  # self-adjoint
     return g
