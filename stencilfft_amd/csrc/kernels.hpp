@@ -94,6 +94,7 @@ __device__ __forceinline__ int bits(const BitMap<K>& m, int v) {
 struct LinePassArgs {
     BitMap<4> in_l, out_l;
     BitMap<3> in_n, out_n, pk;
+    BitMap<6> rows;  // Laplacian passes: global row (plane N + row) -> row base, for both ends
     int lgroups;    // log2 of the line groups per field
     int groups;     // line groups of the whole batch
     int xcd;        // consecutive groups on one XCD
@@ -117,7 +118,9 @@ enum LinePass {
     LP_TILE_FWD = 2,   // tile -> row
     LP_TILE_INV = 3,   // row -> tile
     LP_TILE_SPEC = 4,  // tile -> multiplier -> tile
-    LP_ROW_SPEC = 5    // packed -> multiplier -> packed
+    LP_ROW_SPEC = 5,   // packed -> multiplier -> packed
+    LP_ROW_LAP2 = 6,   // 5-point Laplacian of packed -> row
+    LP_ROW_LAP3 = 7    // 7-point Laplacian of packed -> row
 };
 struct LinePassInfo {
     int lines_log2;  // log2 of the lines per workgroup; -1: not built

@@ -61,17 +61,30 @@ struct NatMaps {
     // of the y pass are kx; the rows of the z pass are kc (e) and kr (y)
     BitMap<3> frequency0() const { return d == 2 ? frequency(0, g.ll) : frequency(g.ll, 2 * g.ll); }
     BitMap<3> frequency1() const { return d == 2 ? BitMap<3>{} : frequency(0, 2 * g.ll + g.lp); }
+    // global row plane N + row of an x pass -> row base
+    BitMap<6> global_rows() const {
+        BitMap<6> m{};
+        for (int axis = 1; axis < d; axis++) {
+            const int at = (axis - 1) * g.ln, local = axis * g.ll;
+            m.f[3 * axis - 3] = bit_field(at, g.lb, local);
+            m.f[3 * axis - 2] = bit_field(at + g.lb, g.lp, member(axis));
+            m.f[3 * axis - 1] = bit_field(at + lm, g.lvec, local + g.lb);
+        }
+        return m;
+    }
     // both ends of pass `kind` along `axis`
     void ends(LinePass kind, int axis, bool tiled, LinePassArgs* a) const {
         const BitMap<4> rl = row_lines(axis, tiled), tl = tile_lines(axis);
         const BitMap<3> rn = row(axis), tn = tile(axis), pn = packed(axis);
         const bool tin = kind == LP_TILE_FWD || kind == LP_TILE_SPEC, tout = kind == LP_TILE_INV || kind == LP_TILE_SPEC;
-        const bool pin = kind == LP_ROW_FWD || kind == LP_ROW_SPEC, pout = kind == LP_ROW_INV || kind == LP_ROW_SPEC;
+        const bool lap = kind == LP_ROW_LAP2 || kind == LP_ROW_LAP3;
+        const bool pin = kind == LP_ROW_FWD || kind == LP_ROW_SPEC || lap, pout = kind == LP_ROW_INV || kind == LP_ROW_SPEC;
         a->in_l = tin ? tl : rl;
         a->in_n = tin ? tn : pin ? pn : rn;
         a->out_l = tout ? tl : rl;
         a->out_n = tout ? tn : pout ? pn : rn;
         a->pk = packed_to_n();
+        if (lap) a->rows = global_rows();
     }
 };
 

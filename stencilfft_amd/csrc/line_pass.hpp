@@ -32,7 +32,8 @@ namespace lp {
 // Ends of a pass.  PACKED goes through LDS (its runs in n are strided in
 // memory); ROW and TILE are loaded and stored straight from the registers of
 // the first and last radix pass, lanes along n (ROW) or along the lines (TILE).
-enum End { PACKED = 0, ROW = 1, TILE = 2 };
+// LAP2 / LAP3 (input): the 5- / 7-point Laplacian of a packed end.
+enum End { PACKED = 0, ROW = 1, TILE = 2, LAP2 = 3, LAP3 = 4 };
 enum Dir { FWD = 0, INV = 1, SPEC = 2 };
 // How a workgroup runs over line groups: one group each, twiddles from the
 // caches (ONCE); a loop with the next group's loads in flight, for tiles that
@@ -165,38 +166,49 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
     // the pass whose registers the input arrives in, and the one that stores
     constexpr int PIN = F ? 0 : NP - 1, POUT = DIR == FWD ? NP - 1 : 0;
     constexpr int RIN = 1 << K::lr(PIN), ROUT = 1 << K::lr(POUT);
-    constexpr bool TIN = IN == TILE, TOUT = OUT == TILE;
+    constexpr bool TIN = IN == TILE, TOUT = OUT == TILE, LAP = IN == LAP2 || IN == LAP3;
+    constexpr bool PIN_LDS = IN == PACKED || LAP;  // the input is staged through LDS
+    static_assert(!LAP || (DIR == FWD && MODE == ONCE), "the Laplacian runs ahead of forward passes");
     extern __shared__ unsigned char smem_raw[];
     C* const lds = reinterpret_cast<C*>(smem_raw);
     int tid = threadIdx.x;
     const C* const tw = MODE == LOOP_LDS ? lds + K::LP * K::LS : tables;
 
-    auto group_base = [&](const BitMap<4>& m, int g) -> int64_t {
+    auto group_base = [&](const auto& m, int g) -> int64_t {
         const int f = g >> a.lgroups;
         return (int64_t)f * a.field + bits(m, (g & ((1 << a.lgroups) - 1)) << LLP);
     };
     // offset of memory-order element e of the group (PACKED ends): line e / N,
     // element e % N of its P rank rows
-    auto packed_off = [&](const BitMap<4>& ml, const BitMap<3>& mn, int e) -> int {
+    auto packed_off = [&](const auto& ml, const BitMap<3>& mn, int e) -> int {
         return bits(ml, e >> LN) + bits(mn, e & (N - 1));
     };
     auto packed_lds = [&](int e) -> int { return (e >> LN) * K::LS + K::pad(bits(a.pk, e & (N - 1))); };
 
-    // a multiplier pass writes where it reads
-    const BitMap<4>& out_l = DIR == SPEC ? a.in_l : a.out_l;
+    // a multiplier pass writes where it reads; a Laplacian's lines are global
+    // rows, in their order
+    const auto& in_l = [&]() -> const auto& {
+        if constexpr (LAP) return a.rows;
+        else return a.in_l;
+    }();
+    const auto& out_l = [&]() -> const auto& {
+        if constexpr (LAP) return a.rows;
+        else if constexpr (DIR == SPEC) return a.in_l;
+        else return a.out_l;
+    }();
     const BitMap<3>& out_n = DIR == SPEC ? a.in_n : a.out_n;
     // An address is a per-thread part plus a uniform one per register, the sum
     // of the offsets of the register number's bits: radix index r (ROW, TILE)
     // or memory-order sweep k (PACKED).
-    constexpr int NB = IN == PACKED || OUT == PACKED ? LEPT : K::LR;
+    constexpr int NB = PIN_LDS || OUT == PACKED ? LEPT : K::LR;
     int in_bit[NB], out_bit[NB], lds_bit[NB];
 #pragma unroll
     for (int i = 0; i < NB; i++) {
-        in_bit[i] = IN == PACKED ? packed_off(a.in_l, a.in_n, NT << i) : bits(a.in_n, (N / RIN) << i);
+        in_bit[i] = PIN_LDS ? packed_off(in_l, a.in_n, NT << i) : bits(a.in_n, (N / RIN) << i);
         out_bit[i] = OUT == PACKED ? packed_off(out_l, out_n, NT << i) : bits(out_n, (N / ROUT) << i);
         lds_bit[i] = packed_lds(NT << i);
     }
-    const int in_thread = packed_off(a.in_l, a.in_n, tid), out_thread = packed_off(out_l, out_n, tid),
+    const int in_thread = packed_off(in_l, a.in_n, tid), out_thread = packed_off(out_l, out_n, tid),
               lds_thread = packed_lds(tid);  // PACKED
     auto uniform_off = [&](const int* bit, int r) -> int {
         int o = 0;
@@ -210,8 +222,12 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
     C pre[EPT];
     auto fetch = [&](int g, auto k0c, auto k1c) __attribute__((always_inline)) {
         constexpr int K0 = decltype(k0c)::value, K1 = decltype(k1c)::value;
-        const C* gb = in + group_base(a.in_l, g);
-        if constexpr (IN == PACKED) {
+        const C* gb = in + group_base(in_l, g);
+        if constexpr (LAP) {
+            // rows and planes that other groups read too: plain loads
+#pragma unroll
+            for (int k = K0; k < K1; k++) pre[k] = gb[uniform_off(in_bit, k) + in_thread];
+        } else if constexpr (IN == PACKED) {
 #pragma unroll
             for (int k = K0; k < K1; k++)
                 pre[k] = ld_nt(gb + uniform_off(in_bit, k) + in_thread);
@@ -221,7 +237,7 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
                 int l, j;
                 K::template item<PIN, TIN>(tid, k / RIN, l, j);
                 const C* p = gb + uniform_off(in_bit, k % RIN);
-                pre[k] = ld_nt(p + (bits(a.in_l, l) + bits(a.in_n, j)));
+                pre[k] = ld_nt(p + (bits(in_l, l) + bits(a.in_n, j)));
             }
         }
     };
@@ -242,6 +258,64 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
         }
     };
 
+    // LAP: pre[] becomes `scale` times its Laplacian.  The rows above and below
+    // (and the planes before and after) are loaded beside it, mostly from the
+    // caches: the groups run in global row order.  The x neighbours come from
+    // the raw rows in LDS, where they are samples n -+ 1.  Operations and their
+    // order are the stencil kernels' (stencil.hip, lap_combine): bit for bit
+    // zm_laplace.  The field is read and written once instead of twice: forward
+    // chain of three 2048^2 FP64 fields, P = 8, 255 -> 183 us, 256^3 FP64 P = 4
+    // 400 -> 318, 1024^2 FP64 25 -> 22, 64^2 8.6 -> 7.6.
+    auto laplacian = [&](int g) __attribute__((always_inline)) {
+#pragma clang fp contract(off)
+        const int lam0 = (g & ((1 << a.lgroups) - 1)) << LLP;
+        const C* const fb = in + (int64_t)(g >> a.lgroups) * a.field;
+        const int in_row = bits(a.in_n, tid & (N - 1));
+        // memory-order element k of the line `rows` down and `planes` on
+        auto neighbour = [&](int k, int rows, int planes) -> C {
+            const int gl = lam0 + (tid >> LN) + ((k * NT) >> LN);  // uniform where NT <= N
+            int to = (gl & ~(N - 1)) | ((gl + rows) & (N - 1));
+            if constexpr (IN == LAP3) to = (to + planes * N) & (N * N - 1);
+            return fb[bits(a.rows, to) + bits(a.in_n, (k * NT) & (N - 1)) + in_row];
+        };
+        C y0[EPT], y1[EPT];
+#pragma unroll
+        for (int k = 0; k < EPT; k++) {
+            y0[k] = neighbour(k, -1, 0);
+            y1[k] = neighbour(k, 1, 0);
+        }
+        C z0[IN == LAP3 ? EPT : 1], z1[IN == LAP3 ? EPT : 1];
+        if constexpr (IN == LAP3) {
+#pragma unroll
+            for (int k = 0; k < EPT; k++) {
+                z0[k] = neighbour(k, 0, -1);
+                z1[k] = neighbour(k, 0, 1);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < EPT; k++) lds[uniform_off(lds_bit, k) + lds_thread] = pre[k];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < EPT; k++) {
+            const int e = tid + k * NT, n = bits(a.pk, e & (N - 1));
+            const C* const row = lds + (e >> LN) * K::LS;
+            const C l = row[K::pad((n - 1) & (N - 1))], r = row[K::pad((n + 1) & (N - 1))], c = pre[k];
+            C s;
+            if constexpr (sizeof(T) == 8) {
+                s = cadd(C{0, 0}, y0[k]);
+                s = cadd(cadd(cadd(s, y1[k]), l), r);
+                constexpr T centre = IN == LAP3 ? 6 : 4;
+                if constexpr (IN == LAP3) s = cadd(cadd(s, z0[k]), z1[k]);
+                s = csub(s, C{c.x * centre, c.y * centre});
+            } else {
+                s = cadd(cadd(csub(y0[k], c), csub(y1[k], c)), cadd(csub(l, c), csub(r, c)));
+                if constexpr (IN == LAP3) s = cadd(s, cadd(csub(z0[k], c), csub(z1[k], c)));
+            }
+            pre[k] = C{s.x * scale, s.y * scale};
+        }
+        __syncthreads();  // the raw rows are overwritten
+    };
+
     int g = a.xcd ? (int)xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x;
     if (g < a.groups) fetch(g, IC<0>{}, IC<EPT>{});
     if constexpr (MODE == LOOP_LDS) {
@@ -250,7 +324,7 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
     __syncthreads();
     // exchanges through LDS in one group, each a point to issue a slice of
     // the next group's loads at
-    constexpr int HIN = IN == PACKED ? 1 : 0;
+    constexpr int HIN = PIN_LDS ? 1 : 0;
     constexpr int HOOKS = (DIR == SPEC ? 2 : 1) * (NP - 1) + HIN + (OUT == PACKED ? 1 : 0);
     // Addresses and a multiplier's frequencies are the same for every group,
     // and the compiler would keep them all live across the loop (spills at 256
@@ -263,7 +337,7 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
 #pragma unroll
             for (int i = 0; i < NB; i++) {
                 asm volatile("" : "+s"(in_bit[i]), "+s"(out_bit[i]));
-                if constexpr (IN == PACKED || OUT == PACKED) asm volatile("" : "+s"(lds_bit[i]));
+                if constexpr (PIN_LDS || OUT == PACKED) asm volatile("" : "+s"(lds_bit[i]));
             }
         }
         const int nxt = g + (int)gridDim.x;
@@ -275,7 +349,8 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
             }
         };
         C v[EPT];
-        if constexpr (IN == PACKED) {
+        if constexpr (LAP) laplacian(g);
+        if constexpr (PIN_LDS) {
 #pragma unroll
             for (int k = 0; k < EPT; k++) lds[uniform_off(lds_bit, k) + lds_thread] = pre[k];
             hook(IC<0>{});
@@ -293,7 +368,7 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
                 if constexpr (P + 1 < NP) {
                     // the previous reads of LDS: this group's, or those
                     // before the barrier that ended the last group
-                    if constexpr (P > 0 || IN == PACKED) __syncthreads();
+                    if constexpr (P > 0 || PIN_LDS) __syncthreads();
                     K::template write<P, false, TL>(lds, v, tid);
                     hook(IC<HIN + P>{});
                     __syncthreads();

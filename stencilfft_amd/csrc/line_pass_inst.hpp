@@ -28,7 +28,10 @@ struct Split {
         static constexpr Mode tile_mode = TM;                                  \
     };
 
-constexpr bool is_row(int kind) { return kind == LP_ROW_FWD || kind == LP_ROW_INV || kind == LP_ROW_SPEC; }
+constexpr bool is_lap(int kind) { return kind == LP_ROW_LAP2 || kind == LP_ROW_LAP3; }
+constexpr bool is_row(int kind) {
+    return kind == LP_ROW_FWD || kind == LP_ROW_INV || kind == LP_ROW_SPEC || is_lap(kind);
+}
 
 template <typename T, int LN, bool R16, int KIND, bool SMALL>
 struct Inst {
@@ -41,16 +44,21 @@ struct Inst {
     static constexpr int LEPT = KIND == LP_TILE_SPEC && LN + LLP - LEPT0 > 9 ? LN + LLP - 9 : LEPT0;
     // row multipliers only where no tile is built (FP64 N = 8192 spills)
     static constexpr bool built =
-        LLP >= 0 && (KIND != LP_ROW_SPEC || (S::tile < 0 && !(sizeof(T) == 8 && LN == 13)));
+        LLP >= 0 && (KIND != LP_ROW_SPEC || (S::tile < 0 && !(sizeof(T) == 8 && LN == 13))) &&
+        (!is_lap(KIND) || LN <= (KIND == LP_ROW_LAP2 ? 11 : 10)) &&
+        // five rows of 16 FP64 values per thread spill
+        !(KIND == LP_ROW_LAP3 && sizeof(T) == 8 && LEPT > 3);
     static constexpr int DIR = KIND == LP_TILE_SPEC || KIND == LP_ROW_SPEC ? SPEC
                                : KIND == LP_ROW_INV || KIND == LP_TILE_INV ? INV
                                                                            : FWD;
-    static constexpr Mode MODE = SMALL || DIR == SPEC ? ONCE : ROWS ? S::row_mode : S::tile_mode;
-    static constexpr int IN = KIND == LP_ROW_FWD || KIND == LP_ROW_SPEC    ? PACKED
+    static constexpr Mode MODE = SMALL || DIR == SPEC || is_lap(KIND) ? ONCE : ROWS ? S::row_mode : S::tile_mode;
+    static constexpr int IN = KIND == LP_ROW_LAP2                          ? LAP2
+                              : KIND == LP_ROW_LAP3                         ? LAP3
+                              : KIND == LP_ROW_FWD || KIND == LP_ROW_SPEC   ? PACKED
                               : KIND == LP_ROW_INV || KIND == LP_TILE_INV ? ROW
                                                                           : TILE;
     static constexpr int OUT = KIND == LP_ROW_INV || KIND == LP_ROW_SPEC    ? PACKED
-                               : KIND == LP_ROW_FWD || KIND == LP_TILE_FWD ? ROW
+                               : KIND == LP_ROW_FWD || KIND == LP_TILE_FWD || is_lap(KIND) ? ROW
                                                                            : TILE;
     using K = Line<T, LN, LLP < 0 ? 4 : LLP, LEPT>;
     static constexpr size_t lds() {
@@ -75,7 +83,7 @@ auto with_line_pass(int kind, const LinePassSize& size, Op&& op) {
 #define ZM_LP1(LN, KIND) ZM_LP2(LN, false, KIND) ZM_LP2(LN, true, KIND)
 #define ZM_LP(LN)                                                                                 \
     ZM_LP1(LN, LP_ROW_FWD) ZM_LP1(LN, LP_ROW_INV) ZM_LP1(LN, LP_TILE_FWD) ZM_LP1(LN, LP_TILE_INV) \
-    ZM_LP1(LN, LP_TILE_SPEC) ZM_LP1(LN, LP_ROW_SPEC)
+    ZM_LP1(LN, LP_TILE_SPEC) ZM_LP1(LN, LP_ROW_SPEC) ZM_LP1(LN, LP_ROW_LAP2) ZM_LP1(LN, LP_ROW_LAP3)
     ZM_LP(4) ZM_LP(5) ZM_LP(6) ZM_LP(7) ZM_LP(8) ZM_LP(9) ZM_LP(10) ZM_LP(11) ZM_LP(12) ZM_LP(13)
 #undef ZM_LP
 #undef ZM_LP1

@@ -47,6 +47,7 @@ struct zm_plan {
         zm::LinePassArgs args;
     };
     NatPass nat_fwd[3], nat_inv[3];
+    NatPass nat_lap;       // the x pass of the Laplacian (grid 0: not used)
     NatPass nat_spec;      // the last axis forward, a spectral multiplier, and back
     bool tiled;            // the passes after the first axis hold the repacks
     void* nat_tables[2];  // twiddles of the row and of the tile passes
@@ -216,16 +217,22 @@ zm_plan::NatPass nat_pass(const zm_plan* p, int cus, zm::LinePass kind, int axis
     if (info.occupancy <= 0 || groups > INT32_MAX) return np;
     const int64_t resident = (int64_t)info.occupancy * cus;
     np.grid = (int)(info.loop && resident < groups ? resident : groups);
-    const bool rows = kind == zm::LP_ROW_FWD || kind == zm::LP_ROW_INV || kind == zm::LP_ROW_SPEC;
+    const bool rows = !(kind >= zm::LP_TILE_FWD && kind <= zm::LP_TILE_SPEC);
     np.tables = p->nat_tables[rows ? 0 : 1];
     zm::LinePassArgs& a = np.args;
     a.lgroups = lines - info.lines_log2;
     a.groups = (int)groups;
-    // tile loads of consecutive groups share the cache lines of shorter runs
-    // and DRAM pages: 512^3 FP32 y + z 0.83 -> 0.80 ms, 2048^2 FP32 0.32 ->
-    // 0.25 ms; stores do not (2048^2 FP64 0.223 -> 0.234 ms), nor do short
-    // lines (128^3 FP32 0.091 -> 0.107 ms)
-    a.xcd = kind == zm::LP_TILE_FWD && g.ln >= 9;
+    // Consecutive groups on one XCD, where they share cache lines or rows:
+    // * tile loads (shorter runs, DRAM pages): 512^3 FP32 y + z 0.83 -> 0.80
+    //   ms, 2048^2 FP32 0.32 -> 0.25 ms; not stores (2048^2 FP64 0.223 -> 0.234
+    //   ms) nor short lines (128^3 FP32 0.091 -> 0.107 ms);
+    // * Laplacian rows in 2D (x pass + y pass, 2048^2 x8 FP32 0.277 -> 0.241
+    //   ms) and in 3D while the fields stay in the last-level cache, whose
+    //   planes the XCDs share otherwise (256^3 FP64 0.362 -> 0.318 ms; four of
+    //   them 1.32 -> 1.49, 512^3 FP64 2.81 -> 3.21).
+    const bool lap = kind == zm::LP_ROW_LAP2 || kind == zm::LP_ROW_LAP3;
+    const double mib = (double)p->batch * (double)g.field * sizeof(zm::Cx<T>) / (1 << 20);
+    a.xcd = (kind == zm::LP_TILE_FWD && g.ln >= 9) || (lap && (g.dims == 2 || mib <= 384.0));
     a.field = g.field;
     m.ends(kind, axis, p->tiled, &a);
     return np;
@@ -266,6 +273,10 @@ hipError_t choose_nat_passes(zm_plan* p, int cus) {
         if (axis > 0 || !p->fast_grid_lapx) p->nat_fwd[axis] = nat_pass<T>(p, cus, zm::LP_ROW_FWD, axis);
         p->nat_inv[axis] = nat_pass<T>(p, cus, zm::LP_ROW_INV, axis);
     }
+    // with the forward x pass as a row pass, its Laplacian form has the same
+    // radix order
+    if (p->nat_fwd[0].grid && p->tiled)
+        p->nat_lap = nat_pass<T>(p, cus, d == 2 ? zm::LP_ROW_LAP2 : zm::LP_ROW_LAP3, 0);
     p->nat_spec = nat_pass<T>(p, cus, p->tiled ? zm::LP_TILE_SPEC : zm::LP_ROW_SPEC, d - 1);
     if (!p->nat_spec.grid) return hipSuccess;
     const hipError_t e = hipMalloc(&p->half_sin, sizeof(double) * (size_t)p->geo.n);
@@ -556,6 +567,11 @@ struct Exec {
     // transforming `scale` times the input's Laplacian
     zm_status line(const void* in, void* out, int axis, bool fwd, double scale, bool lapx = false) const {
         const zm_plan::NatPass& np = fwd ? p->nat_fwd[axis] : p->nat_inv[axis];
+        if (lapx && p->nat_lap.grid) {
+            ZM_TRY(nat(p->nat_lap, in, out, scale));
+            timed_inside(p, ZM_STAGE_LAPLACE, record);
+            return ZM_OK;
+        }
         if (compute && !lapx && np.grid) return nat(np, in, out, scale);
         zm::LineArgs a{axis_stride(p, axis), (int)(p->dims.local / p->dims.l), p->lpb};
         if (p->fast && compute) {
@@ -636,15 +652,15 @@ struct Exec {
     }
 
     // The reference's laplace followed by forward_fft (zmodel/main.cu:50-63).
-    // With the fused pass the Laplacian is formed inside the x pass (one
-    // sweep of the field less: 3 instead of 4 in 2D, 5 instead of 6 in 3D);
+    // With a fused pass (line_fast.hip, or the row pass's Laplacian form) the
+    // Laplacian is formed inside the x pass, one sweep of the field less;
     // otherwise the stencil writes `out` and the
     // forward chain runs in place on it (its first pass reads `out` whole
     // before the repack writes it).  Either way the result is bit for bit
     // zm_forward(zm_laplace(in)).
     zm_status laplace_forward(const void* in, void* out, void* s, double lap_scale) const {
         if (p->two_stage) return ZM_ERR_UNSUPPORTED;
-        if (p->fast_grid_lapx > 0) return forward(in, out, s, true, lap_scale);
+        if (p->fast_grid_lapx > 0 || p->nat_lap.grid) return forward(in, out, s, true, lap_scale);
         ZM_TRY(launch_status(timed_launch(p, ZM_STAGE_LAPLACE, st, [&] {
             return zm::launch_stencil<T>(in, out, p->geo, p->batch, zm::OP_LAPLACE, true, lap_scale, false, st);
         }, record)));

@@ -58,6 +58,14 @@ static bool check(int d, int n, int p, int b) {
         if (at(m.frequency0(), lam) != recip_to_freq(ms, cid, d == 2 ? y : e)) return fail("frequency 0", d, n, p, b, d - 1);
         if (d == 3 && at(m.frequency1(), lam) != recip_to_freq(ms, rid, y)) return fail("frequency 1", d, n, p, b, 2);
     }
+    // global rows of the Laplacian pass
+    for (int gl = 0; gl < lines; gl++) {
+        Where w{};
+        global_row_to_local(ms, gl % n, &w.rid, &w.lr);
+        global_row_to_local(ms, gl / n, &w.did, &w.ld);
+        if (d == 2) w.did = w.ld = 0;
+        if (at(m.global_rows(), gl) != addr(g, w)) return fail("global rows", d, n, p, b, 0);
+    }
     for (int tiled = 0; tiled < 2; tiled++)
         for (int axis = 0; axis < d; axis++)
             for (int kind = LP_ROW_FWD; kind <= LP_ROW_SPEC; kind++) {

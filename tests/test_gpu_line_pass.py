@@ -73,3 +73,22 @@ def test_transforms_against_fft(dims, n, p, b, batch, precision):
         assert mx < 1e-13 and zmx < 1e-13, (mx, zmx)
     else:
         assert l2 < 1e-6 and mx < 1e-5 and zl2 < 1e-6 and zmx < 1e-5, (l2, mx, zl2, zmx)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("dims,n,p,b,batch", [s for s in SHAPES if s[1] <= 2048] + [(3, 32, 1, 1, 2), (2, 64, 2, 1, 3)])
+def test_laplace_forward_bits(dims, n, p, b, batch, precision):
+    """The Laplacian formed in the x pass: bit for bit the two calls, at the wrap
+    of rows, planes and columns, in blocks of one and across every rank edge."""
+    from stencilfft_amd import Plan
+    print(f"[gpu] laplace + line pass {precision} {dims}D N={n} P={p} B={b} batch {batch}", flush=True)
+    sys.stdout.flush()
+    pl = Plan(dims, n, p, b, precision=precision, batch=batch)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(3 * n + p)
+    parts = torch.rand((pl.numel(), 2), generator=g, device="cuda", dtype=torch.float64) * 2 - 1
+    x = torch.view_as_complex(parts).to(pl.complex_dtype)
+    for scale in (1.0, float(n * n)):
+        want = torch.view_as_real(pl.forward(pl.laplace(x, scale))).view(torch.int8)
+        got = torch.view_as_real(pl.laplace_forward(x, scale)).view(torch.int8)
+        assert torch.equal(got, want)
