@@ -52,6 +52,9 @@ template <typename T>
 bool fast_line_supported(int vec, int m);
 template <typename T>
 int fast_line_occupancy(int vec, int m, bool fwd, bool mf, bool lapx);
+// whether the plain pass of this direction is built for this (VEC, M) pair
+template <typename T>
+bool fast_line_built(int vec, int m, bool fwd, bool mf);
 // whether the fused Laplacian + x pass (lapx) exists for this (VEC, M) pair
 // in `dims` dimensions with block size `b`
 template <typename T>

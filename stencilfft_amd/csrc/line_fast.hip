@@ -1155,6 +1155,21 @@ constexpr bool kBuildTwoLevel = !(sizeof(T) == 4 && !MF);
 template <typename T, bool MF, int V, int MM>
 constexpr bool kBuildLapx = sizeof(T) == 4 && !MF && (V + MM >= 12 || V + MM <= 10);
 
+// The plain passes: every pair for the MFMA variant; for the vector ALU the
+// one-line groups (N >= 4096), and in FP32 the forward pass of the N <= 1024
+// pairs that have the fused Laplacian, whose radix order it shares.  The other
+// passes of N <= 2048 are line_pass.hpp's, which write the next axis's rows
+// themselves (512^3 FP32: a line pass here and its repack took 0.415 + 0.370 ms,
+// the one pass there 0.37 to 0.41 ms).
+template <typename T, bool MF, int V, int MM, bool FWD>
+constexpr bool kBuildPlain = MF || V + MM >= 12 || (sizeof(T) == 4 && FWD && V + MM <= 10);
+
+template <typename T>
+bool fast_line_built(int vec, int m, bool fwd, bool mf) {
+    const int n = vec * m;
+    return mf ? sizeof(T) == 4 : n >= 4096 || (sizeof(T) == 4 && fwd && n <= 1024);
+}
+
 // 2D: one-line groups; 3D: groups of LPI = 4096 / N lines that lie in one
 // B-block of rows (consecutive global rows)
 template <typename T, bool MF>
@@ -1167,7 +1182,8 @@ bool lapx_built(int vec, int m, int dims, int b) {
 template <typename T, bool MF, typename Op>
 static auto with_fast(int vec, int m, bool fwd, bool lapx, Op&& op) {
 #define ZM_LF2(V, MM, F, FT, LX)                                                                          \
-    if constexpr ((FT || kBuildTwoLevel<T, MF>) && (!LX || (F && kBuildLapx<T, MF, V, MM>))) {        \
+    if constexpr ((FT || kBuildTwoLevel<T, MF>) &&                                                        \
+                  (LX ? F && kBuildLapx<T, MF, V, MM> : kBuildPlain<T, MF, V, MM, F>)) {                  \
         if (vec == (1 << V) && m == (1 << MM) && fwd == F && lapx == LX &&                                \
             fast_line_fulltab<T>(vec, m, MF) == FT)                                                       \
             return op.template run<V, MM, ((V + MM) >= 12 ? 0 : 12 - (V + MM)), F, FT, MF, LX>();         \
@@ -1305,6 +1321,8 @@ template bool fast_line_supported<float>(int, int);
 template bool fast_line_supported<double>(int, int);
 template int fast_line_occupancy<float>(int, int, bool, bool, bool);
 template int fast_line_occupancy<double>(int, int, bool, bool, bool);
+template bool fast_line_built<float>(int, int, bool, bool);
+template bool fast_line_built<double>(int, int, bool, bool);
 template bool fast_line_lapx<float>(int, int, bool, int, int);
 template bool fast_line_lapx<double>(int, int, bool, int, int);
 template hipError_t launch_line_fast<float>(const float2*, float2*, const Geo&, const LineArgs&, const float2*, int,

@@ -422,7 +422,12 @@ zm_status zm_plan_create(zm_plan** plan, const zm_shape* shape, zm_precision pre
                                  : zm::fast_line_lapx<float>(d.vec, d.m, mfma, shape->dims, shape->b);
             const int ol = !lx ? 0 : fp64 ? zm::fast_line_occupancy<double>(d.vec, d.m, true, false, true)
                                           : zm::fast_line_occupancy<float>(d.vec, d.m, true, mfma, true);
-            if (e == hipSuccess && of > 0 && oi > 0) {
+            // a direction that is not built runs line_pass.hpp's passes (grid 0)
+            const bool bf = fp64 ? zm::fast_line_built<double>(d.vec, d.m, true, false)
+                                 : zm::fast_line_built<float>(d.vec, d.m, true, mfma);
+            const bool bi = fp64 ? zm::fast_line_built<double>(d.vec, d.m, false, false)
+                                 : zm::fast_line_built<float>(d.vec, d.m, false, mfma);
+            if (e == hipSuccess && (of > 0 || !bf) && (oi > 0 || !bi)) {
                 p->fast = true;
                 p->fast_grid_fwd = of * cus;
                 p->fast_grid_inv = oi * cus;
@@ -574,8 +579,8 @@ struct Exec {
         }
         if (compute && !lapx && np.grid) return nat(np, in, out, scale);
         zm::LineArgs a{axis_stride(p, axis), (int)(p->dims.local / p->dims.l), p->lpb};
-        if (p->fast && compute) {
-            const int grid = lapx ? p->fast_grid_lapx : fwd ? p->fast_grid_fwd : p->fast_grid_inv;
+        const int grid = lapx ? p->fast_grid_lapx : fwd ? p->fast_grid_fwd : p->fast_grid_inv;
+        if (p->fast && compute && grid) {
             return launch_status(timed_launch(p, lapx ? ZM_STAGE_LINE_LAPLACE : ZM_STAGE_LINE, st, [&] {
                 return zm::launch_line_fast<T>((const zm::Cx<T>*)in, (zm::Cx<T>*)out, p->geo, a, line_tables(),
                                                p->batch, fwd, scale, grid, p->precision == ZM_FP32_MFMA, lapx, st);
