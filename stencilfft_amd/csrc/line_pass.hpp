@@ -397,15 +397,34 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
                     asm volatile("" : "+v"(lam));  // uniform for one-line groups: scalar registers are short
                     // packed ends: 2D, N >= 4096
                     const LineSymbol ls = line_symbol<FAMILY, IN == PACKED>(sp, bits(sp.f0, lam), bits(sp.f1, lam), N);
+                    // In the rolled loop each of a stencil's sines is waited
+                    // for by itself.  The one-line groups have the registers
+                    // to load a butterfly's R ahead and unroll (the whole
+                    // solve, Poisson times stencil: 4096^2 FP32, eight fields
+                    // 2.21 -> 2.11 ms, FP64, two fields 1.13 -> 1.08, 8192^2
+                    // FP32 1.12 -> 1.09; the kernel 763 -> 687 us for 2.15 GB
+                    // at the first); the tiled forms do not (4 to 10
+                    // spilled scalar registers from 4 sines on), and gained
+                    // nothing (256^3 FP32, four fields 1.07 ms either way).
+                    constexpr int AHEAD = FAMILY == SF_STENCIL && IN == PACKED ? R : 1;
+                    double hs[AHEAD] = {};
+                    if constexpr (AHEAD > 1) {
+#pragma unroll
+                        for (int i = 0; i < AHEAD; i++) hs[i] = sp.half_sin[j + i * (N / R)];
+                    }
 #pragma unroll 1
-                    for (int r = 0; r < R; r++) {
-                        const int f = j + r * (N / R);
-                        C* p = lds + l * K::LS + K::pad(f);
-                        double mr, mi;
-                        line_multiplier<FAMILY>(sp, ls, f, N, &mr, &mi);
-                        mr *= factor, mi *= factor;
-                        const double vx = (double)p->x, vy = (double)p->y;
-                        *p = C{(T)(vx * mr - vy * mi), (T)(vx * mi + vy * mr)};
+                    for (int r = 0; r < R; r += AHEAD) {
+                        if constexpr (FAMILY == SF_STENCIL && AHEAD == 1) hs[0] = sp.half_sin[j + r * (N / R)];
+#pragma unroll
+                        for (int i = 0; i < AHEAD; i++) {
+                            const int f = j + (r + i) * (N / R);
+                            C* p = lds + l * K::LS + K::pad(f);
+                            double mr, mi;
+                            line_multiplier<FAMILY>(sp, ls, f, N, hs[i], &mr, &mi);
+                            mr *= factor, mi *= factor;
+                            const double vx = (double)p->x, vy = (double)p->y;
+                            *p = C{(T)(vx * mr - vy * mi), (T)(vx * mi + vy * mr)};
+                        }
                     }
                 }
             };

@@ -60,11 +60,11 @@ __device__ __forceinline__ LineSymbol line_symbol(const SpectralArgs& sp, int f0
     return ls;
 }
 
-// The multiplier at frequency f of the last axis; half_sin[f] = sin(pi s / N)
-// of its signed wavenumber s.
+// The multiplier at frequency f of the last axis, h = half_sin[f] = sin(pi s /
+// N) of its signed wavenumber s (read by the stencil family only).
 template <int FAMILY>
-__device__ __forceinline__ void line_multiplier(const SpectralArgs& sp, const LineSymbol& ls, int f, int n, double* mr,
-                                                double* mi) {
+__device__ __forceinline__ void line_multiplier(const SpectralArgs& sp, const LineSymbol& ls, int f, int n, double h,
+                                                double* mr, double* mi) {
     const int s = signed_wavenumber(f, n);
     const double k2 = sp.kscale * sp.kscale * (ls.k2 + (double)s * s);
     *mi = 0.0;
@@ -75,7 +75,6 @@ __device__ __forceinline__ void line_multiplier(const SpectralArgs& sp, const Li
         if constexpr (FAMILY == SF_PLAIN) {
             *mr = sp.kind == 0 ? poisson : sp.p0;
         } else {
-            const double h = sp.half_sin[f];
             *mr = -4.0 * sp.p0 * (ls.h2 + h * h);
             *mi = ls.im;
             if (sp.kind == 4) {
