@@ -666,21 +666,27 @@ __global__ void __launch_bounds__(NTH) laplace_zmarch_kernel(const E* __restrict
     load_plane(z0, pl[1]);
     load_plane(z0 + 1, pl[2]);
     load_halo(z0, yh[0], xh[0]);
+    // ADD: the values added to, one plane early with four or more per thread
+    // (512^3 FP32, L = 256 0.587 -> 0.576 ms; at two per thread 128^3 lost 3%)
+    constexpr bool EARLY = ADD && KE >= 4;
+    E old[EARLY ? 2 : 1][ADD ? KE : 1];
+    auto load_old = [&](int z, E* o) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < KE; k++) {
+            const int e = tid + NTH * k;
+            o[k] = ld_nt(dst + row_off(z, r0 + (e >> g.ll), cid) + (e & (L - 1)));
+        }
+    };
+    if constexpr (EARLY) load_old(z0, old[0]);
     auto step = [&](int t, auto uc, auto hc) __attribute__((always_inline)) {
         constexpr int U = decltype(uc)::value, C0 = (U + 1) & 3, D = (U + 2) & 3, X = (U + 3) & 3;
         constexpr int H = decltype(hc)::value, HN = H ^ 1;
         const int gd = z0 + t;
-        E old[ADD ? KE : 1];
-        if constexpr (ADD) {
-#pragma unroll
-            for (int k = 0; k < KE; k++) {
-                const int e = tid + NTH * k;
-                old[k] = ld_nt(dst + row_off(gd, r0 + (e >> g.ll), cid) + (e & (L - 1)));
-            }
-        }
+        if constexpr (ADD && !EARLY) load_old(gd, old[0]);
         if (t + 1 < tz) {
             load_plane(gd + 2, pl[X]);
             load_halo(gd + 1, yh[HN], xh[HN]);
+            if constexpr (EARLY) load_old(gd + 1, old[HN]);
         }
 #pragma unroll
         for (int k = 0; k < KE; k++) {
@@ -709,7 +715,7 @@ __global__ void __launch_bounds__(NTH) laplace_zmarch_kernel(const E* __restrict
             const E a = tile[pos - W], b = tile[pos + W], l = tile[pos - VEC], rr = tile[pos + VEC];
             E acc = lap_combine<sizeof(S) == 8, O, E, S>(a, b, l, rr, pl[U][k], pl[D][k], pl[C0][k], true);
             if (apply_scale) acc = O::mul(acc, scale);
-            if constexpr (ADD) acc = O::add(old[k], O::mul(acc, alpha));
+            if constexpr (ADD) acc = O::add(old[EARLY ? H : 0][k], O::mul(acc, alpha));
             dst[row_off(gd, r0 + r - 1, cid) + c] = acc;
         }
         __syncthreads();
@@ -805,9 +811,16 @@ static hipError_t laplace_zmarch_inst(const E* in, E* out, const Geo& g, int bat
     // workgroups (two per CU); 512^3 FP32 ran 0.41 ms at 128 planes against
     // 0.45-0.47 ms at 32-64.  Small fields go down to 4 planes: with 32 at
     // least, 64^3 and 128^3 FP32 ran on 16 and 128 workgroups (17.0 -> 4.5,
-    // 26.3 -> 10.0 us)
+    // 26.3 -> 10.0 us).  A tile of fewer than 2048 elements has too little in
+    // flight per workgroup for two per CU: down to 32 planes (more strips
+    // re-read too much), L = 128 and 64 strips go on to 1024 workgroups (256^3,
+    // P = 2, four FP32 fields 0.236 -> 0.211 ms, FP64 0.450 -> 0.420; 2048 took
+    // P = 4 0.231 -> 0.236) and L = 32 strips to 4096 (128^3, P = 4, sixteen
+    // fields 0.137 -> 0.111)
     int tz = g.n < 128 ? g.n : 128;
     while (tz > 4 && (int64_t)ntiles * g.p * (g.n / tz) * batch < 512) tz >>= 1;
+    constexpr int fill = KE == 1 ? 4096 : KE * NTH < 2048 ? 1024 : 512;
+    while (tz > 32 && (int64_t)ntiles * g.p * (g.n / tz) * batch < fill) tz >>= 1;
     const unsigned blocks = (unsigned)((int64_t)ntiles * g.p * (g.n / tz));
     const size_t lds = sizeof(E) * (size_t)(R + 2) * (size_t)(g.l + 2 * g.vec);
     const bool two = 2 * R * g.vec > NTH;

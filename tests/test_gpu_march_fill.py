@@ -50,3 +50,26 @@ def test_marches_against_differences(dims, n, p, b, batch, precision):
         want = sum(torch.roll(nat, s, a) for a in range(1, dims + 1) for s in (1, -1)) - 2 * dims * nat
         got = pl.laplace(packed, 1.0).to(nat.dtype)
         assert (got - _pack(want, dims, n, p, b)).abs().max().item() < tol * 2 * 2 * dims
+
+
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+@pytest.mark.parametrize("n,p,b,batch", [(64, 2, 4, 8), (64, 1, 4, 16), (128, 2, 8, 8), (128, 4, 4, 8), (256, 2, 8, 3),
+                                         (256, 1, 16, 1)])
+def test_depth_strips_leave_every_value(n, p, b, batch, precision):
+    """A batch's depth strips are as long as its size asks for; each value is
+    the same sum whatever the strip, so the batch equals its fields alone bit
+    for bit, and the accumulating form equals the two operations."""
+    from stencilfft_amd import Plan
+    print(f"[gpu] depth strips {precision} N={n} P={p} B={b} batch {batch}", flush=True)
+    sys.stdout.flush()
+    pl, one = Plan(3, n, p, b, precision=precision, batch=batch), Plan(3, n, p, b, precision=precision)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + batch)
+    x, z = (torch.rand((2, pl.numel()), generator=g, device="cuda", dtype=torch.float64) * 2 - 1
+            ).to(pl.real_dtype).repeat_interleave(2, 1).reshape(2, -1, 2).unbind(0)
+    x, z = torch.view_as_complex(x.contiguous()), torch.view_as_complex((z * 0.5).contiguous())
+    lap = pl.laplace(x, 2.0)
+    for xf, lf in zip(x.chunk(batch), lap.chunk(batch)):
+        assert torch.equal(one.laplace(xf.contiguous(), 2.0), lf)
+    want = torch.view_as_real(z) + 0.25 * torch.view_as_real(lap)
+    assert torch.equal(torch.view_as_real(pl.laplace_add(x, z, 2.0, 0.25)), want)
