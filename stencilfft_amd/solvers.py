@@ -45,9 +45,16 @@ def sq_norm(r):
     return torch.view_as_real(r).pow(2).sum()
 
 
+def _holds_its_values(t):
+    """The storage of t, read element by element, is t: a contiguous tensor of no
+    subclass, with no conjugation or negation left to carry out."""
+    return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_contiguous() and not t.is_conj()
+            and not t.is_neg())
+
+
 def poisson_loss(f, g, plan, length=1.0, form="spatial"):
     # a target that is a plain constant field: residual and norm in one pass
-    if (form == "spectral" and torch.is_tensor(f) and torch.is_tensor(g) and not g.requires_grad and g.is_contiguous()
+    if (form == "spectral" and torch.is_tensor(f) and _holds_its_values(g) and not g.requires_grad
             and g.shape == f.shape and g.dtype == f.dtype == plan.complex_dtype and g.device == f.device):
         n = plan.shape.n
         return ag.solve_misfit(f, g, plan, "poisson_stencil", float(n * n), 1.0 / n, length)
