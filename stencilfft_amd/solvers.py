@@ -21,6 +21,7 @@ adjoint_heat     the same gradient as a hand-written adjoint loop
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 
 from . import autograd as ag
 
@@ -46,10 +47,11 @@ def sq_norm(r):
 
 
 def _holds_its_values(t):
-    """The storage of t, read element by element, is t: a contiguous tensor of no
-    subclass, with no conjugation or negation left to carry out."""
+    """The storage of t, read element by element, is all of t: a contiguous
+    tensor of no subclass, with no conjugation or negation left to carry out and
+    no forward-mode tangent."""
     return (type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_contiguous() and not t.is_conj()
-            and not t.is_neg())
+            and not t.is_neg() and forward_ad.unpack_dual(t).tangent is None)
 
 
 def poisson_loss(f, g, plan, length=1.0, form="spatial"):

@@ -1,6 +1,7 @@
 """Targets of the Poisson loss whose storage is not their value: lazily conjugated
-or negated, or a subclass that computes its values.  The fused misfit reads the target's storage, so these have
-to take the separate operators, as torch evaluates them.
+or negated, a subclass that computes its values, or with a forward-mode tangent.
+The fused misfit reads the target's storage, so these have to take the separate
+operators, as torch evaluates them.
 
 On the CPU a stand-in plan reads storage through data_ptr() like the library's
 entries do; on the GPU the plan itself."""
@@ -97,3 +98,21 @@ def test_loss_of_a_target_that_is_not_its_storage(form, device):
     assert abs(got.item() - want.item()) <= 1e-13 * want.item()
     (gg,), (gw,) = torch.autograd.grad(got, f), torch.autograd.grad(want, f)
     assert (gg - gw).abs().max().item() <= 1e-12 * gw.abs().max().item()
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_tangent_of_the_target(device):
+    """Forward-mode differentiation along the target: d ||r||^2 = -2 Re <r, dg>."""
+    from torch.autograd import forward_ad
+    from stencilfft_amd import solvers
+    print(f"target tangent on {device}", flush=True)
+    pl = _plan(device)
+    f, g = _fields(device)
+    dg = f.flip(0).resolve_conj().clone()
+    r = solvers.poisson_residual(f, g, pl, form="spectral")
+    with forward_ad.dual_level():
+        loss = solvers.poisson_loss(f, forward_ad.make_dual(g, dg), pl, form="spectral")
+        got = forward_ad.unpack_dual(loss).tangent.item()
+    want = -2 * torch.vdot(dg, r).real.item()
+    scale = 2 * (torch.linalg.vector_norm(r) * torch.linalg.vector_norm(dg)).item()
+    assert abs(got - want) <= 1e-13 * scale
