@@ -22,82 +22,88 @@ from __future__ import annotations
 import torch
 
 
+def _raw(t):
+    """t with its storage in the order and with the values that the library reads:
+    contiguous, lazy conjugations and negations carried out."""
+    return t.resolve_conj().resolve_neg().contiguous()
+
+
 class _Forward(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, plan):
         ctx.plan = plan
-        return plan.forward(x.contiguous())
+        return plan.forward(_raw(x))
 
     @staticmethod
     def backward(ctx, g):
-        return ctx.plan.forward_adjoint(g.contiguous()), None
+        return ctx.plan.forward_adjoint(_raw(g)), None
 
 
 class _Inverse(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, plan, scale):
         ctx.plan, ctx.scale = plan, scale
-        return plan.inverse(x.contiguous(), scale)
+        return plan.inverse(_raw(x), scale)
 
     @staticmethod
     def backward(ctx, g):
-        return ctx.plan.inverse_adjoint(g.contiguous(), ctx.scale), None, None
+        return ctx.plan.inverse_adjoint(_raw(g), ctx.scale), None, None
 
 
 class _Laplace(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, plan, scale):
         ctx.plan, ctx.scale = plan, scale
-        return plan.laplace(x.contiguous(), scale)
+        return plan.laplace(_raw(x), scale)
 
     @staticmethod
     def backward(ctx, g):
-        return ctx.plan.laplace(g.contiguous(), ctx.scale), None, None
+        return ctx.plan.laplace(_raw(g), ctx.scale), None, None
 
 
 class _Dx4(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, plan, delta):
         ctx.plan, ctx.delta = plan, delta
-        return plan.dx4(x.contiguous(), delta)
+        return plan.dx4(_raw(x), delta)
 
     @staticmethod
     def backward(ctx, g):
-        return ctx.plan.dx4(g.contiguous(), ctx.delta, adjoint=True), None, None
+        return ctx.plan.dx4(_raw(g), ctx.delta, adjoint=True), None, None
 
 
 class _Dy4(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, plan, delta):
         ctx.plan, ctx.delta = plan, delta
-        return plan.dy4(x.contiguous(), delta)
+        return plan.dy4(_raw(x), delta)
 
     @staticmethod
     def backward(ctx, g):
-        return ctx.plan.dy4(g.contiguous(), ctx.delta, adjoint=True), None, None
+        return ctx.plan.dy4(_raw(g), ctx.delta, adjoint=True), None, None
 
 
 class _Dz4(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, plan, delta):
         ctx.plan, ctx.delta = plan, delta
-        return plan.dz4(x.contiguous(), delta)
+        return plan.dz4(_raw(x), delta)
 
     @staticmethod
     def backward(ctx, g):
-        return ctx.plan.dz4(g.contiguous(), ctx.delta, adjoint=True), None, None
+        return ctx.plan.dz4(_raw(g), ctx.delta, adjoint=True), None, None
 
 
 class _Spectral(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, plan, kind, p0, p1, length):
         ctx.args = (plan, kind, p0, p1, length)
-        return plan.spectral_multiply(x.contiguous(), kind, p0, p1, length)
+        return plan.spectral_multiply(_raw(x), kind, p0, p1, length)
 
     @staticmethod
     def backward(ctx, g):
         plan, kind, p0, p1, length = ctx.args
-        return (plan.spectral_multiply(g.contiguous(), kind, p0, p1, length, adjoint=True),
+        return (plan.spectral_multiply(_raw(g), kind, p0, p1, length, adjoint=True),
                 None, None, None, None, None)
 
 
@@ -105,29 +111,29 @@ class _SpectralSolve(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, plan, *args):
         ctx.plan, ctx.args = plan, args
-        return plan.spectral_solve(x.contiguous(), *args)
+        return plan.spectral_solve(_raw(x), *args)
 
     @staticmethod
     def backward(ctx, g):
-        return (ctx.plan.spectral_solve(g.contiguous(), *ctx.args, adjoint=True),) + (None,) * (1 + len(ctx.args))
+        return (ctx.plan.spectral_solve(_raw(g), *ctx.args, adjoint=True),) + (None,) * (1 + len(ctx.args))
 
 
 class _HeatStep(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, plan, *args):
         ctx.plan, ctx.args = plan, args
-        return plan.heat_step(x.contiguous(), *args)
+        return plan.heat_step(_raw(x), *args)
 
     @staticmethod
     def backward(ctx, g):
-        return (ctx.plan.heat_step(g.contiguous(), *ctx.args),) + (None,) * (1 + len(ctx.args))
+        return (ctx.plan.heat_step(_raw(g), *ctx.args),) + (None,) * (1 + len(ctx.args))
 
 
 class _SolveMisfit(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, g, plan, *args):
         ctx.plan, ctx.args = plan, args
-        r = plan.spectral_solve(x.contiguous(), *args)
+        r = plan.spectral_solve(_raw(x), *args)
         loss = plan.residual_norm(r, g)
         ctx.save_for_backward(r)
         return loss
@@ -135,7 +141,7 @@ class _SolveMisfit(torch.autograd.Function):
     @staticmethod
     def backward(ctx, gloss):
         (r,) = ctx.saved_tensors
-        grad = ctx.plan.spectral_solve(r, *ctx.args, adjoint=True, factor=2.0 * gloss.to(torch.float64))
+        grad = ctx.plan.spectral_solve(_raw(r), *ctx.args, adjoint=True, factor=2.0 * gloss.to(torch.float64))
         return (grad,) + (None,) * (2 + len(ctx.args))
 
 

@@ -191,6 +191,16 @@ class Plan:
         return out
 
     @staticmethod
+    def _check_raw(like, *tensors):
+        """The storage of each tensor holds its values (no lazy conjugation or
+        negation) and lies on the device of `like`."""
+        for t in tensors:
+            if t.is_conj() or t.is_neg():
+                raise ValueError("a lazily conjugated or negated tensor: call resolve_conj() / resolve_neg() first")
+            if t.device != like.device:
+                raise ValueError(f"tensors on {like.device} and {t.device}")
+
+    @staticmethod
     def _span(t):
         start = t.data_ptr()
         return start, start + t.numel() * t.element_size()
@@ -326,11 +336,13 @@ class Plan:
         two-stage plans).  `factor`: a CUDA tensor of one float64 that
         multiplies the multiplier."""
         out = self._out(x, out)
+        self._check_raw(x, x, out)
         if factor is not None:
             import torch
             if factor.dtype != torch.float64 or factor.numel() != 1 or factor.device != x.device:
                 raise ValueError(f"factor must be one float64 on {x.device}, got {tuple(factor.shape)} {factor.dtype} "
                                  f"on {factor.device}")
+            self._check_raw(x, factor)
         if self.two_stage:
             import torch
             ts = torch.cuda.ExternalStream(stream) if isinstance(stream, int) else stream
@@ -350,6 +362,7 @@ class Plan:
         """acc += alpha * laplace(x, scale) for complex fields; returns acc."""
         self._check_tensor(x)
         self._check_tensor(acc)
+        self._check_raw(x, x, acc)
         L.check(L._lib().zm_laplace_add(self._h, _ptr(x), _ptr(acc), float(scale), float(alpha), _stream(stream)),
                 "zm_laplace_add")
         return acc
@@ -368,6 +381,7 @@ class Plan:
         import torch
         self._check_tensor(acc)
         self._check_tensor(g)
+        self._check_raw(acc, acc, g)
         partials = torch.empty(L.ZM_NORM_PARTIALS, dtype=torch.float64, device=acc.device)
         norm2 = torch.empty((), dtype=self.real_dtype, device=acc.device)
         L.check(L._lib().zm_residual_norm(self._h, _ptr(acc), _ptr(g), _ptr(partials), _ptr(norm2), _stream(None)),

@@ -1,7 +1,7 @@
-"""Targets of the Poisson loss whose storage is not their value: lazily conjugated
-or negated, a subclass that computes its values, or with a forward-mode tangent.
-The fused misfit reads the target's storage, so these have to take the separate
-operators, as torch evaluates them.
+"""Tensors whose storage is not their value: lazily conjugated or negated, a
+subclass that computes its values, or with a forward-mode tangent.  The library
+reads storage, so the operators carry lazy forms out first, and a Poisson target
+of any of these forms takes the separate operators, as torch evaluates them.
 
 On the CPU a stand-in plan reads storage through data_ptr() like the library's
 entries do; on the GPU the plan itself."""
@@ -41,6 +41,9 @@ class RawPlan:
         if factor is not None:
             m = m * factor
         return (torch.fft.ifft2(m * torch.fft.fft2(self.raw(x).reshape(n, n)))).reshape(x.shape)
+
+    def heat_step(self, x, nu, dt, lap_scale, length):
+        return 3.0 * self.raw(x).reshape(x.shape)
 
     def residual_norm(self, acc, g):
         acc.copy_(self.raw(acc) - self.raw(g))
@@ -116,3 +119,50 @@ def test_tangent_of_the_target(device):
     want = -2 * torch.vdot(dg, r).real.item()
     scale = 2 * (torch.linalg.vector_norm(r) * torch.linalg.vector_norm(dg)).item()
     assert abs(got - want) <= 1e-13 * scale
+
+
+def _operators(device):
+    from stencilfft_amd import autograd as ag
+    ops = {"spectral_solve": lambda t, pl: ag.spectral_solve(t, pl, "heat", 1e-3, 1e-2),
+           "heat_step": lambda t, pl: ag.heat_step(t, pl, 1e-3, 1e-2),
+           "solve_misfit": lambda t, pl: ag.solve_misfit(t, torch.ones_like(t, dtype=pl.complex_dtype), pl, "poisson")}
+    if device == "cuda":
+        ops.update({"fft": ag.fft, "ifft": ag.ifft, "laplace": ag.laplace, "dx4": ag.dx4, "dy4": ag.dy4,
+                    "spectral": lambda t, pl: ag.spectral(t, pl, "stencil", 2.0, 0.25)})
+    return ops
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_operators_of_lazy_tensors(device):
+    """Inputs and incoming gradients with the conjugation or negation still to be
+    carried out: bit for bit the operator of the tensor written out."""
+    pl = _plan(device)
+    x, _ = _fields(device)
+    for name, op in _operators(device).items():
+        for form in ("conj", "neg", "neg_conj"):
+            print(f"{name} of {form} on {device}", flush=True)
+            lazy, written_out = FORMS[form]
+            assert torch.equal(op(lazy(x), pl), op(written_out(x), pl)), (name, form)
+            if name == "solve_misfit":  # a real loss
+                continue
+            xr = x.clone().requires_grad_(True)
+            (got,) = torch.autograd.grad(op(xr, pl), xr, grad_outputs=lazy(x))
+            (want,) = torch.autograd.grad(op(xr, pl), xr, grad_outputs=written_out(x))
+            assert torch.equal(got, want), (name, form)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not has_gpu(), reason="needs a GPU")
+def test_plan_refuses_lazy_tensors():
+    pl = _plan("cuda")
+    x, acc = _fields("cuda")
+    factor = torch.ones((), dtype=torch.float64, device="cuda")
+    for lazy in (x.conj(), torch._neg_view(x)):
+        for call in (lambda: pl.spectral_solve(lazy, "poisson"), lambda: pl.spectral_solve(x, "poisson", out=lazy),
+                     lambda: pl.heat_step(lazy, 1e-3, 1e-2), lambda: pl.laplace_add(lazy, acc),
+                     lambda: pl.laplace_add(acc, lazy), lambda: pl.residual_norm(lazy, acc),
+                     lambda: pl.residual_norm(acc, lazy)):
+            with pytest.raises(ValueError, match="lazily"):
+                call()
+    with pytest.raises(ValueError, match="lazily"):
+        pl.spectral_solve(x, "poisson", factor=torch._neg_view(factor))
