@@ -345,6 +345,8 @@ class Plan:
             self._check_raw(x, factor)
         if self.two_stage:
             import torch
+            if out.data_ptr() == x.data_ptr():  # as zm_spectral_solve on the other plans
+                raise L.ZmError(L.ZM_ERR_ALIAS, "zm_spectral_solve")
             ts = torch.cuda.ExternalStream(stream) if isinstance(stream, int) else stream
             with torch.cuda.stream(ts):  # the spectrum belongs to the stream that uses it (None: the current one)
                 y = self.forward(x, scratch=scratch)
