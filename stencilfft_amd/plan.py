@@ -345,8 +345,6 @@ class Plan:
             self._check_raw(x, factor)
         if self.two_stage:
             import torch
-            if out.data_ptr() == x.data_ptr():  # as zm_spectral_solve on the other plans
-                raise L.ZmError(L.ZM_ERR_ALIAS, "zm_spectral_solve")
             ts = torch.cuda.ExternalStream(stream) if isinstance(stream, int) else stream
             with torch.cuda.stream(ts):  # the spectrum belongs to the stream that uses it (None: the current one)
                 y = self.forward(x, scratch=scratch)
@@ -373,6 +371,8 @@ class Plan:
                   stream=None):
         """inverse(exp(-nu |k|^2 dt) forward(x)) / N^d + dt * laplace(x, lap_scale)
         (self-adjoint)."""
+        if out is not None and out.data_ptr() == x.data_ptr():  # the Laplacian reads x after the solve
+            raise L.ZmError(L.ZM_ERR_ALIAS, "heat_step")
         norm = 1.0 / float(self.shape.n) ** self.shape.dims
         out = self.spectral_solve(x, "heat", nu, dt, length, norm, out=out, scratch=scratch, stream=stream)
         return self.laplace_add(x, out, lap_scale, dt, stream=stream)
