@@ -106,7 +106,14 @@ def rollout(u0, step, nsteps, every=8):
 
 def adjoint_heat(g, plan, nsteps, nu, dt, lap_scale=1.0, length=1.0):
     """Pull a final-state gradient back through nsteps heat steps with the
-    adjoint kernels directly: step^H = F^H M IFFT^H + dt Lap (M real, Lap symmetric)."""
+    adjoint kernels directly: step^H = F^H M IFFT^H + dt Lap (M real, Lap symmetric).
+    The operators run one by one, so the result does not share the fused step's
+    kernels (heat_step and its backward) and can check them."""
+    n_d = float(plan.shape.n) ** plan.shape.dims
     for _ in range(nsteps):
-        g = plan.heat_step(g.contiguous(), nu, dt, lap_scale, length)  # self-adjoint
+        g = ag._raw(g)
+        a = plan.inverse_adjoint(g, 1.0 / n_d)
+        a = plan.spectral_multiply(a, "heat", nu, dt, length, adjoint=True)
+        a = plan.forward_adjoint(a)
+        g = a + dt * plan.laplace(g, lap_scale)
     return g
