@@ -52,9 +52,10 @@ template <typename T>
 bool fast_line_supported(int vec, int m);
 template <typename T>
 int fast_line_occupancy(int vec, int m, bool fwd, bool mf, bool lapx);
-// whether the plain pass of this direction is built for this (VEC, M) pair
+// whether the plain passes of both directions are built for this (VEC, M) pair
+// (beside the fused Laplacian, below, the forward one is)
 template <typename T>
-bool fast_line_built(int vec, int m, bool fwd, bool mf);
+bool fast_line_plain(int vec, int m, bool mf);
 // whether the fused Laplacian + x pass (lapx) exists for this (VEC, M) pair
 // in `dims` dimensions with block size `b`
 template <typename T>
@@ -69,8 +70,8 @@ int fast_line_lapx_lines_log2(int vec, int m);
 template <typename T>
 hipError_t launch_line_fast(const Cx<T>* in, Cx<T>* out, const Geo& g, const LineArgs& a, const Cx<T>* tables,
                             int batch, bool fwd, double scale, int grid_x, bool mf, bool lapx, hipStream_t stream);
+// entries of the specialised pass's table
 int line_table_entries(int vec, int m);
-hipError_t launch_line_tables(double2* t64, float2* t32, int vec, int m, hipStream_t stream);
 
 // A bit permutation v -> sum over fields of ((v >> from) & mask) << to.
 struct BitField {
@@ -125,11 +126,17 @@ enum LinePass {
     LP_ROW_LAP2 = 6,   // 5-point Laplacian of packed -> row
     LP_ROW_LAP3 = 7    // 7-point Laplacian of packed -> row
 };
+// the radix passes of a line and the size of their twiddle table: for each pass
+// p >= 1 of radix R after NS = the product of the radices before it, W_{NS R}^(jm r)
+// at r NS + jm, one pass after the other
+struct LineRadices {
+    int np, entries;
+    int lr[7];  // log2 of the radices
+};
 struct LinePassInfo {
     int lines_log2;  // log2 of the lines per workgroup; -1: not built
-    int occupancy;   // workgroups per CU
     bool loop;       // workgroups loop over groups (else one group each)
-    int tables;      // twiddle table entries
+    LineRadices radices;
 };
 // Lines of 2^ln points; small: the variant for fields with few line groups;
 // radix16: the split with the largest radices, where it differs.
@@ -139,8 +146,9 @@ struct LinePassSize {
 };
 template <typename T>
 LinePassInfo line_pass_info(LinePass kind, const LinePassSize& size);
+// workgroups per CU (0: the query failed), the grid of the looping passes
 template <typename T>
-hipError_t launch_line_pass_tables(LinePass kind, const LinePassSize& size, Cx<T>* tables, hipStream_t stream);
+int line_pass_occupancy(LinePass kind, const LinePassSize& size);
 template <typename T>
 hipError_t launch_line_pass(LinePass kind, const LinePassSize& size, const Cx<T>* in, Cx<T>* out, const LinePassArgs& a,
                             const Cx<T>* tables, double scale, const SpectralArgs& sp, int grid, hipStream_t stream);
@@ -156,11 +164,20 @@ template <typename T>
 hipError_t launch_laplace_add(const Cx<T>* in, Cx<T>* out, const Geo& g, int batch, double coef, double alpha,
                               hipStream_t stream);
 
-// twiddle tables exp(-2 pi i t / n), t in [0, n), computed in FP64
-hipError_t launch_twiddles(double2* tw64, float2* tw32, int n, hipStream_t stream);
-
-// half_sin[f] = sin(pi s / n), s the signed wavenumber of f < n
-hipError_t launch_half_sin(double* half_sin, int n, hipStream_t stream);
+// The tables of a plan, computed in FP64 and rounded to its precision; null: not
+// wanted.
+template <typename T>
+struct PlanTables {
+    int n;
+    Cx<T>* tw;                // exp(-2 pi i t / n), t < n
+    Cx<T>* line;              // the specialised pass's (line_fast.hip), of `line_entries`
+    int line_entries, line_s;
+    Cx<T>* nat[2];            // the row and the tile passes' (line_pass.hpp)
+    LineRadices radices[2];
+    double* half_sin;         // sin(pi s / n), s the signed wavenumber of f < n
+};
+template <typename T>
+hipError_t launch_plan_tables(const PlanTables<T>& t, hipStream_t stream);
 
 // r -= g over n elements; *norm2 = sum |r|^2 (FP64 partial sums in `partials`)
 constexpr int kNormBlocks = 2048;

@@ -1165,9 +1165,8 @@ template <typename T, bool MF, int V, int MM, bool FWD>
 constexpr bool kBuildPlain = MF || V + MM >= 12 || (sizeof(T) == 4 && FWD && V + MM <= 10);
 
 template <typename T>
-bool fast_line_built(int vec, int m, bool fwd, bool mf) {
-    const int n = vec * m;
-    return mf ? sizeof(T) == 4 : n >= 4096 || (sizeof(T) == 4 && fwd && n <= 1024);
+bool fast_line_plain(int vec, int m, bool mf) {
+    return mf ? sizeof(T) == 4 : vec * m >= 4096;
 }
 
 // 2D: one-line groups; 3D: groups of LPI = 4096 / N lines that lie in one
@@ -1278,51 +1277,19 @@ hipError_t launch_line_fast(const Cx<T>* in, Cx<T>* out, const Geo& g, const Lin
     return with_fast<T, false>(g.vec, g.m, fwd, lapx, LaunchOp<T>(op));
 }
 
-// FP64 twiddle tables of a line (N = vec*m, S = max(vec, m)), rounded for
-// FP32:  [W_S^t, t < S | W_N^t, t < 64 | W_N^(64 t), t < N/64 | W_N^t, t < N]
-__global__ void line_tables_kernel(double2* t64, float2* t32, int n, int s) {
-    const int nb = n / 64 > 0 ? n / 64 : 1;
-    const int nt = s + 64 + nb + n;
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nt) return;
-    double num, den;
-    if (t < s) {
-        num = t;
-        den = s;
-    } else if (t < s + 64) {
-        num = t - s;
-        den = n;
-    } else if (t < s + 64 + nb) {
-        num = 64.0 * (t - s - 64);
-        den = n;
-    } else {
-        num = t - s - 64 - nb;
-        den = n;
-    }
-    double sn, cs;
-    sincospi(-2.0 * num / den, &sn, &cs);
-    t64[t] = double2{cs, sn};
-    t32[t] = float2{(float)cs, (float)sn};
-}
-
+// The table of a line (N = vec*m, S = max(vec, m)), filled by plan_tables_kernel:
+// [W_S^t, t < S | W_N^t, t < 64 | W_N^(64 t), t < N/64 | W_N^t, t < N]
 int line_table_entries(int vec, int m) {
     const int n = vec * m, s = vec > m ? vec : m;
     return s + 64 + (n / 64 > 0 ? n / 64 : 1) + n;
-}
-
-hipError_t launch_line_tables(double2* t64, float2* t32, int vec, int m, hipStream_t stream) {
-    const int nt = line_table_entries(vec, m);
-    hipLaunchKernelGGL(line_tables_kernel, dim3((nt + 255) / 256), dim3(256), 0, stream, t64, t32, vec * m,
-                       vec > m ? vec : m);
-    return hipGetLastError();
 }
 
 template bool fast_line_supported<float>(int, int);
 template bool fast_line_supported<double>(int, int);
 template int fast_line_occupancy<float>(int, int, bool, bool, bool);
 template int fast_line_occupancy<double>(int, int, bool, bool, bool);
-template bool fast_line_built<float>(int, int, bool, bool);
-template bool fast_line_built<double>(int, int, bool, bool);
+template bool fast_line_plain<float>(int, int, bool);
+template bool fast_line_plain<double>(int, int, bool);
 template bool fast_line_lapx<float>(int, int, bool, int, int);
 template bool fast_line_lapx<double>(int, int, bool, int, int);
 template hipError_t launch_line_fast<float>(const float2*, float2*, const Geo&, const LineArgs&, const float2*, int,

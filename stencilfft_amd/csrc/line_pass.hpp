@@ -55,6 +55,11 @@ struct Line {
     // twiddles of pass p >= 1: W_{NS R}^(jm r) at r NS + jm
     static constexpr int tw_off(int p) { return p <= 1 ? 0 : tw_off(p - 1) + (1 << (lns(p - 1) + lr(p - 1))); }
     static constexpr int TW = tw_off(NP);
+    static constexpr LineRadices radices() {
+        LineRadices r{NP, TW, {}};
+        for (int p = 0; p < NP; p++) r.lr[p] = lr(p);
+        return r;
+    }
 
     // LDS index of element n of line l.  One padding element after every
     // 2^PS, 2^(2 PS), ..: the lanes of an LDS phase (16 of 8 bytes, 8 of 16)
@@ -465,20 +470,6 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
         __syncthreads();  // the next group's writes overwrite LDS
         g = nxt;
     }
-}
-
-// tables[tw_off(p) + r NS + jm] = W_{NS R}^(jm r) for the radices of (LN, LEPT)
-template <typename T, int LN, int LEPT>
-__global__ void line_pass_tables_kernel(Cx<T>* out) {
-    using K = Line<T, LN, (LEPT + 6 > LN ? LEPT + 6 - LN : 0), LEPT>;  // the tables depend on LN and LEPT only
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= K::TW) return;
-    int p = 1;
-    while (p + 1 < K::NP && t >= K::tw_off(p + 1)) p++;
-    const int e = t - K::tw_off(p), lns = K::lns(p);
-    double s, c;
-    sincospi(-2.0 * (double)((e & ((1 << lns) - 1)) * (e >> lns)) / (double)(1 << (lns + K::lr(p))), &s, &c);
-    out[t] = Cx<T>{(T)c, (T)s};
 }
 
 }  // namespace lp

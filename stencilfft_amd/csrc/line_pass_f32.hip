@@ -19,7 +19,7 @@ ZM_SPLIT(float, 13, false, 4, 0, -1, ONCE, 4, -1, -1, ONCE)
 }  // namespace lp
 
 template LinePassInfo line_pass_info<float>(LinePass, const LinePassSize&);
-template hipError_t launch_line_pass_tables<float>(LinePass, const LinePassSize&, float2*, hipStream_t);
+template int line_pass_occupancy<float>(LinePass, const LinePassSize&);
 template hipError_t launch_line_pass<float>(LinePass, const LinePassSize&, const float2*, float2*, const LinePassArgs&, const float2*, double,
                                                const SpectralArgs&, int, hipStream_t);
 

@@ -20,7 +20,7 @@ ZM_SPLIT(double, 13, false, 4, 0, -1, ONCE, 4, -1, -1, ONCE)
 }  // namespace lp
 
 template LinePassInfo line_pass_info<double>(LinePass, const LinePassSize&);
-template hipError_t launch_line_pass_tables<double>(LinePass, const LinePassSize&, double2*, hipStream_t);
+template int line_pass_occupancy<double>(LinePass, const LinePassSize&);
 template hipError_t launch_line_pass<double>(LinePass, const LinePassSize&, const double2*, double2*, const LinePassArgs&, const double2*, double,
                                                 const SpectralArgs&, int, hipStream_t);
 

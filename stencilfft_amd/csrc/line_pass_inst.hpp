@@ -95,26 +95,21 @@ auto with_line_pass(int kind, const LinePassSize& size, Op&& op) {
 struct InfoOp {
     template <typename I>
     LinePassInfo run() {
-        LinePassInfo r{I::LLP, 0, I::MODE != ONCE, I::K::TW};
-        if (I::prepare() != hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&r.occupancy, I::fn(), I::K::NT, I::lds()) != hipSuccess)
-            r.occupancy = 0;
-        return r;
+        return LinePassInfo{I::LLP, I::MODE != ONCE, I::K::radices()};
     }
-    LinePassInfo none() { return LinePassInfo{-1, 0, false, 0}; }
+    LinePassInfo none() { return LinePassInfo{-1, false, {}}; }
 };
 
-template <typename T>
-struct TablesOp {
-    Cx<T>* out;
-    hipStream_t stream;
+struct OccupancyOp {
     template <typename I>
-    hipError_t run() {
-        hipLaunchKernelGGL((line_pass_tables_kernel<T, I::LNP, I::LEPT>), dim3((I::K::TW + 255) / 256), dim3(256), 0,
-                           stream, out);
-        return hipGetLastError();
+    int run() {
+        int blocks = 0;
+        if (I::prepare() != hipSuccess ||
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, I::fn(), I::K::NT, I::lds()) != hipSuccess)
+            return 0;
+        return blocks;
     }
-    hipError_t none() { return hipErrorInvalidValue; }
+    int none() { return 0; }
 };
 
 template <typename T>
@@ -145,8 +140,8 @@ LinePassInfo line_pass_info(LinePass kind, const LinePassSize& size) {
     return lp::with_line_pass<T>((int)kind, size, lp::InfoOp{});
 }
 template <typename T>
-hipError_t launch_line_pass_tables(LinePass kind, const LinePassSize& size, Cx<T>* tables, hipStream_t stream) {
-    return lp::with_line_pass<T>((int)kind, size, lp::TablesOp<T>{tables, stream});
+int line_pass_occupancy(LinePass kind, const LinePassSize& size) {
+    return lp::with_line_pass<T>((int)kind, size, lp::OccupancyOp{});
 }
 template <typename T>
 hipError_t launch_line_pass(LinePass kind, const LinePassSize& size, const Cx<T>* in, Cx<T>* out, const LinePassArgs& a,

@@ -25,19 +25,21 @@ struct zm_plan {
     unsigned flags;
     int device;
     Geo geo;
-    double2* tw64;  // exp(-2 pi i t / N), t < N
-    float2* tw32;
+    // the plan's tables, one allocation holding in its precision what its passes
+    // read: tw = exp(-2 pi i t / N), t < N; and those below
+    void* tables;
+    void* tw;
     bool two_stage;
     int lpb;  // lines per workgroup of the fused line kernel
     int rpb;  // rank rows per workgroup of the two-stage kernels
     void* own_scratch;
     size_t scratch_bytes;
-    // compile-time specialised line pass (line_fast.hip)
+    // compile-time specialised line pass (line_fast.hip): grids, 0 where the
+    // plan does not use it
     bool fast;
-    double2* ltab64;  // per-line twiddle tables (W_S, W_N two-level)
-    float2* ltab32;
+    void* ltab;  // per-line twiddle tables (W_S, W_N two-level)
     int fast_grid_fwd, fast_grid_inv;
-    int fast_grid_lapx;  // the fused Laplacian + x pass's grid (0: not built for this plan)
+    int fast_grid_lapx;  // the fused Laplacian + x pass
     // natural-order line passes (line_pass.hpp) by axis; grid 0: not used
     struct NatPass {
         zm::LinePass kind;
@@ -214,9 +216,14 @@ zm_plan::NatPass nat_pass(const zm_plan* p, int cus, zm::LinePass kind, int axis
         else np.size.small = false;
     }
     const int64_t groups = (int64_t)p->batch << (lines - info.lines_log2);
-    if (info.occupancy <= 0 || groups > INT32_MAX) return np;
-    const int64_t resident = (int64_t)info.occupancy * cus;
-    np.grid = (int)(info.loop && resident < groups ? resident : groups);
+    if (groups > INT32_MAX) return np;
+    int64_t grid = groups;
+    if (info.loop) {
+        const int64_t resident = (int64_t)zm::line_pass_occupancy<T>(kind, np.size) * cus;
+        if (resident < groups) grid = resident;
+    }
+    if (grid <= 0) return np;
+    np.grid = (int)grid;
     const bool rows = !(kind >= zm::LP_TILE_FWD && kind <= zm::LP_TILE_SPEC);
     np.tables = p->nat_tables[rows ? 0 : 1];
     zm::LinePassArgs& a = np.args;
@@ -238,31 +245,93 @@ zm_plan::NatPass nat_pass(const zm_plan* p, int cus, zm::LinePass kind, int axis
     return np;
 }
 
-// The twiddle tables and passes of a plan's natural-order line passes.
+// At N >= 4096 the specialised pass (line_fast.hip) is as fast as a row pass or
+// faster where it is built (forward + inverse: 4096^2 FP32 0.293 against 0.306
+// ms, eight fields 2.43 against 2.32; 8192^2 FP32 line 0.20 against 0.22-0.23
+// ms); elsewhere the generic one took 8192^2, P = 1, B = 32 4.54 against 1.46 ms.
+bool row_passes_lose(const Geo& g, bool fast) { return g.ln >= 12 && fast; }
+
+// The grids of the specialised line pass (line_fast.hip) in the directions that
+// a plan runs it in: the MFMA variant and N >= 4096 both, else only the forward
+// x pass beside the fused Laplacian.
 template <typename T>
-hipError_t choose_nat_passes(zm_plan* p, int cus) {
-    const int ln = p->geo.ln, d = p->geo.dims;
-    const zm::LinePass kinds[2] = {zm::LP_ROW_FWD, zm::LP_TILE_FWD};
-    for (int i = 0; i < 2; i++) {
-        const zm::LinePassSize size = nat_size(p->geo, sizeof(T) == 8);
-        const zm::LinePassInfo info = zm::line_pass_info<T>(kinds[i], size);
-        if (info.lines_log2 < 0) continue;
-        hipError_t e = hipMalloc(&p->nat_tables[i], sizeof(zm::Cx<T>) * (size_t)info.tables);
-        if (e == hipSuccess) e = zm::launch_line_pass_tables<T>(kinds[i], size, (zm::Cx<T>*)p->nat_tables[i], nullptr);
-        if (e != hipSuccess) return e;
+void choose_fast_passes(zm_plan* p, int cus, bool mfma) {
+    const Geo& g = p->geo;
+    if (!zm::fast_line_supported<T>(g.vec, g.m)) return;
+    const bool plain = zm::fast_line_plain<T>(g.vec, g.m, mfma);
+    const bool lapx = zm::fast_line_lapx<T>(g.vec, g.m, mfma, g.dims, g.b);
+    if (!plain && !lapx) return;
+    const int of = zm::fast_line_occupancy<T>(g.vec, g.m, true, mfma, false);
+    const int oi = plain ? zm::fast_line_occupancy<T>(g.vec, g.m, false, mfma, false) : 0;
+    const int ol = lapx ? zm::fast_line_occupancy<T>(g.vec, g.m, true, mfma, true) : 0;
+    if (of <= 0 || (plain && oi <= 0)) return;
+    p->fast_grid_fwd = of * cus;
+    p->fast_grid_inv = oi * cus;
+    p->fast_grid_lapx = ol * cus;
+    if (g.dims == 3 && ol > 0) {
+        // 3D: row tiles times plane chunks, about the resident workgroups, the
+        // chunks at least two planes long
+        const int ntile = g.n >> zm::fast_line_lapx_lines_log2(g.vec, g.m);
+        int nzc = 1;
+        while (2 * nzc * ntile <= ol * cus && 2 * nzc <= g.n / 2) nzc *= 2;
+        p->fast_grid_lapx = ntile * nzc;
     }
+}
+
+// Allocates and fills the tables that the plan's passes read: one allocation and
+// one launch, in the plan's precision.  A 1024^2 FP64 plan on a caller's scratch
+// takes 19 us to create; with an allocation and a launch for each table, those of
+// passes it does not run, and every pass's occupancy queried it took 31.
+template <typename T>
+hipError_t make_tables(zm_plan* p, bool mfma) {
+    const Geo& g = p->geo;
+    const bool nat = !p->two_stage && !mfma, fast = p->fast_grid_fwd > 0;
+    const zm::LinePassSize size = nat_size(g, sizeof(T) == 8);
+    const zm::LinePassInfo none{-1, false, {}};
+    const zm::LinePassInfo row = nat ? zm::line_pass_info<T>(zm::LP_ROW_FWD, size) : none;
+    const zm::LinePassInfo tile = nat ? zm::line_pass_info<T>(zm::LP_TILE_FWD, size) : none;
+    const zm::LinePassInfo solve = nat ? zm::line_pass_info<T>(zm::LP_ROW_SPEC, size) : none;
+    const bool rows = row.lines_log2 >= 0 && (!row_passes_lose(g, fast) || solve.lines_log2 >= 0);
+    const bool tiles = tile.lines_log2 >= 0;
+    zm::PlanTables<T> t{};
+    t.n = g.n;
+    t.line_entries = fast ? zm::line_table_entries(g.vec, g.m) : 0;
+    t.line_s = g.vec > g.m ? g.vec : g.m;
+    t.radices[0] = row.radices;
+    t.radices[1] = tile.radices;
+    size_t bytes = 0;
+    auto place = [&](size_t need) {
+        const size_t at = bytes;
+        bytes += (need + 255) & ~(size_t)255;
+        return at;
+    };
+    const size_t es = sizeof(zm::Cx<T>);
+    const size_t tw = place(es * (size_t)g.n), line = place(es * (size_t)t.line_entries);
+    const size_t nat0 = place(rows ? es * (size_t)row.radices.entries : 0);
+    const size_t nat1 = place(tiles ? es * (size_t)tile.radices.entries : 0);
+    const size_t half = place(rows || tiles ? sizeof(double) * (size_t)g.n : 0);
+    const hipError_t e = hipMalloc(&p->tables, bytes);
+    if (e != hipSuccess) return e;
+    char* const base = (char*)p->tables;
+    p->tw = t.tw = (zm::Cx<T>*)(base + tw);
+    if (fast) p->ltab = t.line = (zm::Cx<T>*)(base + line);
+    if (rows) p->nat_tables[0] = t.nat[0] = (zm::Cx<T>*)(base + nat0);
+    if (tiles) p->nat_tables[1] = t.nat[1] = (zm::Cx<T>*)(base + nat1);
+    if (rows || tiles) p->half_sin = t.half_sin = (double*)(base + half);
+    return zm::launch_plan_tables<T>(t, nullptr);
+}
+
+// The natural-order line passes of a plan.
+template <typename T>
+void choose_nat_passes(zm_plan* p, int cus) {
+    const int d = p->geo.dims;
     p->tiled = p->nat_tables[1] != nullptr;
     for (int axis = 1; axis < d && p->tiled; axis++) {
         p->nat_fwd[axis] = nat_pass<T>(p, cus, zm::LP_TILE_FWD, axis);
         p->nat_inv[axis] = nat_pass<T>(p, cus, zm::LP_TILE_INV, axis);
         if (!p->nat_fwd[axis].grid || !p->nat_inv[axis].grid) p->tiled = false;
     }
-    // At N >= 4096 the specialised pass (line_fast.hip) is as fast or faster as
-    // a row pass where it is built (forward + inverse: 4096^2 FP32 0.293
-    // against 0.306 ms, eight fields 2.43 against 2.32; 8192^2 FP32 line 0.20
-    // against 0.22-0.23 ms); elsewhere the generic one took 8192^2, P = 1,
-    // B = 32 4.54 against 1.46 ms.
-    const bool rows = p->nat_tables[0] && !(ln >= 12 && p->fast);
+    const bool rows = p->nat_tables[0] && !row_passes_lose(p->geo, p->fast_grid_fwd > 0);
     for (int axis = 0; axis < d; axis++) {
         if (axis > 0 && p->tiled) break;
         p->nat_fwd[axis] = p->nat_inv[axis] = zm_plan::NatPass{};
@@ -278,9 +347,25 @@ hipError_t choose_nat_passes(zm_plan* p, int cus) {
     if (p->nat_fwd[0].grid && p->tiled)
         p->nat_lap = nat_pass<T>(p, cus, d == 2 ? zm::LP_ROW_LAP2 : zm::LP_ROW_LAP3, 0);
     p->nat_spec = nat_pass<T>(p, cus, p->tiled ? zm::LP_TILE_SPEC : zm::LP_ROW_SPEC, d - 1);
-    if (!p->nat_spec.grid) return hipSuccess;
-    const hipError_t e = hipMalloc(&p->half_sin, sizeof(double) * (size_t)p->geo.n);
-    return e == hipSuccess ? zm::launch_half_sin(p->half_sin, p->geo.n, nullptr) : e;
+}
+
+// The passes of a plan and their tables.
+template <typename T>
+hipError_t choose_passes(zm_plan* p, bool mfma) {
+    int cus = 0;
+    hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, p->device);
+    if (e != hipSuccess) return e;
+    if (!p->two_stage) choose_fast_passes<T>(p, cus, mfma);
+    e = make_tables<T>(p, mfma);
+    if (e != hipSuccess) return e;
+    if (!p->two_stage && !mfma) choose_nat_passes<T>(p, cus);
+    // the specialised (VEC, M) pairs, as long as every pass of the plan has a
+    // compile-time kernel
+    p->fast = !p->two_stage && zm::fast_line_supported<T>(p->geo.vec, p->geo.m);
+    for (int axis = 0; axis < p->geo.dims; axis++)
+        if (!(p->nat_fwd[axis].grid || p->fast_grid_fwd) || !(p->nat_inv[axis].grid || p->fast_grid_inv))
+            p->fast = false;
+    return hipSuccess;
 }
 
 }  // namespace
@@ -391,76 +476,13 @@ zm_status zm_plan_create(zm_plan** plan, const zm_shape* shape, zm_precision pre
         delete p;
         return ZM_ERR_NOMEM;
     }
-    if (hipMalloc(&p->tw64, sizeof(double2) * n) != hipSuccess) {
-        if (p->own_scratch) (void)hipFree(p->own_scratch);
-        delete p;
-        return ZM_ERR_NOMEM;
-    }
-    if (hipMalloc(&p->tw32, sizeof(float2) * n) != hipSuccess) {
-        (void)hipFree(p->tw64);
-        if (p->own_scratch) (void)hipFree(p->own_scratch);
-        delete p;
-        return ZM_ERR_NOMEM;
-    }
-    hipError_t e = zm::launch_twiddles(p->tw64, p->tw32, n, nullptr);
-    // the specialised line pass, when the (VEC, M) pair has one and its LDS fits
-    const bool fp64 = precision == ZM_FP64;
-    if (e == hipSuccess && !two_stage &&
-        (fp64 ? zm::fast_line_supported<double>(d.vec, d.m) : zm::fast_line_supported<float>(d.vec, d.m))) {
-        const int nt = zm::line_table_entries(d.vec, d.m);
-        if (hipMalloc(&p->ltab64, sizeof(double2) * nt) == hipSuccess &&
-            hipMalloc(&p->ltab32, sizeof(float2) * nt) == hipSuccess) {
-            e = zm::launch_line_tables(p->ltab64, p->ltab32, d.vec, d.m, nullptr);
-            int cus = 0;
-            if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
-            const int of = fp64 ? zm::fast_line_occupancy<double>(d.vec, d.m, true, false, false)
-                                : zm::fast_line_occupancy<float>(d.vec, d.m, true, mfma, false);
-            const int oi = fp64 ? zm::fast_line_occupancy<double>(d.vec, d.m, false, false, false)
-                                : zm::fast_line_occupancy<float>(d.vec, d.m, false, mfma, false);
-            // the fused Laplacian + x pass (FP32 vector ALU)
-            const bool lx = fp64 ? zm::fast_line_lapx<double>(d.vec, d.m, false, shape->dims, shape->b)
-                                 : zm::fast_line_lapx<float>(d.vec, d.m, mfma, shape->dims, shape->b);
-            const int ol = !lx ? 0 : fp64 ? zm::fast_line_occupancy<double>(d.vec, d.m, true, false, true)
-                                          : zm::fast_line_occupancy<float>(d.vec, d.m, true, mfma, true);
-            // a direction that is not built runs line_pass.hpp's passes (grid 0)
-            const bool bf = fp64 ? zm::fast_line_built<double>(d.vec, d.m, true, false)
-                                 : zm::fast_line_built<float>(d.vec, d.m, true, mfma);
-            const bool bi = fp64 ? zm::fast_line_built<double>(d.vec, d.m, false, false)
-                                 : zm::fast_line_built<float>(d.vec, d.m, false, mfma);
-            if (e == hipSuccess && (of > 0 || !bf) && (oi > 0 || !bi)) {
-                p->fast = true;
-                p->fast_grid_fwd = of * cus;
-                p->fast_grid_inv = oi * cus;
-                p->fast_grid_lapx = ol * cus;
-                if (shape->dims == 3 && ol > 0) {
-                    // 3D: row tiles times plane chunks, about the resident
-                    // workgroups, the chunks at least two planes long
-                    const int ntile = n >> zm::fast_line_lapx_lines_log2(d.vec, d.m);
-                    int nzc = 1;
-                    while (2 * nzc * ntile <= ol * cus && 2 * nzc <= n / 2) nzc *= 2;
-                    p->fast_grid_lapx = ntile * nzc;
-                }
-            }
-        }
-    }
-    // the natural-order line passes (FP64 and FP32 vector ALU)
-    if (e == hipSuccess && !two_stage && !mfma) {
-        int cus = 0;
-        e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
-        if (e == hipSuccess) e = fp64 ? choose_nat_passes<double>(p, cus) : choose_nat_passes<float>(p, cus);
-    }
+    hipError_t e = precision == ZM_FP64 ? choose_passes<double>(p, false) : choose_passes<float>(p, mfma);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess || (mfma && !p->fast)) {
-        if (p->half_sin) (void)hipFree(p->half_sin);
-        for (void* t : p->nat_tables)
-            if (t) (void)hipFree(t);
-        (void)hipFree(p->tw64);
-        (void)hipFree(p->tw32);
-        if (p->ltab64) (void)hipFree(p->ltab64);
-        if (p->ltab32) (void)hipFree(p->ltab32);
+        if (p->tables) (void)hipFree(p->tables);
         if (p->own_scratch) (void)hipFree(p->own_scratch);
         delete p;
-        return e != hipSuccess ? ZM_ERR_DEVICE : ZM_ERR_UNSUPPORTED;
+        return e == hipErrorOutOfMemory ? ZM_ERR_NOMEM : e != hipSuccess ? ZM_ERR_DEVICE : ZM_ERR_UNSUPPORTED;
     }
     *plan = p;
     return ZM_OK;
@@ -469,13 +491,7 @@ zm_status zm_plan_create(zm_plan** plan, const zm_shape* shape, zm_precision pre
 zm_status zm_plan_destroy(zm_plan* p) {
     if (!p) return ZM_ERR_INVALID_ARG;
     zm_status st = ZM_OK;
-    if (p->tw64 && hipFree(p->tw64) != hipSuccess) st = ZM_ERR_DEVICE;
-    if (p->tw32 && hipFree(p->tw32) != hipSuccess) st = ZM_ERR_DEVICE;
-    if (p->ltab64 && hipFree(p->ltab64) != hipSuccess) st = ZM_ERR_DEVICE;
-    if (p->ltab32 && hipFree(p->ltab32) != hipSuccess) st = ZM_ERR_DEVICE;
-    if (p->half_sin && hipFree(p->half_sin) != hipSuccess) st = ZM_ERR_DEVICE;
-    for (void* t : p->nat_tables)
-        if (t && hipFree(t) != hipSuccess) st = ZM_ERR_DEVICE;
+    if (p->tables && hipFree(p->tables) != hipSuccess) st = ZM_ERR_DEVICE;
     if (p->own_scratch && hipFree(p->own_scratch) != hipSuccess) st = ZM_ERR_DEVICE;
     drop_timing(p);
     delete p;
@@ -548,7 +564,7 @@ struct Exec {
     bool record = true;  // per-launch timing events when the plan records them
 
     const zm::Cx<T>* line_tables() const {
-        return p->precision == ZM_FP64 ? (const zm::Cx<T>*)p->ltab64 : (const zm::Cx<T>*)p->ltab32;
+        return (const zm::Cx<T>*)p->ltab;
     }
     // natural-order line pass of one axis; a tile pass holds a repack stage,
     // counted inside it
@@ -580,7 +596,7 @@ struct Exec {
         if (compute && !lapx && np.grid) return nat(np, in, out, scale);
         zm::LineArgs a{axis_stride(p, axis), (int)(p->dims.local / p->dims.l), p->lpb};
         const int grid = lapx ? p->fast_grid_lapx : fwd ? p->fast_grid_fwd : p->fast_grid_inv;
-        if (p->fast && compute && grid) {
+        if (compute && grid) {
             return launch_status(timed_launch(p, lapx ? ZM_STAGE_LINE_LAPLACE : ZM_STAGE_LINE, st, [&] {
                 return zm::launch_line_fast<T>((const zm::Cx<T>*)in, (zm::Cx<T>*)out, p->geo, a, line_tables(),
                                                p->batch, fwd, scale, grid, p->precision == ZM_FP32_MFMA, lapx, st);
@@ -781,10 +797,10 @@ zm_status run_transform(zm_plan* p, const void* in, void* out, void* scratch, vo
     if (s == in || s == out) return ZM_ERR_ALIAS;
     hipStream_t st = (hipStream_t)stream;
     if (p->precision == ZM_FP64) {
-        Exec<double> ex{p, st, compute, (const double2*)p->tw64, record};
+        Exec<double> ex{p, st, compute, (const double2*)p->tw, record};
         return fwd ? ex.forward(in, out, s) : ex.inverse(in, out, s, scale);
     }
-    Exec<float> ex{p, st, compute, (const float2*)p->tw32, record};
+    Exec<float> ex{p, st, compute, (const float2*)p->tw, record};
     return fwd ? ex.forward(in, out, s) : ex.inverse(in, out, s, scale);
 }
 
@@ -813,10 +829,10 @@ zm_status zm_laplace_forward(zm_plan* p, const void* in, void* out, double scale
     if (s == in || s == out) return ZM_ERR_ALIAS;
     const hipStream_t st = (hipStream_t)stream;
     if (p->precision == ZM_FP64) {
-        Exec<double> ex{p, st, true, (const double2*)p->tw64};
+        Exec<double> ex{p, st, true, (const double2*)p->tw};
         return ex.laplace_forward(in, out, s, scale);
     }
-    Exec<float> ex{p, st, true, (const float2*)p->tw32};
+    Exec<float> ex{p, st, true, (const float2*)p->tw};
     return ex.laplace_forward(in, out, s, scale);
 }
 
@@ -935,8 +951,8 @@ static zm_status spectral(zm_plan* p, const void* in, void* out, zm_spectral kin
     zm::SpectralArgs sp;
     ZM_TRY(spectral_args(p, kind, p0, p1, length, conj, &sp));
     const hipStream_t st = (hipStream_t)stream;
-    if (p->precision == ZM_FP64) return Exec<double>{p, st, true, (const double2*)p->tw64}.multiply(in, out, sp);
-    return Exec<float>{p, st, true, (const float2*)p->tw32}.multiply(in, out, sp);
+    if (p->precision == ZM_FP64) return Exec<double>{p, st, true, (const double2*)p->tw}.multiply(in, out, sp);
+    return Exec<float>{p, st, true, (const float2*)p->tw}.multiply(in, out, sp);
 }
 
 static zm_status spectral_solve(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
@@ -950,8 +966,8 @@ static zm_status spectral_solve(zm_plan* p, const void* in, void* out, zm_spectr
     ZM_TRY(scratch_for(p, scratch, &s));
     if (s == in || s == out) return ZM_ERR_ALIAS;
     const hipStream_t st = (hipStream_t)stream;
-    if (p->precision == ZM_FP64) return Exec<double>{p, st, true, (const double2*)p->tw64}.solve(in, out, s, scale, sp);
-    return Exec<float>{p, st, true, (const float2*)p->tw32}.solve(in, out, s, scale, sp);
+    if (p->precision == ZM_FP64) return Exec<double>{p, st, true, (const double2*)p->tw}.solve(in, out, s, scale, sp);
+    return Exec<float>{p, st, true, (const float2*)p->tw}.solve(in, out, s, scale, sp);
 }
 
 zm_status zm_spectral_multiply(zm_plan* p, const void* in, void* out, zm_spectral kind, double p0, double p1,
