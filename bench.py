@@ -540,7 +540,7 @@ def main():
     achieved = per_launch / (dom_avg * 1e-3) / 1e9
     traffic = load_traffic(f"traffic_{dom_name}_n{n}_p{p}_b{b}_{args.precision}.json")
     kernel = KERNELS.get(dom_name, dom_name)
-    if dom_name == "line" and 16 <= n <= 2048 and args.precision != "fp32_mfma" and not args.two_stage:
+    if dom_name == "line" and plan.tiled:
         kernel = "line_pass_kernel (one whole line's FFT, pack, exchange, twiddle and repack in a pass)"
     elif dom_name == "line" and not plan.fast:
         kernel = "line_kernel (fused FFT1a + exchange + twiddle + FFT1b direction pass)"

@@ -108,8 +108,11 @@ zm_status zm_plan_dims(const zm_plan* plan, zm_shape* shape, zm_dims* dims, zm_p
 /* The kernel path a plan runs (no reference counterpart): a bitwise OR of
  * the flags below. */
 #define ZM_PATH_TWO_STAGE 1u   /* two kernels per direction (post-exchange buffer materialised) */
-#define ZM_PATH_FAST_LINE 2u   /* compile-time specialised fused line pass */
+#define ZM_PATH_FAST_LINE 2u   /* VEC and M in 16 .. 128, and every line pass a compile-time kernel */
 #define ZM_PATH_MFMA 4u        /* radix-16 stages as split-precision MFMA GEMMs */
+#define ZM_PATH_TILES 8u       /* line passes over tiles: the transforms launch no repacks */
+#define ZM_PATH_LAPLACE 16u    /* zm_laplace_forward forms the Laplacian in the x pass */
+#define ZM_PATH_SOLVE 32u      /* zm_spectral_solve runs the last axis and the multiplier as one kernel */
 zm_status zm_plan_path(const zm_plan* plan, unsigned* path);
 
 /* Bytes of device scratch the transforms need (0 when none). */
@@ -250,7 +253,7 @@ zm_status zm_spectral_multiply_adjoint(zm_plan* plan, const void* in, void* out,
  * solve on real-space fields (Poisson, heat, ..), and its adjoint, the same
  * with the conjugate multiplier (the forward and inverse adjoints cancel).
  * The last axis's two passes and the multiplier run as one kernel where the
- * plan has it (N <= 2048, 2D N = 4096, 2D FP32 N = 8192; FP64 and FP32 vector
+ * plan has it (16 <= N <= 2048, 2D N = 4096, 2D FP32 N = 8192; FP64 and FP32 vector
  * ALU), else as the three calls; the values agree with them to rounding.
  * `factor`, when not NULL, is a device address holding an FP64 value that
  * multiplies the multiplier (a loss's incoming gradient, say).

@@ -510,7 +510,8 @@ zm_status zm_plan_dims(const zm_plan* p, zm_shape* shape, zm_dims* dims, zm_prec
 zm_status zm_plan_path(const zm_plan* p, unsigned* path) {
     if (!p || !path) return ZM_ERR_INVALID_ARG;
     *path = (p->two_stage ? ZM_PATH_TWO_STAGE : 0u) | (p->fast ? ZM_PATH_FAST_LINE : 0u) |
-            (p->precision == ZM_FP32_MFMA ? ZM_PATH_MFMA : 0u);
+            (p->precision == ZM_FP32_MFMA ? ZM_PATH_MFMA : 0u) | (p->tiled ? ZM_PATH_TILES : 0u) |
+            (p->fast_grid_lapx || p->nat_lap.grid ? ZM_PATH_LAPLACE : 0u) | (p->nat_spec.grid ? ZM_PATH_SOLVE : 0u);
     return ZM_OK;
 }
 

@@ -134,6 +134,9 @@ class Plan:
         self.two_stage = bool(path.value & L.ZM_PATH_TWO_STAGE)
         self.fast = bool(path.value & L.ZM_PATH_FAST_LINE)
         self.mfma = bool(path.value & L.ZM_PATH_MFMA)
+        self.tiled = bool(path.value & L.ZM_PATH_TILES)
+        self.fused_laplace = bool(path.value & L.ZM_PATH_LAPLACE)
+        self.fused_solve = bool(path.value & L.ZM_PATH_SOLVE)
 
     # ---- lifetime ----
     def close(self):
@@ -395,7 +398,8 @@ class Plan:
         L.check(L._lib().zm_timing_enable(self._h, 1 if enable else 0), "zm_timing_enable")
 
     def timing_read(self) -> dict:
-        """{stage name: (launch count, total ms)} for every stage with launches."""
+        """{stage name: (count, total ms)} for every stage that ran; one that ran
+        inside another's launch counts with no time of its own."""
         out = {}
         for k, name in enumerate(L.STAGES):
             c = ctypes.c_int()
