@@ -40,26 +40,33 @@ enum Dir { FWD = 0, INV = 1, SPEC = 2 };
 // leave a CU one workgroup (LOOP); the same with the twiddles in LDS (LOOP_LDS).
 enum Mode { ONCE = 0, LOOP = 1, LOOP_LDS = 2 };
 
-// Lines of N = 2^LN points, LP = 2^LLP of them per workgroup, 2^LEPT elements
-// per thread.
-template <typename T, int LN, int LLP, int LEPT>
-struct Line {
-    using C = Cx<T>;
-    static constexpr int N = 1 << LN, LP = 1 << LLP, E = N * LP, EPT = 1 << LEPT, NT = E >> LEPT;
-    static constexpr int LR = LEPT < 4 ? LEPT : 4;  // largest radix 16
+// The radix passes of a line of 2^LN points with 2^LEPT elements per thread: of
+// at most 16 points, as even as possible, the larger ones first.
+template <int LN, int LEPT>
+struct Radices {
+    static constexpr int LR = LEPT < 4 ? LEPT : 4;
     static constexpr int NP = (LN + LR - 1) / LR;
-    static_assert(NP >= 2 && NT >= 64 && NT <= 1024, "split");
-    // radices: as even as possible, the larger ones first
     static constexpr int lr(int p) { return LN / NP + (p < LN % NP ? 1 : 0); }
     static constexpr int lns(int p) { return p == 0 ? 0 : lns(p - 1) + lr(p - 1); }
     // twiddles of pass p >= 1: W_{NS R}^(jm r) at r NS + jm
     static constexpr int tw_off(int p) { return p <= 1 ? 0 : tw_off(p - 1) + (1 << (lns(p - 1) + lr(p - 1))); }
     static constexpr int TW = tw_off(NP);
-    static constexpr LineRadices radices() {
+    static constexpr LineRadices list() {
         LineRadices r{NP, TW, {}};
         for (int p = 0; p < NP; p++) r.lr[p] = lr(p);
         return r;
     }
+};
+
+// Lines of N = 2^LN points, LP = 2^LLP of them per workgroup, 2^LEPT elements
+// per thread.
+template <typename T, int LN, int LLP, int LEPT>
+struct Line : Radices<LN, LEPT> {
+    using C = Cx<T>;
+    using Base = Radices<LN, LEPT>;
+    using Base::lns, Base::lr, Base::NP, Base::TW, Base::tw_off;
+    static constexpr int N = 1 << LN, LP = 1 << LLP, E = N * LP, EPT = 1 << LEPT, NT = E >> LEPT;
+    static_assert(NP >= 2 && NT >= 64 && NT <= 1024, "split");
 
     // LDS index of element n of line l.  One padding element after every
     // 2^PS, 2^(2 PS), ..: the lanes of an LDS phase (16 of 8 bytes, 8 of 16)

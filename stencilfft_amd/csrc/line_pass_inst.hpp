@@ -33,13 +33,21 @@ constexpr bool is_row(int kind) {
     return kind == LP_ROW_FWD || kind == LP_ROW_INV || kind == LP_ROW_SPEC || is_lap(kind);
 }
 
+// the same radix passes, and so the same twiddle table
+constexpr bool same_radices(const LineRadices& a, const LineRadices& b) {
+    if (a.np != b.np || a.entries != b.entries) return false;
+    for (int p = 0; p < a.np; p++)
+        if (a.lr[p] != b.lr[p]) return false;
+    return true;
+}
+
 template <typename T, int LN, bool R16, int KIND, bool SMALL>
 struct Inst {
     using S = Split<T, LN, R16>;
     static constexpr bool ROWS = is_row(KIND);
     static constexpr int LNP = LN, LLP = ROWS ? (SMALL ? S::row_small : S::row) : (SMALL ? S::tile_small : S::tile);
-    // multiplier tiles with at most 512 threads (256 VGPRs; the radices, and so
-    // the tables, are the same)
+    // multiplier tiles with at most 512 threads (256 VGPRs), on the tile passes'
+    // tables
     static constexpr int LEPT0 = ROWS ? S::row_ept : S::tile_ept;
     static constexpr int LEPT = KIND == LP_TILE_SPEC && LN + LLP - LEPT0 > 9 ? LN + LLP - 9 : LEPT0;
     // row multipliers only where no tile is built (FP64 N = 8192 spills)
@@ -61,6 +69,7 @@ struct Inst {
                                : KIND == LP_ROW_FWD || KIND == LP_TILE_FWD || is_lap(KIND) ? ROW
                                                                            : TILE;
     using K = Line<T, LN, LLP < 0 ? 4 : LLP, LEPT>;
+    static_assert(!built || same_radices(Radices<LN, LEPT>::list(), Radices<LN, LEPT0>::list()), "the table of the row or tile passes");
     static constexpr size_t lds() {
         static_assert(K::lds_bytes(MODE == LOOP_LDS) <= kLdsLimit, "LDS");
         return K::lds_bytes(MODE == LOOP_LDS);
@@ -95,7 +104,7 @@ auto with_line_pass(int kind, const LinePassSize& size, Op&& op) {
 struct InfoOp {
     template <typename I>
     LinePassInfo run() {
-        return LinePassInfo{I::LLP, I::MODE != ONCE, I::K::radices()};
+        return LinePassInfo{I::LLP, I::MODE != ONCE, I::K::list()};
     }
     LinePassInfo none() { return LinePassInfo{-1, false, {}}; }
 };
