@@ -96,6 +96,9 @@ struct ConvertArgs {
     int ltile, lfield;
 };
 
+// log2 of the elements of a converter tile (spectral.hip)
+constexpr int kConvertTile = 10;
+
 inline ConvertArgs convert_args(const Geo& g, int le) {
     ConvertArgs a{};
     const int d = g.dims, lm = g.lb + g.lp, slab = d * g.ll;

@@ -354,7 +354,7 @@ __global__ void __launch_bounds__(256) convert_kernel(const Cx<T>* __restrict__ 
 template <typename T>
 hipError_t launch_natural_packed(const Cx<T>* in, Cx<T>* out, const Geo& g, int batch, bool to_packed,
                                  hipStream_t stream) {
-    constexpr int LE = 10;
+    constexpr int LE = kConvertTile;
     const ConvertArgs a = convert_args(g, LE);
     const dim3 grid((unsigned)(g.field >> a.ltile), (unsigned)batch);
     if (a.ltile == LE)
