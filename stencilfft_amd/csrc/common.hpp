@@ -99,6 +99,7 @@ __device__ __forceinline__ void st_nt(float4* p, float4 v) {
 // count is a multiple of 8.
 // ---------------------------------------------------------------------------
 constexpr unsigned kXcds = 8;
+constexpr int64_t kLastLevelCache = (int64_t)256 << 20;  // bytes, shared by the XCDs
 __device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned nb) {
     if (nb % kXcds) return b;
     return (b % kXcds) * (nb / kXcds) + b / kXcds;

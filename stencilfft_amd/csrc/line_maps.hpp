@@ -96,8 +96,9 @@ struct ConvertArgs {
     int ltile, lfield;
 };
 
-// log2 of the elements of a converter tile (spectral.hip)
-constexpr int kConvertTile = 10;
+// log2 of the elements of a converter tile (spectral.hip): 8 KB
+template <typename T>
+constexpr int kConvertTile = sizeof(T) == 8 ? 9 : 10;
 
 inline ConvertArgs convert_args(const Geo& g, int le) {
     ConvertArgs a{};

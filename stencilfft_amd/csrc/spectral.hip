@@ -288,15 +288,19 @@ hipError_t launch_index_table(int64_t* out, const Geo& g, bool reciprocal, hipSt
 // element had read or written every VEC-th element per lane.  Both sides are
 // permutations of the bits of one element index q, whose low `ltile` bits are
 // the element of the tile: r, jj, rows.
-// Memory-bound: tiles of 1024 elements (four per thread, as fast as 2048 or
-// 4096 and faster on small fields), plain loads (non-temporal ones missed
-// fields that the last-level cache still held: 2048^2 FP32 11.3 against 14.5
-// us) and non-temporal stores (4096^2 FP64 78 against 102 us).  to / from
-// packed against one thread per element: 4096^2 FP64 127 / 145 -> 78 / 78 us,
-// 8192^2 FP32 387 / 579 -> 189 / 185 (5.7 TB/s), 512^3 FP32 594 / 575 -> 391 /
-// 368, 1024^2 FP32 7.0 -> 5.0.
-// FULL: the field holds at least one tile (no guards).
-template <typename T, int LE, bool FULL>
+// Memory-bound: tiles of 8 KB (two FP64 or four FP32 elements per thread; half of
+// it in FP32 took 128 MB fields from 34 to 43 us, twice of it in FP64 512 MB from
+// 175 to 185), in FP64 consecutive tiles on one XCD (768 MB 261 -> 250 us; not in
+// FP32, 128 MB 43 -> 45), non-temporal stores (256 MB FP64 93 -> 62 us).
+// Loads: plain while the last-level cache can still hold the field (256 MB FP64
+// 62 us, non-temporal 85), non-temporal beyond (512 MB FP64 181 -> 169, FP32 179
+// -> 169, 384 MB FP32 135 -> 129).  Geometric means over the distributions, to /
+// from packed, against one thread per element: FP32 128 MB 65 / 67 -> 34 / 35
+// us, 1 GB 661 / 803 -> 344 / 333; FP64 128 MB 39 / 41 -> 32 / 32, 512 MB 224 /
+// 262 -> 169 / 171 (6.3 TB/s), where the best of the former, whose runs were long
+// enough, took 167.
+// FULL: the field holds at least one tile (no guards).  NTL: non-temporal loads.
+template <typename T, int LE, bool FULL, bool NTL>
 __global__ void __launch_bounds__(256) convert_kernel(const Cx<T>* __restrict__ in, Cx<T>* __restrict__ out,
                                                       ConvertArgs a, int to_packed) {
     using C = Cx<T>;
@@ -305,7 +309,7 @@ __global__ void __launch_bounds__(256) convert_kernel(const Cx<T>* __restrict__ 
     const int tid = threadIdx.x;
     auto pad = [](int i) { return i + (i >> 4) + (i >> 8); };  // distinct banks at every power-of-two stride
     const int64_t f = (int64_t)blockIdx.y << a.lfield;
-    const int base = (int)blockIdx.x << a.ltile;
+    const int base = (int)(sizeof(T) == 8 ? xcd_block(blockIdx.x, gridDim.x) : blockIdx.x) << a.ltile;
     // every address is a part of this tile, of this thread and of register k,
     // the last the sum of its bits' offsets
     const int slot = bits(a.order, tid);
@@ -326,11 +330,15 @@ __global__ void __launch_bounds__(256) convert_kernel(const Cx<T>* __restrict__ 
         for (int i = 0; i < NB; i++) o += (k >> i) & 1 ? bit[i] : 0;
         return o;
     };
+    auto ld = [](const C* p) -> C {
+        if constexpr (NTL) return ld_nt(p);
+        else return *p;
+    };
     const int n = FULL ? EPT : tid >= (1 << a.ltile) ? 0 : a.ltile > 8 ? 1 << (a.ltile - 8) : 1;
     C v[EPT];
     if (to_packed) {
 #pragma unroll
-        for (int k = 0; k < EPT; k++) v[k] = k < n ? nat_in[sum(nat_bit, k)] : C{0, 0};
+        for (int k = 0; k < EPT; k++) v[k] = k < n ? ld(nat_in + sum(nat_bit, k)) : C{0, 0};
 #pragma unroll
         for (int k = 0; k < EPT; k++)
             if (k < n) tile[pad(tid + 256 * k)] = v[k];
@@ -340,7 +348,7 @@ __global__ void __launch_bounds__(256) convert_kernel(const Cx<T>* __restrict__ 
             if (k < n) st_nt(pk_out + sum(pk_bit, k), tile[pad(sum(slot_bit, k) + slot)]);
     } else {
 #pragma unroll
-        for (int k = 0; k < EPT; k++) v[k] = k < n ? pk_in[sum(pk_bit, k)] : C{0, 0};
+        for (int k = 0; k < EPT; k++) v[k] = k < n ? ld(pk_in + sum(pk_bit, k)) : C{0, 0};
 #pragma unroll
         for (int k = 0; k < EPT; k++)
             if (k < n) tile[pad(sum(slot_bit, k) + slot)] = v[k];
@@ -354,13 +362,16 @@ __global__ void __launch_bounds__(256) convert_kernel(const Cx<T>* __restrict__ 
 template <typename T>
 hipError_t launch_natural_packed(const Cx<T>* in, Cx<T>* out, const Geo& g, int batch, bool to_packed,
                                  hipStream_t stream) {
-    constexpr int LE = kConvertTile;
+    constexpr int LE = kConvertTile<T>;
     const ConvertArgs a = convert_args(g, LE);
     const dim3 grid((unsigned)(g.field >> a.ltile), (unsigned)batch);
-    if (a.ltile == LE)
-        hipLaunchKernelGGL((convert_kernel<T, LE, true>), grid, dim3(256), 0, stream, in, out, a, to_packed ? 1 : 0);
+    const int tp = to_packed ? 1 : 0;
+    if (a.ltile < LE)
+        hipLaunchKernelGGL((convert_kernel<T, LE, false, false>), grid, dim3(256), 0, stream, in, out, a, tp);
+    else if ((int64_t)batch * g.field * (int64_t)sizeof(Cx<T>) <= kLastLevelCache)
+        hipLaunchKernelGGL((convert_kernel<T, LE, true, false>), grid, dim3(256), 0, stream, in, out, a, tp);
     else
-        hipLaunchKernelGGL((convert_kernel<T, LE, false>), grid, dim3(256), 0, stream, in, out, a, to_packed ? 1 : 0);
+        hipLaunchKernelGGL((convert_kernel<T, LE, true, true>), grid, dim3(256), 0, stream, in, out, a, tp);
     return hipGetLastError();
 }
 

@@ -48,22 +48,24 @@ static bool check(int d, int n, int p, int b) {
     // converters: every element, each tile a permutation of its slots, and the
     // element in slot order where the tile's own bits say (kernel: bits(order,
     // slot), then the packed map of it)
-    const ConvertArgs a = convert_args(g, kConvertTile);
-    std::vector<char> seen(g.field);
-    for (int q = 0; q < g.field; q++) {
-        const int nat = at(a.nat, q);
-        if (nat < 0 || nat >= g.field || seen[nat]++) return fail("natural side", g);
-        if (real_index(g, ms, nat / n / n, nat / n % n, nat % n) != at(a.pk, q)) return fail("packed side", g);
-    }
-    const int tile = 1 << a.ltile;
-    if (a.ltile != (kConvertTile < a.lfield ? kConvertTile : a.lfield)) return fail("tile size", g);
-    for (int base = 0; base < g.field; base += tile) {
-        std::vector<char> slot(tile);
-        for (int e = 0; e < tile; e++) {
-            const int s = at(a.order, e);
-            if (s < 0 || s >= tile || slot[s]++) return fail("tile order", g);
-            if (at(a.pk, base) + at(a.pk, s) != at(a.pk, base + s)) return fail("tile base", g);
-            if (at(a.nat, base) + at(a.nat, e) != at(a.nat, base + e)) return fail("tile base", g);
+    for (int le : {kConvertTile<float>, kConvertTile<double>}) {
+        const ConvertArgs a = convert_args(g, le);
+        std::vector<char> seen(g.field);
+        for (int q = 0; q < g.field; q++) {
+            const int nat = at(a.nat, q);
+            if (nat < 0 || nat >= g.field || seen[nat]++) return fail("natural side", g);
+            if (real_index(g, ms, nat / n / n, nat / n % n, nat % n) != at(a.pk, q)) return fail("packed side", g);
+        }
+        const int tile = 1 << a.ltile;
+        if (a.ltile != (le < a.lfield ? le : a.lfield)) return fail("tile size", g);
+        for (int base = 0; base < g.field; base += tile) {
+            std::vector<char> slot(tile);
+            for (int e = 0; e < tile; e++) {
+                const int s = at(a.order, e);
+                if (s < 0 || s >= tile || slot[s]++) return fail("tile order", g);
+                if (at(a.pk, base) + at(a.pk, s) != at(a.pk, base + s)) return fail("tile base", g);
+                if (at(a.nat, base) + at(a.nat, e) != at(a.nat, base + e)) return fail("tile base", g);
+            }
         }
     }
 
