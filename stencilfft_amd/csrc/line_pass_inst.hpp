@@ -13,7 +13,7 @@ constexpr size_t kLdsLimit = 160 * 1024;
 // Row and tile passes of 2^LN-point lines: log2 of the elements per thread and
 // of the lines per workgroup (and of the lines in the small variant), mode;
 // -1 lines: not built.  RADIX16: the alternative split of a plan that prefers
-// the largest radices (line_pass_radix16).
+// the largest radices (LinePassSize::radix16).
 template <typename T, int LN, bool RADIX16>
 struct Split {
     static constexpr int row_ept = 4, row = -1, row_small = -1, tile_ept = 4, tile = -1, tile_small = -1;

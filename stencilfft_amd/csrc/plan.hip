@@ -189,12 +189,18 @@ constexpr int kStageTarget = 4096;
 constexpr size_t kMaxLds = 160 * 1024;
 static_assert(ZM_NORM_PARTIALS == zm::kNormBlocks, "partial sums of zm_residual_norm");
 
-// FP64 lines of 256 points run as 16 x 16 on at most two ranks per axis and as
-// 8 x 8 x 4 on more.  16 x 16 rounds once less: the FP64 rounding noise of a
-// 32-step 256^3 rollout is 6.1e-7 against 1.0e-6 of its gradient, at equal
-// speed (four 256^3 fields, P = 2: forward 1.135 against 1.131 ms, inverse
-// 1.149 against 1.081).  But its last pass stores runs of 16 / P values: P = 4
+// FP64 lines of 256 points run as 16 x 16 on at most two ranks per axis, the
+// radices of the VEC = M = 16 pass that these plans ran before, and as 8 x 8 x 4
+// on more, where 16 x 16 stores runs of 16 / P values in its last pass: P = 4
 // 0.357 against 0.300 ms, P = 8 0.820 against 0.290.
+// On P <= 2 the choice keeps the rounding that the gradient check of the 256^3
+// rollout was set for: the noise of its central difference (two losses' rounding
+// over 2 eps) is 6.1e-7 with 16 x 16 and 1.00e-6, its bar, with 8 x 8 x 4.  It is
+// neither closer nor faster.  Against long double, rel L2 of a 256^3 forward
+// transform 3.4e-16 (8 x 8 x 4: 3.2e-16), of 32 heat steps 9.4e-15 (7.5e-15); one
+// field at P = 2 forward 293 us (291), inverse 302 (281), heat step 629 (611), and
+// Laplacian + forward 391 (325), as 16 values per thread leave no registers for
+// the fused 3D Laplacian.
 zm::LinePassSize nat_size(const Geo& g, bool fp64) {
     return zm::LinePassSize{g.ln, false, fp64 && g.ln == 8 && g.p <= 2};
 }

@@ -1,7 +1,10 @@
 // spectral_math.hpp -- the reciprocal-space multipliers, evaluated in FP64 for
-// every storage precision, shared by the standalone multiplier kernel
-// (spectral.hip) and the line passes that apply one between a forward and an
-// inverse transform (line_pass.hpp).
+// every storage precision, as the line passes apply them between a forward and
+// an inverse transform (line_pass.hpp): the parts that a line shares first, the
+// sines from a table.  The standalone multiplier kernel (spectral.hip) shares
+// signed_wavenumber only and evaluates its element's multiplier whole, sines by
+// sinpi; the two are compared for every kind in test_gpu_spectral_solve.py
+// (test_solve_is_the_three_calls).
 #pragma once
 
 #include "common.hpp"
