@@ -362,7 +362,10 @@ __global__ void __launch_bounds__(256) deriv4_march_kernel(const E* __restrict__
 // dx4 2048^2 FP32 26 -> 16; dz4 256^3 FP32 160 -> 57, real FP64 155 -> 57,
 // 64^3 31 -> 4.3.  With the limit at 1024 workgroups dz4 512^3 took 0.434
 // against 0.407 ms; with the z target for y, dy4 4096^2 67 against 55 us.
-constexpr int kMarchFill = 512, kMarchShort = 8;
+// FP64 y lines of 128 positions or more in 3D fill the CUs with one workgroup
+// each: 128^3 12.2 to 12.7 us in strips of 32, shortened 13.2 to 18 (eight fields
+// of 64^3, 256 workgroups too: 15 to 18 us, shortened 12.2 to 13.5).
+constexpr int kMarchFill = 512, kMarchFillWide = 256, kMarchShort = 8;
 template <int AXIS>
 constexpr int kMarchTarget = AXIS == 2 ? 2048 : 1024;
 
@@ -376,7 +379,8 @@ static hipError_t launch_march(const E* in, E* out, const Geo& g, int batch, int
     }
     int T = len < tmax ? len : tmax;
     const int64_t sets = ((int64_t)lines + 256 * K - 1) / (256 * K);
-    if (sets * (len / T) * batch < kMarchFill) {
+    const int fill = AXIS == 1 && sizeof(E) == 16 && g.dims == 3 && len >= 128 ? kMarchFillWide : kMarchFill;
+    if (sets * (len / T) * batch < fill) {
         if constexpr (K > 1)
             return launch_march<E, S, AXIS, 1, 16, 12, NTL>(in, out, g, batch, lines, len, tmax, denom, negate, stream,
                                                             order);
