@@ -820,10 +820,14 @@ static hipError_t laplace_zmarch_inst(const E* in, E* out, const Geo& g, int bat
     // re-read too much), L = 128 and 64 strips go on to 1024 workgroups (256^3,
     // P = 2, four FP32 fields 0.236 -> 0.211 ms, FP64 0.450 -> 0.420; 2048 took
     // P = 4 0.231 -> 0.236) and L = 32 strips to 4096 (128^3, P = 4, sixteen
-    // fields 0.137 -> 0.111)
+    // fields 0.137 -> 0.111).  Not 16-byte elements at L = 64 from N = 256 on,
+    // whose planes a strip's ends read again from memory: 256^3, P = 4 FP64, B =
+    // 16 / 4: one field 104 / 121 us at 512 workgroups, 117 / 117 at 1024, two
+    // 196 / 227 against 226 / 250 (sixteen of 128^3, P = 2: 213 against 209)
     int tz = g.n < 128 ? g.n : 128;
     while (tz > 4 && (int64_t)ntiles * g.p * (g.n / tz) * batch < 512) tz >>= 1;
-    constexpr int fill = KE == 1 ? 4096 : KE * NTH < 2048 ? 1024 : 512;
+    const bool few = KE == 2 && sizeof(E) == 16 && g.n >= 256;
+    const int fill = KE == 1 ? 4096 : KE * NTH < 2048 && !few ? 1024 : 512;
     while (tz > 32 && (int64_t)ntiles * g.p * (g.n / tz) * batch < fill) tz >>= 1;
     const unsigned blocks = (unsigned)((int64_t)ntiles * g.p * (g.n / tz));
     const size_t lds = sizeof(E) * (size_t)(R + 2) * (size_t)(g.l + 2 * g.vec);

@@ -15,13 +15,16 @@ def _fields(pl, seed):
     return torch.view_as_complex(torch.rand((pl.numel(), 2), generator=g, device="cuda", dtype=torch.float64) * 2 - 1)
 
 
-# workgroups of a field: y lines of 64 in 32, of 128 in 256
+# workgroups of a field: y lines of 64 in 32, of 128 in 256; depth tiles of L = 64
+# in 16 (N = 64), 64 (N = 128) and 128 (N = 256) per strip
 @pytest.mark.parametrize("n,p,b,batch", [(64, 2, 4, 16), (64, 1, 8, 5), (128, 4, 2, 2), (128, 2, 4, 8), (256, 4, 16, 3)])
 def test_fp64_strips_leave_every_value(n, p, b, batch):
     from stencilfft_amd import Plan
     print(f"[gpu] FP64 strips N={n} P={p} B={b} batch {batch}", flush=True)
     sys.stdout.flush()
     one, pl = (Plan(3, n, p, b, precision="fp64", batch=k, caller_scratch=True) for k in (1, batch))
-    x = _fields(pl, n)
-    want = torch.cat([one.dy4(u, 0.5) for u in x.chunk(batch)])
-    assert torch.equal(pl.dy4(x, 0.5), want)
+    x, acc = _fields(pl, n), _fields(pl, n + 1)
+    for fn in (lambda q, u, a: q.dy4(u, 0.5), lambda q, u, a: q.laplace(u, 1.5),
+               lambda q, u, a: q.laplace_add(u, a.clone(), 1.5, 0.25)):
+        want = torch.cat([fn(one, u, a) for u, a in zip(x.chunk(batch), acc.chunk(batch))])
+        assert torch.equal(fn(pl, x, acc), want)
