@@ -1,5 +1,7 @@
 // spectral.hip -- the plans' tables, reciprocal-space multipliers, the
 // device forms of the index maps and the natural <-> packed converters.
+#include <type_traits>
+
 #include "common.hpp"
 #include "kernels.hpp"
 #include "line_maps.hpp"
@@ -291,7 +293,10 @@ hipError_t launch_index_table(int64_t* out, const Geo& g, bool reciprocal, hipSt
 // Memory-bound: tiles of 8 KB (two FP64 or four FP32 elements per thread; half of
 // it in FP32 took 128 MB fields from 34 to 43 us, twice of it in FP64 512 MB from
 // 175 to 185), in FP64 consecutive tiles on one XCD (768 MB 261 -> 250 us; not in
-// FP32, 128 MB 43 -> 45), non-temporal stores (256 MB FP64 93 -> 62 us).
+// FP32, 128 MB 43 -> 45), non-temporal stores (256 MB FP64 93 -> 62 us), but plain
+// ones in FP64 while the cache holds input and output together (128 MB 0.97 of
+// the time over sixteen distributions, none above 1.02; rank rows of 64 bytes, 16^3
+// with P = 4, B = 1, 50 -> 38 us; not in FP32, 1.03 from packed).
 // Loads: plain while the last-level cache can still hold the field (256 MB FP64
 // 62 us, non-temporal 85), non-temporal beyond (512 MB FP64 181 -> 169, FP32 179
 // -> 169, 384 MB FP32 135 -> 129).  Geometric means over the distributions, to /
@@ -299,8 +304,9 @@ hipError_t launch_index_table(int64_t* out, const Geo& g, bool reciprocal, hipSt
 // us, 1 GB 661 / 803 -> 344 / 333; FP64 128 MB 39 / 41 -> 32 / 32, 512 MB 224 /
 // 262 -> 169 / 171 (6.3 TB/s), where the best of the former, whose runs were long
 // enough, took 167.
-// FULL: the field holds at least one tile (no guards).  NTL: non-temporal loads.
-template <typename T, int LE, bool FULL, bool NTL>
+// FULL: the field holds at least one tile (no guards).  NTL, NTS: non-temporal
+// loads and stores.
+template <typename T, int LE, bool FULL, bool NTL, bool NTS>
 __global__ void __launch_bounds__(256) convert_kernel(const Cx<T>* __restrict__ in, Cx<T>* __restrict__ out,
                                                       ConvertArgs a, int to_packed) {
     using C = Cx<T>;
@@ -334,6 +340,10 @@ __global__ void __launch_bounds__(256) convert_kernel(const Cx<T>* __restrict__ 
         if constexpr (NTL) return ld_nt(p);
         else return *p;
     };
+    auto st = [](C* p, const C& v) {
+        if constexpr (NTS) st_nt(p, v);
+        else *p = v;
+    };
     const int n = FULL ? EPT : tid >= (1 << a.ltile) ? 0 : a.ltile > 8 ? 1 << (a.ltile - 8) : 1;
     C v[EPT];
     if (to_packed) {
@@ -345,7 +355,7 @@ __global__ void __launch_bounds__(256) convert_kernel(const Cx<T>* __restrict__ 
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < EPT; k++)
-            if (k < n) st_nt(pk_out + sum(pk_bit, k), tile[pad(sum(slot_bit, k) + slot)]);
+            if (k < n) st(pk_out + sum(pk_bit, k), tile[pad(sum(slot_bit, k) + slot)]);
     } else {
 #pragma unroll
         for (int k = 0; k < EPT; k++) v[k] = k < n ? ld(pk_in + sum(pk_bit, k)) : C{0, 0};
@@ -355,7 +365,7 @@ __global__ void __launch_bounds__(256) convert_kernel(const Cx<T>* __restrict__ 
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < EPT; k++)
-            if (k < n) st_nt(nat_out + sum(nat_bit, k), tile[pad(tid + 256 * k)]);
+            if (k < n) st(nat_out + sum(nat_bit, k), tile[pad(tid + 256 * k)]);
     }
 }
 
@@ -366,12 +376,17 @@ hipError_t launch_natural_packed(const Cx<T>* in, Cx<T>* out, const Geo& g, int 
     const ConvertArgs a = convert_args(g, LE);
     const dim3 grid((unsigned)(g.field >> a.ltile), (unsigned)batch);
     const int tp = to_packed ? 1 : 0;
-    if (a.ltile < LE)
-        hipLaunchKernelGGL((convert_kernel<T, LE, false, false>), grid, dim3(256), 0, stream, in, out, a, tp);
-    else if ((int64_t)batch * g.field * (int64_t)sizeof(Cx<T>) <= kLastLevelCache)
-        hipLaunchKernelGGL((convert_kernel<T, LE, true, false>), grid, dim3(256), 0, stream, in, out, a, tp);
-    else
-        hipLaunchKernelGGL((convert_kernel<T, LE, true, true>), grid, dim3(256), 0, stream, in, out, a, tp);
+    const int64_t bytes = (int64_t)batch * g.field * (int64_t)sizeof(Cx<T>);
+    auto launch = [&](auto full, auto ntl, auto nts) {
+        hipLaunchKernelGGL((convert_kernel<T, LE, full.value, ntl.value, nts.value>), grid, dim3(256), 0, stream, in,
+                           out, a, tp);
+    };
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    if (a.ltile < LE) launch(no, no, yes);
+    else if (bytes > kLastLevelCache) launch(yes, yes, yes);
+    else if (sizeof(T) == 4 || 2 * bytes > kLastLevelCache) launch(yes, no, yes);
+    else if constexpr (sizeof(T) == 8) launch(yes, no, no);
     return hipGetLastError();
 }
 

@@ -1,12 +1,14 @@
-"""Either side of the sizes at which the FP64 marches shorten their strips: a batch
-takes one side, its fields alone the other.  The values do not depend on the side,
-so they agree bit for bit."""
+"""Either side of the sizes at which the FP64 marches shorten their strips and the
+FP64 converter takes other stores: a batch takes one side, its fields alone the
+other.  The values do not depend on the side, so they agree bit for bit."""
 import sys
 
 import pytest
 
 torch = pytest.importorskip("torch")
 pytestmark = pytest.mark.gpu
+
+from test_gpu_line_pass import _pack  # noqa: E402
 
 
 def _fields(pl, seed):
@@ -28,3 +30,17 @@ def test_fp64_strips_leave_every_value(n, p, b, batch):
                lambda q, u, a: q.laplace_add(u, a.clone(), 1.5, 0.25)):
         want = torch.cat([fn(one, u, a) for u, a in zip(x.chunk(batch), acc.chunk(batch))])
         assert torch.equal(fn(pl, x, acc), want)
+
+
+# the last batch of 128 MB together with the output, and the first beyond it
+@pytest.mark.parametrize("dims,n,p,b,batch", [(2, 64, 1, 4, 2048), (2, 64, 1, 4, 2049), (3, 16, 4, 1, 2048),
+                                              (3, 16, 4, 1, 2049), (3, 128, 2, 8, 4), (3, 128, 2, 8, 5)])
+def test_converter_stores_on_either_side(dims, n, p, b, batch):
+    from stencilfft_amd import Plan
+    print(f"[gpu] convert {dims}D N={n} P={p} B={b} batch {batch}", flush=True)
+    sys.stdout.flush()
+    pl = Plan(dims, n, p, b, precision="fp64", batch=batch, caller_scratch=True)
+    x = _fields(pl, batch)
+    packed = pl.natural_to_packed(x)
+    assert torch.equal(packed, _pack(x.reshape((batch,) + (n,) * dims), dims, n, p, b))
+    assert torch.equal(pl.packed_to_natural(packed), x)
