@@ -35,10 +35,9 @@ namespace lp {
 // LAP2 / LAP3 (input): the 5- / 7-point Laplacian of a packed end.
 enum End { PACKED = 0, ROW = 1, TILE = 2, LAP2 = 3, LAP3 = 4 };
 enum Dir { FWD = 0, INV = 1, SPEC = 2 };
-// How a workgroup runs over line groups: one group each, twiddles from the
-// caches (ONCE); a loop with the next group's loads in flight, for tiles that
-// leave a CU one workgroup (LOOP); the same with the twiddles in LDS (LOOP_LDS).
-enum Mode { ONCE = 0, LOOP = 1, LOOP_LDS = 2 };
+// How a workgroup runs over line groups: one group each (ONCE); a loop with the
+// next group's loads in flight, for lines that leave a CU one workgroup (LOOP).
+enum Mode { ONCE = 0, LOOP = 1 };
 
 // The radix passes of a line of 2^LN points with 2^LEPT elements per thread: of
 // at most 16 points, as even as possible, the larger ones first.
@@ -84,7 +83,7 @@ struct Line : Radices<LN, LEPT> {
         return s;
     }
     static constexpr int LS = line_stride();
-    static constexpr size_t lds_bytes(bool tables) { return sizeof(C) * (size_t)(LP * LS + (tables ? TW : 0)); }
+    static constexpr size_t lds_bytes() { return sizeof(C) * (size_t)(LP * LS); }
 
     // work item k of this thread in pass P: line l, butterfly j
     template <int P, bool TILED>
@@ -165,8 +164,9 @@ using IC = std::integral_constant<int, I>;
 // transforms back: both transforms and the multiplier in one sweep.
 //
 // `tables` holds the twiddles of passes 1, 2, .. one after the other
-// (Line::tw_off), read from there (the caches keep them, and the lanes read
-// consecutive entries) or, LOOP_LDS, copied to LDS first.
+// (Line::tw_off), read from there: the caches keep them, and the lanes read
+// consecutive entries.  A copy in LDS for looping workgroups lost: 2048^2 FP64, P =
+// 1 .. 8, one field forward 60-64 against 55-59 us, eight 450-480 against 443-478.
 template <typename T, int LN, int LLP, int LEPT, int IN, int OUT, int DIR, int MODE>
 __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9 ? 2 : 1)
     line_pass_kernel(const Cx<T>* in, Cx<T>* out, LinePassArgs a, const Cx<T>* __restrict__ tables, T scale,
@@ -184,7 +184,6 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
     extern __shared__ unsigned char smem_raw[];
     C* const lds = reinterpret_cast<C*>(smem_raw);
     int tid = threadIdx.x;
-    const C* const tw = MODE == LOOP_LDS ? lds + K::LP * K::LS : tables;
 
     auto group_base = [&](const auto& m, int g) -> int64_t {
         const int f = g >> a.lgroups;
@@ -330,9 +329,8 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
 
     int g = a.xcd ? (int)xcd_block(blockIdx.x, gridDim.x) : (int)blockIdx.x;
     if (g < a.groups) fetch(g, IC<0>{}, IC<EPT>{});
-    if constexpr (MODE == LOOP_LDS) {
-        for (int t = tid; t < K::TW; t += NT) lds[K::LP * K::LS + t] = tables[t];
-    }
+    // keeps the first loads' addresses apart from what follows: without it the
+    // one-line Laplacian passes spill 4 to 8 scalar registers
     __syncthreads();
     // exchanges through LDS in one group, each a point to issue a slice of
     // the next group's loads at
@@ -376,7 +374,7 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
             auto fwd = [&](auto self, auto pc) __attribute__((always_inline)) -> void {
                 constexpr int P = decltype(pc)::value;
                 constexpr bool TL = P == 0 && TIN;
-                K::template butterflies<P, true, TL>(v, tw, tid);
+                K::template butterflies<P, true, TL>(v, tables, tid);
                 if constexpr (P + 1 < NP) {
                     // the previous reads of LDS: this group's, or those
                     // before the barrier that ended the last group
@@ -450,7 +448,7 @@ __global__ void __launch_bounds__(1 << (LN + LLP - LEPT), (LN + LLP - LEPT) <= 9
             auto inv = [&](auto self, auto pc) __attribute__((always_inline)) -> void {
                 constexpr int P = decltype(pc)::value;
                 constexpr bool TL = P == 0 && TOUT;
-                K::template butterflies<P, false, TL>(v, tw, tid);
+                K::template butterflies<P, false, TL>(v, tables, tid);
                 if constexpr (P > 0) {
                     // SPEC: the last forward pass read exactly the elements
                     // this thread now writes

@@ -13,7 +13,7 @@ ZM_SPLIT(double, 8, false, 3, 3, 1, ONCE, 3, 4, 2, ONCE)
 ZM_SPLIT(double, 8, true, 4, 3, 2, ONCE, 4, 4, 2, ONCE)
 ZM_SPLIT(double, 9, false, 3, 3, 1, ONCE, 4, 3, 1, ONCE)
 ZM_SPLIT(double, 10, false, 4, 1, 0, ONCE, 4, 3, 2, LOOP)
-ZM_SPLIT(double, 11, false, 4, 1, 0, LOOP_LDS, 4, 2, -1, LOOP)
+ZM_SPLIT(double, 11, false, 4, 1, 0, LOOP, 4, 2, -1, LOOP)
 ZM_SPLIT(double, 12, false, 4, 0, -1, ONCE, 4, -1, -1, ONCE)
 ZM_SPLIT(double, 13, false, 4, 0, -1, ONCE, 4, -1, -1, ONCE)
 

@@ -14,6 +14,23 @@ constexpr size_t kLdsLimit = 160 * 1024;
 // of the lines per workgroup (and of the lines in the small variant), mode;
 // -1 lines: not built.  RADIX16: the alternative split of a plan that prefers
 // the largest radices (LinePassSize::radix16).
+//
+// Elements per thread: 8, whose radices of 8 need the fewest registers per value
+// in flight, up to the N where a line would then take a fourth radix pass or more
+// than 1024 threads; fewer for lines of 16 points, 32 where a 2048-point tile of
+// eight lines needs them.
+// Lines per workgroup, against half and twice as many (512 MB of fields, P = 2 and
+// 8, forward and inverse, time over the table's):
+//   rows   half 0.95-1.10, mostly 1.00; twice 0.98-1.07, at N = 512 FP64 1.07-1.12:
+//          about 1024 to 4096 elements, several workgroups per CU.
+//   tiles  half FP32 1.0-1.4 (runs of 64 bytes instead of 128), FP64 1.0-1.3 and at
+//          N = 2048 both 1.3-2.3 (runs of 32); twice 0.90-1.03 up to N = 256 and
+//          1.03-1.12 at N = 512, where it leaves a CU one workgroup, and beyond
+//          that LDS is full.
+// Mode, the other one: ONCE for N <= 512 (LOOP 1.03-1.27, N = 512 0.98-1.21), LOOP
+// where the tile leaves a CU one workgroup, N >= 1024 (ONCE in FP32 1.00-1.12, FP64
+// 0.98-1.02).  Rows loop at N = 2048 FP64 only: one field forward 55-59 us against
+// 59-63, eight 443-478 against 433-465.
 template <typename T, int LN, bool RADIX16>
 struct Split {
     static constexpr int row_ept = 4, row = -1, row_small = -1, tile_ept = 4, tile = -1, tile_small = -1;
@@ -71,8 +88,8 @@ struct Inst {
     using K = Line<T, LN, LLP < 0 ? 4 : LLP, LEPT>;
     static_assert(!built || same_radices(Radices<LN, LEPT>::list(), Radices<LN, LEPT0>::list()), "the table of the row or tile passes");
     static constexpr size_t lds() {
-        static_assert(K::lds_bytes(MODE == LOOP_LDS) <= kLdsLimit, "LDS");
-        return K::lds_bytes(MODE == LOOP_LDS);
+        static_assert(K::lds_bytes() <= kLdsLimit, "LDS");
+        return K::lds_bytes();
     }
     static const void* fn() { return (const void*)&line_pass_kernel<T, LN, LLP, LEPT, IN, OUT, DIR, MODE>; }
     static hipError_t prepare() {
