@@ -294,9 +294,10 @@ hipError_t launch_index_table(int64_t* out, const Geo& g, bool reciprocal, hipSt
 // it in FP32 took 128 MB fields from 34 to 43 us, twice of it in FP64 512 MB from
 // 175 to 185), in FP64 consecutive tiles on one XCD (768 MB 261 -> 250 us; not in
 // FP32, 128 MB 43 -> 45), non-temporal stores (256 MB FP64 93 -> 62 us), but plain
-// ones in FP64 while the cache holds input and output together (128 MB 0.97 of
-// the time over sixteen distributions, none above 1.02; rank rows of 64 bytes, 16^3
-// with P = 4, B = 1, 50 -> 38 us; not in FP32, 1.03 from packed).
+// ones in FP64 for rank rows shorter than a cache line while the last-level cache
+// holds input and output together: 128 MB of 16^3 with P = 4, B = 1, 50 -> 38 us
+// (256 MB as fast either way; longer rows, 32 MB of 128^3 9.1 -> 11.0 us with plain
+// stores, 128 MB within 5%).
 // Loads: plain while the last-level cache can still hold the field (256 MB FP64
 // 62 us, non-temporal 85), non-temporal beyond (512 MB FP64 181 -> 169, FP32 179
 // -> 169, 384 MB FP32 135 -> 129).  Geometric means over the distributions, to /
@@ -385,7 +386,7 @@ hipError_t launch_natural_packed(const Cx<T>* in, Cx<T>* out, const Geo& g, int 
     constexpr std::false_type no{};
     if (a.ltile < LE) launch(no, no, yes);
     else if (bytes > kLastLevelCache) launch(yes, yes, yes);
-    else if (sizeof(T) == 4 || 2 * bytes > kLastLevelCache) launch(yes, no, yes);
+    else if (sizeof(T) == 4 || g.l >= 8 || 2 * bytes > kLastLevelCache) launch(yes, no, yes);
     else if constexpr (sizeof(T) == 8) launch(yes, no, no);
     return hipGetLastError();
 }

@@ -32,9 +32,10 @@ def test_fp64_strips_leave_every_value(n, p, b, batch):
         assert torch.equal(fn(pl, x, acc), want)
 
 
-# the last batch of 128 MB together with the output, and the first beyond it
-@pytest.mark.parametrize("dims,n,p,b,batch", [(2, 64, 1, 4, 2048), (2, 64, 1, 4, 2049), (3, 16, 4, 1, 2048),
-                                              (3, 16, 4, 1, 2049), (3, 128, 2, 8, 4), (3, 128, 2, 8, 5)])
+# rank rows of 64 bytes (of 128 in the third): the last batch of 128 MB, and the
+# first beyond it
+@pytest.mark.parametrize("dims,n,p,b,batch", [(3, 16, 4, 1, 2048), (3, 16, 4, 1, 2049), (3, 16, 2, 1, 2048),
+                                              (3, 8, 2, 1, 16384), (3, 8, 2, 1, 16385), (2, 64, 1, 4, 2048)])
 def test_converter_stores_on_either_side(dims, n, p, b, batch):
     from stencilfft_amd import Plan
     print(f"[gpu] convert {dims}D N={n} P={p} B={b} batch {batch}", flush=True)
