@@ -25,7 +25,9 @@ import torch
 def _raw(t):
     """t with its storage in the order and with the values that the library reads:
     contiguous, lazy conjugations and negations carried out."""
-    return t.resolve_conj().resolve_neg().contiguous()
+    if t.is_conj() or t.is_neg():
+        t = t.resolve_conj().resolve_neg()
+    return t.contiguous()
 
 
 class _Forward(torch.autograd.Function):

@@ -200,7 +200,7 @@ class Plan:
         for t in tensors:
             if t.is_conj() or t.is_neg():
                 raise ValueError("a lazily conjugated or negated tensor: call resolve_conj() / resolve_neg() first")
-            if t.device != like.device:
+            if t is not like and t.device != like.device:
                 raise ValueError(f"tensors on {like.device} and {t.device}")
 
     @staticmethod
@@ -338,14 +338,15 @@ class Plan:
         the multiplier in one kernel where the plan has it (the three calls on
         two-stage plans).  `factor`: a CUDA tensor of one float64 that
         multiplies the multiplier."""
+        self._check_raw(x, *((x,) if out is None else (x, out)))
         out = self._out(x, out)
-        self._check_raw(x, x, out)
         if factor is not None:
             import torch
             if factor.dtype != torch.float64 or factor.numel() != 1 or factor.device != x.device:
                 raise ValueError(f"factor must be one float64 on {x.device}, got {tuple(factor.shape)} {factor.dtype} "
                                  f"on {factor.device}")
-            self._check_raw(x, factor)
+            if factor.is_neg():
+                raise ValueError("a lazily negated factor: call resolve_neg() first")
         if self.two_stage:
             import torch
             ts = torch.cuda.ExternalStream(stream) if isinstance(stream, int) else stream
@@ -366,6 +367,9 @@ class Plan:
         self._check_tensor(x)
         self._check_tensor(acc)
         self._check_raw(x, x, acc)
+        return self._laplace_add(x, acc, scale, alpha, stream)
+
+    def _laplace_add(self, x, acc, scale, alpha, stream):
         L.check(L._lib().zm_laplace_add(self._h, _ptr(x), _ptr(acc), float(scale), float(alpha), _stream(stream)),
                 "zm_laplace_add")
         return acc
@@ -378,7 +382,7 @@ class Plan:
             raise L.ZmError(L.ZM_ERR_ALIAS, "heat_step")
         norm = 1.0 / float(self.shape.n) ** self.shape.dims
         out = self.spectral_solve(x, "heat", nu, dt, length, norm, out=out, scratch=scratch, stream=stream)
-        return self.laplace_add(x, out, lap_scale, dt, stream=stream)
+        return self._laplace_add(x, out, lap_scale, dt, stream)  # the solve has checked both
 
     def residual_norm(self, acc, g):
         """acc -= g on the current stream; returns sum |acc|^2, a 0-dim tensor of
